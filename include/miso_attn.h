@@ -171,8 +171,15 @@ int miso_attn_prefill(const float* q, const float* qg, const uint16_t* k_cache,
  * miso_attn_prefill_workspace_bytes(4096) bytes serves every n). Calls that overlap on one
  * workspace race. For other n it runs miso_attn_prefill and the workspace is not used
  * (miso_attn_prefill_workspace_bytes returns 0). Rejects what miso_attn_prefill rejects and, for
- * the balanced sizes, a NULL or misaligned workspace or one smaller than required. */
+ * the balanced sizes, a NULL or misaligned workspace or one smaller than required.
+ *
+ * With a workspace of miso_attn_prefill_parts_workspace_bytes(max_n) bytes (which also holds the
+ * balanced form's for n <= 2048; same zero fill), launches of n <= max_n tokens up to 3072 that
+ * leave the chip idle otherwise -- few tokens after a prefix -- run in parts: the keys of every
+ * token block are split between workgroups and a second kernel joins the parts (two launches,
+ * bit-equal from call to call). A smaller workspace keeps the forms above. */
 uint64_t miso_attn_prefill_workspace_bytes(uint32_t n);
+uint64_t miso_attn_prefill_parts_workspace_bytes(uint32_t max_n);
 int miso_attn_prefill_ws(const float* q, const float* qg, const uint16_t* k_cache,
                          const uint16_t* v_cache, float* core, uint32_t pos0, uint32_t n,
                          uint32_t max_ctx, uint32_t qg_stride, void* workspace,
@@ -266,6 +273,14 @@ int miso_attn_prefill_fp8(const float* q, const float* qg, const uint8_t* k8, co
                           uint16_t* v_ws, float* core, uint32_t pos0, uint32_t n,
                           uint32_t max_ctx, uint32_t qg_stride, void* stream);
 
+/* miso_attn_prefill_fp8 with the causal prefill's own workspace: after the widening it is
+ * miso_attn_prefill_ws over the widened rows, with that call's workspace contract. */
+int miso_attn_prefill_fp8_ws(const float* q, const float* qg, const uint8_t* k8,
+                             const uint8_t* v8, const float* k_scale, const float* v_scale,
+                             uint16_t* k_ws, uint16_t* v_ws, float* core, uint32_t pos0,
+                             uint32_t n, uint32_t max_ctx, uint32_t qg_stride, void* workspace,
+                             uint64_t workspace_bytes, void* stream);
+
 /* Q4_K GEMV y = W x (the attention's Q4_K projections attn_q, attn_k, attn_output). Replaces the
  * launches of q4k_gemv_kernel<ActFormat, K, 256, R> in gemv() (src/engine/weights.hip:248-275,
  * kernels/q4k_gemv.hpp:196-239). w: n_rows rows of k / 256 Q4_K blocks in the r1 layout
@@ -354,8 +369,8 @@ typedef struct miso_attn_layer {
 
 /* Device floats of the decode / prefill workspaces (the engine's AttentionScratch and
  * AttentionPrefillScratch, src/engine/attention.hpp:44-69), for chunks of up to max_tok tokens.
- * The prefill workspace ends with the balanced prefill's workspace (miso_attn_prefill_ws), which
- * chunks of up to 4096 tokens use: zero-fill it once when it is allocated (every call leaves its
+ * The prefill workspace ends with the causal prefill's (miso_attn_prefill_ws, balanced pairs and
+ * parts): zero-fill it once when it is allocated (every call leaves its
  * pair counters zero). */
 uint64_t miso_attn_layer_decode_ws(void);
 uint64_t miso_attn_layer_prefill_ws(uint32_t max_tok);

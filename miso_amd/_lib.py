@@ -32,6 +32,7 @@ SIGNATURES = {
     "miso_attn_decode_noalloc": (c_int, [P, P, P, P, P, c_uint32, c_uint32, c_uint32, P]),
     "miso_attn_prefill": (c_int, [P, P, P, P, P, c_uint32, c_uint32, c_uint32, c_uint32, P]),
     "miso_attn_prefill_workspace_bytes": (c_uint64, [c_uint32]),
+    "miso_attn_prefill_parts_workspace_bytes": (c_uint64, [c_uint32]),
     "miso_attn_prefill_ws": (c_int, [P, P, P, P, P, c_uint32, c_uint32, c_uint32, c_uint32, P,
                                      c_uint64, P]),
     "miso_attn_ragged_splits": (c_uint32, [c_uint32]),
@@ -49,6 +50,8 @@ SIGNATURES = {
                                          c_float, c_uint32, c_uint32, P]),
     "miso_attn_prefill_fp8": (c_int, [P, P, P, P, P, P, P, P, P, c_uint32, c_uint32, c_uint32,
                                       c_uint32, P]),
+    "miso_attn_prefill_fp8_ws": (c_int, [P, P, P, P, P, P, P, P, P, c_uint32, c_uint32, c_uint32,
+                                         c_uint32, P, c_uint64, P]),
     "miso_attn_q4k_gemv": (c_int, [P, P, P, c_uint32, c_uint32, c_int, P]),
     "miso_attn_q6k_gemv": (c_int, [P, P, P, c_uint32, c_uint32, P]),
     "miso_attn_q4k_q6k_gemv_pair": (c_int, [P, c_uint32, P, P, c_uint32, P, P, P]),

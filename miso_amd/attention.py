@@ -189,21 +189,22 @@ def prefill_workspace_bytes(n: int) -> int:
 
 
 class PrefillScratch:
-    """Workspace of the balanced prefill (miso_attn_prefill_ws) for launches of up to max_n
-    tokens (the form covers n <= 2048 and 3841 <= n <= 4096), zero-filled once; every call leaves
-    it reusable."""
+    """Workspace of miso_attn_prefill_ws for launches of up to max_n tokens (balanced pairs:
+    n <= 2048 and 3841 <= n <= 4096; parts: up to 3072 tokens after a prefix), zero-filled once;
+    every call leaves it reusable."""
 
     def __init__(self, max_n: int = 4096, device="cuda"):
         nbytes = max(prefill_workspace_bytes(min(max_n, 2048)),
-                     prefill_workspace_bytes(min(max_n, 4096)))
+                     prefill_workspace_bytes(min(max_n, 4096)),
+                     int(_lib.load().miso_attn_prefill_parts_workspace_bytes(max_n)))
         self.buf = torch.zeros(max((nbytes + 3) // 4, 4), dtype=torch.int32, device=device)
         self.nbytes = self.buf.numel() * 4
 
 
 def attn_prefill(q, qg, k_cache, v_cache, core, pos0: int, n: int, max_ctx: int,
                  qg_stride: int = QG_STRIDE, stream=None, scratch: PrefillScratch = None) -> None:
-    """Causal prefill of tokens pos0 .. pos0 + n - 1; with `scratch`, the balanced form
-    (miso_attn_prefill_ws)."""
+    """Causal prefill of tokens pos0 .. pos0 + n - 1; with `scratch`, in balanced pairs or in
+    parts where those are faster (miso_attn_prefill_ws)."""
     f32 = torch.float32
     _need(q, "q", f32, n * Q_HEADS * DIM)
     _need(qg, "qg", f32, (n - 1) * qg_stride + Q_HEADS * 2 * DIM if n else 0)
@@ -356,12 +357,14 @@ def attn_prep_batch_fp8(qg, k, v, q_norm, k_norm, inv_freq, cache: Fp8Cache, q, 
 
 
 class Fp8PrefillScratch:
-    """f16 workspaces for attn_prefill_fp8 over up to max_rows cache rows (pos0 + n)."""
+    """f16 workspaces for attn_prefill_fp8 over up to max_rows cache rows (pos0 + n), and the
+    prefill's own workspace for as many tokens."""
 
     def __init__(self, max_rows: int, device="cuda"):
         self.max_rows = max_rows
         self.k = torch.empty(KV_HEADS * max_rows * DIM, dtype=torch.float16, device=device)
         self.v = torch.empty(KV_HEADS * max_rows * DIM, dtype=torch.float16, device=device)
+        self.prefill = PrefillScratch(max_rows, device)
 
 
 def attn_prefill_fp8(q, qg, cache: Fp8Cache, core, pos0: int, n: int,
@@ -378,9 +381,10 @@ def attn_prefill_fp8(q, qg, cache: Fp8Cache, core, pos0: int, n: int,
     _need(qg, "qg", f32, (n - 1) * qg_stride + Q_HEADS * 2 * DIM if n else 0)
     _need(core, "core", f32, n * Q_HEADS * DIM)
     _need_fp8(cache)
-    _lib.check(_lib.load().miso_attn_prefill_fp8(
+    _lib.check(_lib.load().miso_attn_prefill_fp8_ws(
         _ptr(q), _ptr(qg), *(_ptr(b) for b in cache.buffers()), _ptr(scratch.k), _ptr(scratch.v),
-        _ptr(core), pos0, n, cache.max_ctx, qg_stride, _stream(stream)))
+        _ptr(core), pos0, n, cache.max_ctx, qg_stride, _ptr(scratch.prefill.buf),
+        scratch.prefill.nbytes, _stream(stream)))
     return scratch
 
 

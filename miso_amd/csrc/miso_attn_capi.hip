@@ -375,6 +375,25 @@ uint64_t miso_attn_prefill_workspace_bytes(uint32_t n) {
   return k::attn_prefill_balanced(n) ? k::attn_prefill_split_workspace_bytes(n) : 0;
 }
 
+uint64_t miso_attn_prefill_parts_workspace_bytes(uint32_t max_n) {
+  return k::attn_prefill_parts_workspace_bytes(max_n);
+}
+
+// Checks the workspace of a prefill whose other arguments are good, and launches it.
+static int prefill_with_ws(const char* fn, const k::AttnPrefillParams& a, void* workspace,
+                           uint64_t bytes, void* stream) {
+  // A launch that would run one workgroup per block takes any workspace, also none.
+  const bool usable = !bad_ptr(workspace);
+  if (k::attn_prefill_balanced(a.n)) {
+    if (!usable)
+      return fail(fn, "workspace must be a non-null, 16-byte aligned device pointer");
+    if (bytes < k::attn_prefill_split_workspace_bytes(a.n))
+      return fail(fn, "workspace smaller than miso_attn_prefill_workspace_bytes(n)");
+  }
+  k::attn_prefill_launch(a, workspace, usable ? bytes : 0, as_stream(stream));
+  return launched(fn);
+}
+
 int miso_attn_prefill_ws(const float* q, const float* qg, const uint16_t* k_cache,
                          const uint16_t* v_cache, float* core, uint32_t pos0, uint32_t n,
                          uint32_t max_ctx, uint32_t qg_stride, void* workspace,
@@ -385,22 +404,7 @@ int miso_attn_prefill_ws(const float* q, const float* qg, const uint16_t* k_cach
     return rc;
   const k::AttnPrefillParams a{q,    qg, as_half(k_cache), as_half(v_cache), core, pos0,
                                n,    max_ctx, qg_stride};
-  if (!k::attn_prefill_balanced(n)) {  // the one-block-per-workgroup layout
-    k::attn_prefill_kernel<256><<<k::attn_prefill_items(n), 256, 0, as_stream(stream)>>>(a);
-    return launched(fn);
-  }
-  if (bad_ptr(workspace))
-    return fail(fn, "workspace must be a non-null, 16-byte aligned device pointer");
-  if (workspace_bytes < k::attn_prefill_split_workspace_bytes(n))
-    return fail(fn, "workspace smaller than miso_attn_prefill_workspace_bytes(n)");
-  char* const ws = static_cast<char*>(workspace);
-  float* const part_ml = reinterpret_cast<float*>(ws + k::kAttnSplitCounterBytes);
-  float* const part_o = part_ml + std::size_t{k::attn_prefill_split_pairs(n)} * 2 *
-                                       k::attn_prefill_split_rows(n) * 2;
-  const k::AttnPrefillSplitParams p{a, part_o, part_ml, reinterpret_cast<unsigned*>(ws)};
-  k::attn_prefill_split_kernel<256><<<k::attn_prefill_split_items(n), 256, 0,
-                                      as_stream(stream)>>>(p);
-  return launched(fn);
+  return prefill_with_ws(fn, a, workspace, workspace_bytes, stream);
 }
 
 uint32_t miso_attn_ragged_splits(uint32_t max_len) { return k::attn_ragged_splits(max_len); }
@@ -573,30 +577,53 @@ int miso_attn_prep_batch_fp8(const float* qg, const float* kp, const float* v,
   return launched("miso_attn_prep_batch_fp8");
 }
 
-int miso_attn_prefill_fp8(const float* q, const float* qg, const uint8_t* k8, const uint8_t* v8,
-                          const float* k_scale, const float* v_scale, uint16_t* k_ws,
-                          uint16_t* v_ws, float* core, uint32_t pos0, uint32_t n,
-                          uint32_t max_ctx, uint32_t qg_stride, void* stream) {
+// The argument checks of the fp8 prefills, then the rows [0, pos0 + n) widened into k_ws / v_ws.
+static int prefill_fp8_widen(const char* fn, const float* q, const float* qg, const uint8_t* k8,
+                             const uint8_t* v8, const float* k_scale, const float* v_scale,
+                             uint16_t* k_ws, uint16_t* v_ws, float* core, uint32_t pos0,
+                             uint32_t n, uint32_t max_ctx, uint32_t qg_stride, void* stream) {
   if (any_bad(q, qg, k8, v8, k_ws, v_ws, core) || bad_scalars(k_scale) || bad_scalars(v_scale))
-    return fail("miso_attn_prefill_fp8", kBadPtr);
+    return fail(fn, kBadPtr);
   if (n == 0)
-    return fail("miso_attn_prefill_fp8", "n must be >= 1");
+    return fail(fn, "n must be >= 1");
   if (static_cast<uint64_t>(pos0) + n > max_ctx)
-    return fail("miso_attn_prefill_fp8", "KV cache is full (pos0 + n > max_ctx)");
+    return fail(fn, "KV cache is full (pos0 + n > max_ctx)");
   if (qg_stride < 8192 || qg_stride % 4 != 0)
-    return fail("miso_attn_prefill_fp8", "qg_stride must be >= 8192 and a multiple of 4");
+    return fail(fn, "qg_stride must be >= 8192 and a multiple of 4");
   const uint32_t rows = pos0 + n;
   const k::AttnKvFp8WidenParams w{k8,           v8, k_scale, v_scale, as_half(k_ws),
                                   as_half(v_ws), rows, max_ctx};
   const uint32_t wgrid = std::min<uint32_t>(rows, 4096);  // 4 rows per workgroup, grid-stride
   k::attn_kv_fp8_widen_kernel<256><<<wgrid, 256, 0, as_stream(stream)>>>(w);
-  const int rc = launched("miso_attn_prefill_fp8");
-  if (rc != 0)
+  return launched(fn);
+}
+
+int miso_attn_prefill_fp8(const float* q, const float* qg, const uint8_t* k8, const uint8_t* v8,
+                          const float* k_scale, const float* v_scale, uint16_t* k_ws,
+                          uint16_t* v_ws, float* core, uint32_t pos0, uint32_t n,
+                          uint32_t max_ctx, uint32_t qg_stride, void* stream) {
+  constexpr const char* fn = "miso_attn_prefill_fp8";
+  if (const int rc = prefill_fp8_widen(fn, q, qg, k8, v8, k_scale, v_scale, k_ws, v_ws, core, pos0,
+                                       n, max_ctx, qg_stride, stream))
     return rc;
-  const k::AttnPrefillParams p{q, qg, as_half(k_ws), as_half(v_ws), core, pos0, n, rows,
-                               qg_stride};
+  const k::AttnPrefillParams p{q,    qg, as_half(k_ws), as_half(v_ws), core, pos0,
+                               n,    pos0 + n, qg_stride};
   k::attn_prefill_kernel<256><<<k::attn_prefill_items(n), 256, 0, as_stream(stream)>>>(p);
-  return launched("miso_attn_prefill_fp8");
+  return launched(fn);
+}
+
+int miso_attn_prefill_fp8_ws(const float* q, const float* qg, const uint8_t* k8,
+                             const uint8_t* v8, const float* k_scale, const float* v_scale,
+                             uint16_t* k_ws, uint16_t* v_ws, float* core, uint32_t pos0,
+                             uint32_t n, uint32_t max_ctx, uint32_t qg_stride, void* workspace,
+                             uint64_t workspace_bytes, void* stream) {
+  constexpr const char* fn = "miso_attn_prefill_fp8_ws";
+  if (const int rc = prefill_fp8_widen(fn, q, qg, k8, v8, k_scale, v_scale, k_ws, v_ws, core, pos0,
+                                       n, max_ctx, qg_stride, stream))
+    return rc;
+  const k::AttnPrefillParams p{q,    qg, as_half(k_ws), as_half(v_ws), core, pos0,
+                               n,    pos0 + n, qg_stride};
+  return prefill_with_ws(fn, p, workspace, workspace_bytes, stream);
 }
 
 int miso_attn_q4k_gemv(const uint8_t* w, const float* x, float* y, uint32_t n_rows, uint32_t k,

@@ -268,10 +268,10 @@ inline DecodeWorkspace decode_workspace(float* ws) {
   return d;
 }
 
-// The prefill workspace ends with the balanced prefill's workspace for chunks of up to
-// min(max_tok, 4096) tokens (attention_prefill.hpp): its pair counters must be zero before the
-// first chunk, so the whole prefill workspace is zero-filled once when it is allocated (every
-// chunk leaves the counters zero).
+// The prefill workspace ends with the causal prefill's own (attn_prefill_launch: balanced pairs
+// or parts, for chunks of up to max_tok tokens): its pair counters must be zero before the first
+// chunk, so the whole prefill workspace is zero-filled once when it is allocated (every chunk
+// leaves the counters zero).
 struct PrefillWorkspace {
   float* xn;     // [max_tok][2048]
   float* proj;   // [max_tok][9216]
@@ -279,11 +279,13 @@ struct PrefillWorkspace {
   float* core;   // [max_tok][16][256]
   float* xs;     // [max_tok][4096 / 32] GEMM input sums
   _Float16* xh;  // [max_tok][4096] GEMM input values
-  char* balance;  // attn_prefill_split_workspace_bytes(min(max_tok, 4096)) bytes
+  char* balance;  // prefill_balance_floats(max_tok) floats
 };
 
 inline constexpr std::size_t prefill_balance_floats(unsigned max_tok) {
-  return (attn_prefill_split_workspace_bytes(max_tok < 4096 ? max_tok : 4096) + 15) / 16 * 4;
+  const std::size_t pairs = attn_prefill_split_workspace_bytes(max_tok < 4096 ? max_tok : 4096);
+  const std::size_t parts = attn_prefill_parts_workspace_bytes(max_tok);
+  return ((parts > pairs ? parts : pairs) + 15) / 16 * 4;
 }
 
 inline constexpr std::size_t prefill_workspace_floats(unsigned max_tok) {
@@ -346,8 +348,7 @@ inline const char* decode_step(const Weights& w, attn::half_t* k_cache, attn::ha
 }
 
 // n consecutive tokens at pos0 ([n][2048] h / delta / y): the prefill GEMMs, batched prep and
-// causal flash attention over the cache up to each token (the balanced form for chunks of up to
-// 4096 tokens).
+// causal flash attention over the cache up to each token (attn_prefill_launch).
 inline const char* prefill_step(const Weights& w, attn::half_t* k_cache, attn::half_t* v_cache,
                                 unsigned pos0, unsigned n, unsigned max_ctx, float* h,
                                 const float* delta, float* y, float eps,
@@ -374,16 +375,7 @@ inline const char* prefill_step(const Weights& w, attn::half_t* k_cache, attn::h
                                  kProj};
   attn_prep_batch_kernel<256><<<n * 18, 256, 0, stream>>>(prep);
   const AttnPrefillParams ap{ws.q, ws.proj, k_cache, v_cache, ws.core, pos0, n, max_ctx, kProj};
-  if (attn_prefill_balanced(n)) {  // n <= 4096 and n <= max_tok: within its workspace
-    float* const part_ml = reinterpret_cast<float*>(ws.balance + kAttnSplitCounterBytes);
-    const std::size_t ml_floats =
-        std::size_t{attn_prefill_split_pairs(n)} * 2 * attn_prefill_split_rows(n) * 2;
-    const AttnPrefillSplitParams sp{ap, part_ml + ml_floats, part_ml,
-                                    reinterpret_cast<unsigned*>(ws.balance)};
-    attn_prefill_split_kernel<256><<<attn_prefill_split_items(n), 256, 0, stream>>>(sp);
-  } else {
-    attn_prefill_kernel<256><<<attn_prefill_items(n), 256, 0, stream>>>(ap);
-  }
+  attn_prefill_launch(ap, ws.balance, prefill_balance_floats(max_tok) * sizeof(float), stream);
   gemm_input(ws.core, kCore, n, ws.xh, ws.xs, stream);
   return gemm(w.o, ws.xh, ws.xs, n, y, kHidden, stream);
 }

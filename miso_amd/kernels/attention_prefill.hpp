@@ -160,6 +160,133 @@ __host__ __device__ constexpr std::size_t attn_prefill_split_workspace_bytes(uns
                                       attn_prefill_split_rows(n) * (attn::kDim + 2) * sizeof(float);
 }
 
+// ------------------------------------------------------------------------------------------------
+// Prefill in parts (no reference counterpart): the keys of a token block split between workgroups.
+// A launch of few tokens has few token blocks (203 tokens: 26 workgroups of 16 tokens for 256 CUs),
+// and each streams the whole prefix alone. Here the tiles of all blocks of a KV head, block after
+// block, are one list, cut into `workers` even runs, one workgroup each. A run covers the end of a
+// block, whole blocks and the start of another; a block that no cut falls into is stored at once,
+// a part of a cut block goes to the workspace as (m, l, O) and attn_prefill_merge_kernel joins the
+// parts in tile order (the output is the same on every call).
+//
+// The cuts are made on the host (AttnPrefillCuts, by value in both launches: KV heads share them).
+// A cut closer than kAttnSplitMinTiles tiles to a block's start or end moves there, so that a part
+// is worth its prologue and the first tile of a part has a visible key for every row of the block.
+// ------------------------------------------------------------------------------------------------
+
+constexpr unsigned kAttnPartsMaxWorkers = 128;  // per KV head: 256 CUs, one workgroup each
+constexpr unsigned kAttnPartsMaxBlocks = 256;   // token blocks per KV head (8 bits of a cut)
+
+struct AttnPrefillCuts {
+  unsigned workers, blocks;
+  // Worker w runs the tiles from at[w] up to at[w + 1]; a place is block << 23 | tile.
+  unsigned at[kAttnPartsMaxWorkers + 1];
+};
+
+struct AttnPrefillPartsParams {
+  AttnPrefillParams a;
+  float* part_o;   // [slot][rows][256], rows = 128 per row block per wave, relative to 2^m
+  float* part_ml;  // [slot][rows][2]: m (log2 units), l
+  AttnPrefillCuts cuts;
+};
+
+// A part's slot: a worker's parts and a block's parts both follow each other in the tile list, so
+// worker + block is a number of its own for each part of a KV head.
+__host__ __device__ constexpr unsigned attn_prefill_parts_slots(unsigned workers,
+                                                                unsigned blocks) {
+  return attn::kKvHeads * (workers + blocks);
+}
+__host__ __device__ constexpr std::size_t attn_prefill_parts_bytes(unsigned workers,
+                                                                   unsigned blocks,
+                                                                   unsigned row_blocks) {
+  return std::size_t{attn_prefill_parts_slots(workers, blocks)} * 128 * row_blocks *
+         (attn::kDim + 2) * sizeof(float);
+}
+
+// Tiles of 32 keys that block b (of `tokens` tokens each) of a launch sees.
+__host__ __device__ constexpr unsigned attn_prefill_block_tiles(unsigned pos0, unsigned n,
+                                                                unsigned tokens, unsigned b) {
+  const unsigned end = (b + 1) * tokens < n ? (b + 1) * tokens : n;
+  return (pos0 + end + 31) / 32;
+}
+
+// What a job (a worker's run inside one block) costs besides its tiles, in tiles: the query
+// prologue, the first tile's latency and the partial's way out.
+constexpr unsigned kAttnPartsJobTiles = 12;
+
+// Largest launch in parts, and the row blocks per wave it takes: 0 where the other forms are as
+// fast. Measured on one MI355X (parts against the form it replaces, N(0,1) inputs, us):
+//   - Up to 2048 tokens the balanced pairs fill 2 of every 256 CUs per token block. Parts fill all
+//     of them and cost a merge launch and a job's prologue more: 10 tiles and an eighth of a
+//     pair's run. 203 tokens after 12001: 69 against 346; 37 after 1000: 19 against 39; 512 after
+//     1536: 41 against 68; 1300 after 2000: 91 both; 1024 after 0: 37 against 35 (pairs kept);
+//     2000 after 4000: 202 against 182 (pairs kept).
+//   - 2049 to 3072 tokens leave the last round of one-block workgroups half empty, which a long
+//     prefix makes costly: 2100 after 8000 336 against 506, 3001 after 5003 363 against 388; 3001
+//     after 0 112 against 104 and 3300 after 4000 352 against 343 (one workgroup per block kept).
+//   - Two row blocks per wave (half the LDS reads per MFMA, twice the prologue and partial) pay
+//     from about 150 one-block tiles per worker: 512 after 32000 280 against 330 with one, 700
+//     after 14000 207 against 223; 512 after 4096 (34 tiles) 78 against 65, 2500 after 2500 (145)
+//     206 against 190.
+constexpr unsigned kAttnPartsMaxTokens = 3072;
+inline unsigned attn_prefill_parts_row_blocks(unsigned pos0, unsigned n) {
+  if (n == 0 || n > kAttnPartsMaxTokens || std::uint64_t{pos0} + n >= 1u << 27)
+    return 0;
+  const unsigned blocks = (n + kAttnQBlock - 1) / kAttnQBlock;
+  std::uint64_t total = 0;
+  for (unsigned b = 0; b < blocks; ++b)
+    total += attn_prefill_block_tiles(pos0, n, kAttnQBlock, b);
+  const std::uint64_t per_block = total / blocks, per_worker = total / kAttnPartsMaxWorkers;
+  const bool pays = n <= 2048 ? per_block >= per_worker + 10 + per_block / 8 : pos0 >= n;
+  return !pays ? 0 : per_worker >= 150 ? 2 : 1;
+}
+
+// Workspace with which every launch of up to max_n tokens can run in parts or in balanced pairs:
+// the pairs' counters, then the parts' (m, l) and O.
+constexpr std::size_t attn_prefill_parts_workspace_bytes(unsigned max_n) {
+  const unsigned n = max_n < kAttnPartsMaxTokens ? max_n : kAttnPartsMaxTokens;
+  return kAttnSplitCounterBytes +
+         attn_prefill_parts_bytes(kAttnPartsMaxWorkers, (n + 31) / 32, 2);
+}
+
+// Cuts the tiles of n tokens after pos0 in blocks of 16 row_blocks tokens into at most
+// `max_workers` runs of about equal cost, kAttnPartsJobTiles per job included: the least cost per
+// run, in steps of 1/16, with which the runs filled one after another suffice.
+inline AttnPrefillCuts attn_prefill_cuts(unsigned pos0, unsigned n, unsigned row_blocks,
+                                         unsigned max_workers) {
+  constexpr unsigned job = kAttnPartsJobTiles, kMin = kAttnSplitMinTiles;
+  const unsigned tokens = kAttnQBlock * row_blocks;
+  AttnPrefillCuts c{};
+  c.blocks = (n + tokens - 1) / tokens;
+  std::uint64_t total = std::uint64_t{c.blocks > max_workers ? c.blocks : max_workers} * job;
+  for (unsigned b = 0; b < c.blocks; ++b)
+    total += attn_prefill_block_tiles(pos0, n, tokens, b);
+  std::uint64_t cap = (total + max_workers - 1) / max_workers;
+  cap = cap > job + 2 * kMin ? cap : job + 2 * kMin;
+  for (;; cap += cap / 16 + 1) {
+    unsigned b = 0, off = 0, w = 0;  // the next tile
+    for (; w < max_workers && b < c.blocks; ++w) {
+      c.at[w] = b << 23 | off;
+      for (std::uint64_t room = cap; b < c.blocks && room >= job + kMin;) {
+        const unsigned tiles = attn_prefill_block_tiles(pos0, n, tokens, b);
+        const unsigned left = tiles - off;
+        room -= job;
+        if (left < room + kMin) {  // the rest of the block (no part shorter than kMin remains)
+          room = room > left ? room - left : 0;
+          ++b, off = 0;
+        } else {
+          off += static_cast<unsigned>(room);
+          room = 0;
+        }
+      }
+    }
+    c.workers = w;
+    c.at[w] = c.blocks << 23;
+    if (b == c.blocks)
+      return c;
+  }
+}
+
 namespace prefill_detail {
 
 using cdna4::float16_t;
@@ -181,6 +308,7 @@ constexpr unsigned kVBase = kStages * kTileBytes;
 // After the ring: each wave's Q^T B operands of its second row block (16 k-steps x 64 lanes x
 // 16 bytes), read from LDS per tile instead of occupying 64 more VGPRs.
 constexpr unsigned kQ1Bytes = 16 * 64 * 16;
+constexpr unsigned kTileMask = (1u << 23) - 1;  // the tile of a place in AttnPrefillCuts
 struct alignas(1024) Shared {
   unsigned char kv[2 * kStages * kTileBytes];
   unsigned char q1[4][kQ1Bytes];
@@ -714,7 +842,8 @@ struct PrefillJob {
 template <unsigned kTokens>
 __device__ __attribute__((always_inline)) inline unsigned block_tiles(const AttnPrefillParams& p,
                                                                       unsigned b) {
-  return (p.pos0 + min((b + 1) * kTokens, p.n) + kKeys - 1) / kKeys;
+  static_assert(kKeys == 32);
+  return attn_prefill_block_tiles(p.pos0, p.n, kTokens, b);
 }
 
 // The jobs of item `item` (wave-uniform): one for the one-block-per-workgroup layout of
@@ -763,10 +892,13 @@ __device__ __attribute__((always_inline)) inline unsigned item_jobs(const AttnPr
   }
 }
 
-template <int kBlocks, bool kSplit = false>
+// The forms of a launch: one workgroup per token block, balanced pairs, parts.
+struct PlainForm {};
+template <int kBlocks, class Form>
 __device__ __attribute__((always_inline)) inline void prefill_items(
-    const AttnPrefillParams& p, const AttnPrefillSplitParams* sp, unsigned first, unsigned count,
-    Shared& sh) {
+    const AttnPrefillParams& p, const Form* sp, unsigned first, unsigned count, Shared& sh) {
+  constexpr bool kSplit = std::is_same_v<Form, AttnPrefillSplitParams>;
+  constexpr bool kParts = std::is_same_v<Form, AttnPrefillPartsParams>;
   using attn::kDim;
   constexpr int kGroup = attn::kQHeads / attn::kKvHeads;
   constexpr unsigned kItemTokens = kAttnQBlock * kBlocks;
@@ -806,9 +938,33 @@ __device__ __attribute__((always_inline)) inline void prefill_items(
 
   for (unsigned item = first + blockIdx.x; item < first + count; item += gridDim.x) {
     PrefillJob jobs[2];
-    const unsigned njobs = item_jobs<kItemTokens, kSplit>(p, item, blocks, jobs);
+    unsigned njobs, run = 0, run_end = 0;
+    if constexpr (kParts) {
+      // Workgroups 4 .. 7 of every 8 (their XCDs) serve KV head 1.
+      const unsigned w = item / 8 * 4 + item % 4;
+      if (w >= sp->cuts.workers)
+        continue;
+      run = sp->cuts.at[w];
+      run_end = sp->cuts.at[w + 1];
+      if (run >= run_end)
+        continue;
+      njobs = (run_end >> 23) - (run >> 23) + ((run_end & kTileMask) != 0 ? 1 : 0);
+    } else {
+      njobs = item_jobs<kItemTokens, kSplit>(p, item, blocks, jobs);
+    }
     for (unsigned j = 0; j < njobs; ++j) {  // uniform across the workgroup
-      const PrefillJob jb = j == 0 ? jobs[0] : jobs[1];
+      PrefillJob jb;
+      if constexpr (kParts) {
+        const unsigned kvh = item / 4 % 2, blk = (run >> 23) + j;
+        const unsigned all = block_tiles<kItemTokens>(p, blk);
+        const unsigned tb = j == 0 ? run & kTileMask : 0;
+        const unsigned te = blk == run_end >> 23 ? run_end & kTileMask : all;
+        const unsigned w = item / 8 * 4 + item % 4;
+        jb = PrefillJob{kvh, blk, tb, te, kvh * (sp->cuts.workers + blocks) + w + blk,
+                        tb != 0 || te != all};
+      } else {
+        jb = j == 0 ? jobs[0] : jobs[1];
+      }
       const unsigned kvh = jb.kvh, blk = jb.blk, tb = jb.tb;
       const unsigned t0 = blk * kItemTokens;
       const unsigned t_end = min(t0 + kItemTokens, p.n);
@@ -1112,6 +1268,24 @@ __device__ __attribute__((always_inline)) inline void prefill_items(
           }
         }
       }
+      if constexpr (kParts) {
+        if (jb.part) {  // uniform: (m, l) and the rows of O to the part's slot, for the merge
+          store = false;
+          const std::size_t row0 = std::size_t{jb.slot} * kPartRows + 32 * kBlocks * wave;
+#pragma unroll
+          for (int c = 0; c < kBlocks; ++c) {
+            stage_o(c, 1.0f);
+            if (hi == 0)
+              *reinterpret_cast<float2*>(sp->part_ml + 2 * (row0 + 32 * c + col)) =
+                  float2{rw.m[c], l_row[c]};
+            float* out = sp->part_o + (row0 + 32 * c) * kDim + 4 * lane;
+#pragma unroll
+            for (int r = 0; r < 32; ++r)
+              if (tw + 4 * c + r / 8 < p.n)  // uniform
+                *reinterpret_cast<cdna4::float4_t*>(out + r * kDim) = staged_row(r);
+          }
+        }
+      }
       if (store) {
 #pragma unroll
         for (int c = 0; c < kBlocks; ++c) {
@@ -1190,10 +1364,11 @@ template <int kBlock>
 __device__ void attn_prefill_op(const AttnPrefillParams& p, unsigned first, unsigned count) {
   static_assert(kBlock == 256, "four waves per prefill workgroup");
   __shared__ prefill_detail::Shared sh;
+  constexpr const prefill_detail::PlainForm* kPlain = nullptr;
   if (attn_prefill_row_blocks(p.n) == 2)  // uniform: the item size follows n
-    prefill_detail::prefill_items<2>(p, nullptr, first, count, sh);
+    prefill_detail::prefill_items<2>(p, kPlain, first, count, sh);
   else
-    prefill_detail::prefill_items<1>(p, nullptr, first, count, sh);
+    prefill_detail::prefill_items<1>(p, kPlain, first, count, sh);
 }
 
 template <int kBlock>
@@ -1208,9 +1383,147 @@ __global__ void __launch_bounds__(kBlock) attn_prefill_split_kernel(AttnPrefillS
   __shared__ prefill_detail::Shared sh;
   const unsigned items = attn_prefill_split_items(p.a.n);
   if (attn_prefill_balanced_blocks(p.a.n) == 2)  // uniform: the block size follows n
-    prefill_detail::prefill_items<2, true>(p.a, &p, 0, items, sh);
+    prefill_detail::prefill_items<2>(p.a, &p, 0, items, sh);
   else
-    prefill_detail::prefill_items<1, true>(p.a, &p, 0, items, sh);
+    prefill_detail::prefill_items<1>(p.a, &p, 0, items, sh);
+}
+
+// Prefill in parts: 8 ceil(workers / 4) workgroups of 256, then the merge.
+template <int kRowBlocks>
+__global__ void __launch_bounds__(256) attn_prefill_parts_kernel(AttnPrefillPartsParams p) {
+  __shared__ prefill_detail::Shared sh;
+  prefill_detail::prefill_items<kRowBlocks>(p.a, &p, 0, gridDim.x, sh);
+}
+
+// Joins the parts of the cut blocks: workgroup (token, KV head) of n x 2, wave w heads 2 w and
+// 2 w + 1, lane l dimensions 4 l .. 4 l + 3. With M the largest m of a row's parts,
+// O = sum O_i 2^(m_i - M) and L = sum l_i 2^(m_i - M) in tile order; core = O / L * sigmoid(gate).
+// Bound by the partials it reads (1 KiB per row and part, mostly from the memory-side cache), so
+// every part of both rows is in flight before the first is used, eight parts at a time.
+template <int kRowBlocks>
+__global__ void __launch_bounds__(256) attn_prefill_merge_kernel(AttnPrefillPartsParams p) {
+  using attn::kDim;
+  constexpr unsigned kTokens = kAttnQBlock * kRowBlocks, kPartRows = 128 * kRowBlocks;
+  constexpr unsigned kGroup = attn::kQHeads / attn::kKvHeads, kBatch = 8;
+  const unsigned tok = blockIdx.x / attn::kKvHeads, kvh = blockIdx.x % attn::kKvHeads;
+  const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const unsigned blk = tok / kTokens;
+  // The block's workers: the last one that starts no later than it, and the last one that
+  // starts before its end.
+  unsigned w0 = 0, w1 = 0;
+#pragma unroll
+  for (unsigned i = 0; i < (kAttnPartsMaxWorkers + 63) / 64; ++i) {
+    const unsigned w = 64 * i + lane;
+    const unsigned at = w < p.cuts.workers ? p.cuts.at[w] : ~0u;
+    w0 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(at <= blk << 23));
+    w1 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(at < (blk + 1) << 23));
+  }
+  if (w0 == w1)  // one worker ran the whole block and stored it
+    return;
+  const unsigned parts = w1 - w0 + 1;
+  // Worker w0 - 1 + i, slot + block as attn_prefill_parts_slots says; rows 8 (token in block) + head.
+  const std::size_t slot0 = std::size_t{kvh} * (p.cuts.workers + p.cuts.blocks) + w0 - 1 + blk;
+  const std::size_t row0 = slot0 * kPartRows + 8 * (tok % kTokens) + 2 * wave;
+  const float* o0 = p.part_o + row0 * kDim + 4 * lane;
+  const float* ml0 = p.part_ml + row0 * 2;
+  const std::size_t gate_at =
+      std::size_t{tok} * p.a.qg_stride + (kvh * kGroup + 2 * wave) * 2 * kDim + kDim + 4 * lane;
+  const float4 g0 = *reinterpret_cast<const float4*>(p.a.qg + gate_at);
+  const float4 g1 = *reinterpret_cast<const float4*>(p.a.qg + gate_at + 2 * kDim);
+  float top[2] = {-__builtin_inff(), -__builtin_inff()}, l[2] = {0.0f, 0.0f};
+  float4 o[2] = {};
+  for (unsigned i0 = 0; i0 < parts; i0 += kBatch) {
+    float4 x[kBatch][2], ml[kBatch];
+#pragma unroll
+    for (unsigned i = 0; i < kBatch; ++i) {
+      const std::size_t at = std::size_t{i0 + i < parts ? i0 + i : parts - 1} * kPartRows;
+      ml[i] = *reinterpret_cast<const float4*>(ml0 + at * 2);  // (m, l) of both rows
+      x[i][0] = *reinterpret_cast<const float4*>(o0 + at * kDim);
+      x[i][1] = *reinterpret_cast<const float4*>(o0 + (at + 1) * kDim);
+    }
+#pragma unroll
+    for (unsigned h = 0; h < 2; ++h) {
+      float mx = top[h];
+#pragma unroll
+      for (unsigned i = 0; i < kBatch; ++i)
+        mx = fmaxf(mx, h == 0 ? ml[i].x : ml[i].z);
+      const float old = __builtin_amdgcn_exp2f(top[h] - mx);  // 0 in the first batch
+      top[h] = mx;
+      l[h] *= old;
+      o[h] = float4{o[h].x * old, o[h].y * old, o[h].z * old, o[h].w * old};
+#pragma unroll
+      for (unsigned i = 0; i < kBatch; ++i) {
+        const float e = i0 + i < parts
+                            ? __builtin_amdgcn_exp2f((h == 0 ? ml[i].x : ml[i].z) - mx)
+                            : 0.0f;
+        l[h] = __builtin_fmaf(h == 0 ? ml[i].y : ml[i].w, e, l[h]);
+        o[h].x = __builtin_fmaf(x[i][h].x, e, o[h].x);
+        o[h].y = __builtin_fmaf(x[i][h].y, e, o[h].y);
+        o[h].z = __builtin_fmaf(x[i][h].z, e, o[h].z);
+        o[h].w = __builtin_fmaf(x[i][h].w, e, o[h].w);
+      }
+    }
+  }
+#pragma unroll
+  for (unsigned h = 0; h < 2; ++h) {
+    const float inv = __builtin_amdgcn_rcpf(l[h]);
+    const float4 g = h == 0 ? g0 : g1;
+    float4 r;
+    r.x = o[h].x * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.x));
+    r.y = o[h].y * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.y));
+    r.z = o[h].z * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.z));
+    r.w = o[h].w * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.w));
+    *reinterpret_cast<float4*>(
+        p.a.core + (std::size_t{tok} * attn::kQHeads + kvh * kGroup + 2 * wave + h) * kDim +
+        4 * lane) = r;
+  }
+}
+
+// Launches the prefill in parts where it pays and the workspace (attn_prefill_parts_workspace_bytes)
+// holds its partials; false if neither kernel was launched.
+inline bool attn_prefill_in_parts(const AttnPrefillParams& a, void* workspace, std::size_t bytes,
+                                  hipStream_t stream) {
+  const unsigned row_blocks = attn_prefill_parts_row_blocks(a.pos0, a.n);
+  if (row_blocks == 0)
+    return false;
+  const unsigned blocks = (a.n + kAttnQBlock * row_blocks - 1) / (kAttnQBlock * row_blocks);
+  if (bytes < kAttnSplitCounterBytes +
+                  attn_prefill_parts_bytes(kAttnPartsMaxWorkers, blocks, row_blocks))
+    return false;
+  AttnPrefillPartsParams p{a, nullptr, nullptr,
+                           attn_prefill_cuts(a.pos0, a.n, row_blocks, kAttnPartsMaxWorkers)};
+  p.part_ml =
+      reinterpret_cast<float*>(static_cast<char*>(workspace) + kAttnSplitCounterBytes);
+  p.part_o = p.part_ml + std::size_t{attn_prefill_parts_slots(p.cuts.workers, blocks)} * 128 *
+                             row_blocks * 2;
+  const unsigned grid = 8 * ((p.cuts.workers + 3) / 4), rows = a.n * attn::kKvHeads;
+  if (row_blocks == 2) {
+    attn_prefill_parts_kernel<2><<<grid, 256, 0, stream>>>(p);
+    attn_prefill_merge_kernel<2><<<rows, 256, 0, stream>>>(p);
+  } else {
+    attn_prefill_parts_kernel<1><<<grid, 256, 0, stream>>>(p);
+    attn_prefill_merge_kernel<1><<<rows, 256, 0, stream>>>(p);
+  }
+  return true;
+}
+
+// The causal prefill with a workspace: in parts, in balanced pairs, or one workgroup per block,
+// whichever the launch's size asks for. The workspace holds the balanced form's where
+// attn_prefill_balanced(n) (the caller checks); a larger one also lets the launch run in parts.
+inline void attn_prefill_launch(const AttnPrefillParams& a, void* workspace, std::size_t bytes,
+                                hipStream_t stream) {
+  if (attn_prefill_in_parts(a, workspace, bytes, stream))
+    return;
+  if (!attn_prefill_balanced(a.n)) {
+    attn_prefill_kernel<256><<<attn_prefill_items(a.n), 256, 0, stream>>>(a);
+    return;
+  }
+  char* const ws = static_cast<char*>(workspace);
+  float* const part_ml = reinterpret_cast<float*>(ws + kAttnSplitCounterBytes);
+  float* const part_o = part_ml + std::size_t{attn_prefill_split_pairs(a.n)} * 2 *
+                                      attn_prefill_split_rows(a.n) * 2;
+  const AttnPrefillSplitParams p{a, part_o, part_ml, reinterpret_cast<unsigned*>(ws)};
+  attn_prefill_split_kernel<256><<<attn_prefill_split_items(a.n), 256, 0, stream>>>(p);
 }
 
 }  // namespace miso::kernels

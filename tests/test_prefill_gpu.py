@@ -199,3 +199,48 @@ def test_prefill_balanced_wide_is_plain(O, attn, torch_mod, prefill_scratch, n):
     assert attn.prefill_workspace_bytes(n) == 0
     assert np.array_equal(run_prefill(attn, torch, p, scratch=prefill_scratch),
                           run_prefill(attn, torch, p))
+
+
+# Prefill in parts (few tokens after a prefix): one row block per wave, a single token block, odd
+# counts and a ragged last block, cuts at and across block ends, a launch above the balanced
+# sizes, and two row blocks per wave.
+PARTS = [(500, 13), (1000, 37), (1001, 100), (700, 256), (12001, 203), (1536, 512), (4099, 700),
+         (3000, 2100), (20000, 1), (33000, 471)]
+
+
+@pytest.mark.parametrize("pos0,n", PARTS)
+def test_prefill_parts_match_oracle(O, attn, torch_mod, prefill_scratch, pos0, n):
+    """The oracle's gate of every other form, and bit-equal on a second call over the workspace."""
+    rng = np.random.default_rng(n + pos0)
+    rows = np.unique(np.concatenate([np.arange(min(n, 17)), np.arange(max(0, n - 33), n),
+                                     rng.choice(n, min(n, 24), replace=False)]))
+    check(O, attn, torch_mod, pos0, n, rows=rows, name="parts", scratch=prefill_scratch)
+    p = O.prefill_inputs(n, pos0, n, pos0 + n + 3, q_scale=2.0)
+    first = run_prefill(attn, torch_mod, p, scratch=prefill_scratch)
+    assert np.array_equal(run_prefill(attn, torch_mod, p, scratch=prefill_scratch), first)
+    plain = run_prefill(attn, torch_mod, p)
+    st = O.compare(first, plain.astype(np.float64))
+    report("parts vs one workgroup per block", st)
+    assert st["ok"], st
+    assert not np.array_equal(first, plain)  # the launch did run in parts
+
+
+def test_prefill_parts_small_workspace(O, attn, torch_mod):
+    """A workspace of the balanced form's size keeps the balanced form (bitwise the result of a
+    launch that never knew parts), and a launch outside both takes no workspace at all."""
+    torch = torch_mod
+    p = O.prefill_inputs(203, 2000, 203, 2203, q_scale=2.0)
+    small = attn.PrefillScratch(203)
+    need = attn.prefill_workspace_bytes(203)
+    assert small.nbytes > need
+    parts = run_prefill(attn, torch, p, scratch=small)
+    small.nbytes = need
+    pairs = run_prefill(attn, torch, p, scratch=small)
+    assert np.array_equal(run_prefill(attn, torch, p, scratch=small), pairs)
+    assert not np.array_equal(parts, pairs)
+    st = O.compare(parts, pairs.astype(np.float64))
+    assert st["ok"], st
+    wide = O.prefill_inputs(2100, 3000, 2100, 5100, q_scale=2.0)
+    small.nbytes = 0
+    assert np.array_equal(run_prefill(attn, torch, wide, scratch=small),
+                          run_prefill(attn, torch, wide))
