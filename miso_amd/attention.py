@@ -190,14 +190,15 @@ def prefill_workspace_bytes(n: int) -> int:
 
 class PrefillScratch:
     """Workspace of miso_attn_prefill_ws for launches of up to max_n tokens (balanced pairs:
-    n <= 2048 and 3841 <= n <= 4096; parts: up to 3072 tokens after a prefix), zero-filled once;
-    every call leaves it reusable."""
+    n <= 2048 and 3841 <= n <= 4096; parts: up to 3072 tokens after a prefix), its pair counters
+    (the first 1 KiB) zeroed once; every call leaves it reusable."""
 
     def __init__(self, max_n: int = 4096, device="cuda"):
         nbytes = max(prefill_workspace_bytes(min(max_n, 2048)),
                      prefill_workspace_bytes(min(max_n, 4096)),
                      int(_lib.load().miso_attn_prefill_parts_workspace_bytes(max_n)))
-        self.buf = torch.zeros(max((nbytes + 3) // 4, 4), dtype=torch.int32, device=device)
+        self.buf = torch.empty(max((nbytes + 3) // 4, 256), dtype=torch.int32, device=device)
+        self.buf[:256].zero_()
         self.nbytes = self.buf.numel() * 4
 
 
@@ -558,9 +559,12 @@ class LayerWorkspace:
         self.max_tok = max_tok
         self.decode = torch.empty(int(lib.miso_attn_layer_decode_ws()), dtype=torch.float32,
                                   device=device)
-        # zero-filled once: the balanced prefill's pair counters sit at its end
-        self.prefill = torch.zeros(max(1, int(lib.miso_attn_layer_prefill_ws(max_tok))),
+        self.prefill = torch.empty(max(1, int(lib.miso_attn_layer_prefill_ws(max_tok))),
                                    dtype=torch.float32, device=device)
+        # only the causal prefill's pair counters (256 after core [max_tok][4096], the GEMM input's
+        # sums [max_tok][128] and its f16 values [max_tok][4096]) have to start at zero
+        at = int(lib.miso_attn_layer_prefill_core(max_tok)) + max_tok * (4096 + 128 + 2048)
+        self.prefill[at:at + 256].zero_()
         # the attention output before the output projection (the engine's scratch.core /
         # ps.core): the last decode step's [16 * 256], the last prefill chunk's [n][16 * 256]
         at = int(lib.miso_attn_layer_decode_core())

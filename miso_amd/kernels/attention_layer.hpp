@@ -21,7 +21,7 @@
 // format mix falls back to one GEMV per matrix), the per-head norms, RoPE and the K/V append
 // (attn_prep), split-K attention over len + 1 keys with the LSE merge and the gate (attn_split +
 // attn_combine), and the output projection. Prefill step (n tokens at pos0): the same with the
-// prefill GEMMs (qgemm_act + qgemm) for the projections, attn_prep_batch, and the causal
+// prefill GEMMs (qgemm_act + qgemm_wide, q / k / v in one launch) for the projections, attn_prep_batch, and the causal
 // attn_prefill. ingest() applies the engine's policy to a run of n tokens: below the threshold one
 // decode step per token, otherwise prefill chunks of at most the chunk size.
 //
@@ -210,23 +210,30 @@ inline void gemm_input(const float* x, unsigned k, unsigned n_tok, _Float16* xh,
   qgemm_act_kernel<<<(quarters + 255) / 256, 256, 0, stream>>>(p);
 }
 
-inline const char* gemm(const Matrix& w, const _Float16* xh, const float* xs, unsigned n_tok,
-                        float* y, unsigned ldy, hipStream_t stream) {
-  if (w.n == 0 || n_tok == 0)
+// Up to three products of the prepared chunk in one launch: Y_i = W_i x with row stride ldy.
+struct GemmOut {
+  const Matrix& w;
+  float* y;
+};
+template <class... Out>
+inline const char* gemm(const _Float16* xh, const float* xs, unsigned n_tok, unsigned ldy,
+                        hipStream_t stream, const Out&... out) {
+  static_assert(sizeof...(Out) >= 1 && sizeof...(Out) <= 3);
+  if (n_tok == 0)
     return nullptr;
-  if (w.k % 256 != 0)
-    return "GEMM k must be a multiple of 256";
-  const QGemmParams p{w.data, xh, xs, y, w.k, w.n, n_tok, ldy};
-  const unsigned grid = qgemm_tiles(w.n, n_tok);
-  if (w.format == Format::Q4K) {
-    if (const unsigned big = qgemm_big_tiles(w.n, n_tok))
-      qgemm_q4k_big_kernel<><<<big, 256, 0, stream>>>(p);
-    else
-      qgemm_kernel<QFormat::Q4K><<<grid, 256, 0, stream>>>(p);
-  } else if (w.format == Format::Q6K)
-    qgemm_kernel<QFormat::Q6K><<<grid, 256, 0, stream>>>(p);
-  else
-    return "weight format must be Q4_K (0) or Q6_K (1)";
+  QGemmBatch b{};
+  for (const GemmOut* o : {static_cast<const GemmOut*>(&out)...}) {
+    if (o->w.n == 0)
+      continue;
+    if (o->w.k % 256 != 0)
+      return "GEMM k must be a multiple of 256";
+    if (o->w.format != Format::Q4K && o->w.format != Format::Q6K)
+      return "weight format must be Q4_K (0) or Q6_K (1)";
+    b.m[b.count] = QGemmParams{o->w.data, xh, xs, o->y, o->w.k, o->w.n, n_tok, ldy};
+    b.format[b.count++] = o->w.format == Format::Q4K ? QFormat::Q4K : QFormat::Q6K;
+  }
+  if (b.count != 0)
+    qgemm_launch(b, stream);
   return nullptr;
 }
 
@@ -362,12 +369,8 @@ inline const char* prefill_step(const Weights& w, attn::half_t* k_cache, attn::h
     return "KV cache is full";
   add_rmsnorm_kernel<<<n, 256, 0, stream>>>(AddRmsNormParams{h, delta, w.attn_norm, ws.xn, eps});
   gemm_input(ws.xn, kHidden, n, ws.xh, ws.xs, stream);
-  const char* err = gemm(w.q, ws.xh, ws.xs, n, ws.proj, kProj, stream);
-  if (err == nullptr)
-    err = gemm(w.k, ws.xh, ws.xs, n, ws.proj + 8192, kProj, stream);
-  if (err == nullptr)
-    err = gemm(w.v, ws.xh, ws.xs, n, ws.proj + 8704, kProj, stream);
-  if (err != nullptr)
+  if (const char* err = gemm(ws.xh, ws.xs, n, kProj, stream, GemmOut{w.q, ws.proj},
+                             GemmOut{w.k, ws.proj + 8192}, GemmOut{w.v, ws.proj + 8704}))
     return err;
   const AttnPrepBatchParams prep{{ws.proj, ws.proj + 8192, ws.proj + 8704, w.q_norm, w.k_norm,
                                   w.inv_freq, k_cache, v_cache, ws.q, pos0, max_ctx, eps},
@@ -377,7 +380,7 @@ inline const char* prefill_step(const Weights& w, attn::half_t* k_cache, attn::h
   const AttnPrefillParams ap{ws.q, ws.proj, k_cache, v_cache, ws.core, pos0, n, max_ctx, kProj};
   attn_prefill_launch(ap, ws.balance, prefill_balance_floats(max_tok) * sizeof(float), stream);
   gemm_input(ws.core, kCore, n, ws.xh, ws.xs, stream);
-  return gemm(w.o, ws.xh, ws.xs, n, y, kHidden, stream);
+  return gemm(ws.xh, ws.xs, n, kHidden, stream, GemmOut{w.o, y});
 }
 
 // n tokens at pos0 through the layer, the engine's policy (src/engine/model.hip:130-175 for this

@@ -30,10 +30,9 @@
 // a contiguous part of that order, so an XCD's activations and weights are read from the memory
 // side about once and reused through its L2.
 //
-// Q4_K products with at least 256 tiles of 128 x 128 can run qgemm_q4k_big_kernel instead (no
-// reference counterpart; qgemm_big_tiles gives its grid, 0 where it does not pay): each wave a
-// 64 x 64 quarter, so an LDS operand read feeds two MFMAs, with the dequantizing store of the
-// next stage in the same step as the MFMAs; results bit-identical to qgemm_kernel's.
+// The layer wiring and the C ABI run qgemm_wide_kernel instead (no reference counterpart): wide
+// tiles fed by LDS DMA in four shapes, up to three products in one launch; qgemm_launch picks the
+// shape. Results are bit-identical to qgemm_kernel's.
 
 #include <hip/hip_runtime.h>
 
@@ -398,124 +397,333 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const QGemmParam
   }
 }
 
-// ---- Q4_K in 128 x 128 tiles (no reference counterpart) ----
-// A workgroup computes 128 tokens x 128 rows, each wave a 64 x 64 quarter (2 x 2 MFMA blocks),
-// so every operand read from LDS feeds two MFMAs instead of one. A stage's tiles are the 64 x 64
-// fetch and store above done twice, at tile rows 0 and 64, and the store of stage s + 1 runs in
-// the same step as the MFMAs of stage s, into the other buffer. Per output element the
-// arithmetic is gemm_tile's in the same order, so both tile shapes give bit-identical results.
-// The LDS (148 KiB) allows one workgroup per CU, against two for the 64 x 64 tiles, so these
-// tiles pay only when they alone fill the chip (qgemm_big_tiles).
-constexpr unsigned kBig = 128, kBigGroupTok = 4;
+// ---- Wide tiles (no reference counterpart) ----
+// A workgroup of WM x WN waves computes kTok tokens x kRow rows, each wave a (kTok / WM) x
+// (kRow / WN) part of it in 32 x 32 MFMA blocks. K advances in stages of 64 (Q4_K: a nibble group
+// of a block; Q6_K: one of the two 64-element sets of a block half).
+//
+// What bounds it: per stage, a wave's LDS operand reads, its share of expanding the weights, its
+// MFMAs and one barrier. Activations (and Q4_K's nibbles, headers and activation sums) come in by
+// LDS DMA, each instruction 1 KiB of whole row segments: fetched into registers row by row, as
+// gemm_tile does, a wave's loads touch 64 separate segments each, which the address unit takes
+// one per cycle -- that was the bound of the 128 x 128 tiles these replace. Two workgroups per CU
+// (or two waves per SIMD in the 256 x 128 tile) let one's expansion and barrier run beside the
+// other's MFMAs. Measured, Q4_K, before and after on one box: 8192 rows x 2048, 4096 tokens 354 ->
+// 196 us (389 -> 702 TFLOP/s), 2048 x 4096, 4096 tokens 158 -> 85 us (435 -> 804); matrix units
+// 40% busy, VALU 36%, LDS 32% (256 x 128): what is left is the lock step of one barrier per stage.
+//
+// Stage s: the MFMAs read activations and expanded weights of stage s while the same threads
+// expand stage s + 1 into the other weight buffer. kRing 3 keeps two stages of activations in
+// flight, with counted waits (the waves then have no other loads); kRing 2 one stage.
+// Per output element the arithmetic is gemm_tile's in the same order: all tile shapes give
+// bit-identical results.
+//
+// LDS tiles are rows of 64 f16 (128 bytes, 8 chunks); chunk c of row r is at position
+// c ^ ((r / 2) % 8), so the 16 rows an operand read takes at once (two rows span the 64 banks) are
+// 16 distinct chunk positions.
+constexpr unsigned kWideK = 64;
 
-struct alignas(16) LdsBig {
-  _Float16 x[2][kBig * kBK];
-  _Float16 w[2][kBig * kBK];
-  _Float16 xm[2][kBig][16];
-  _Float16 wm[2][kBig][16];
-  float dd[2][kBig][4];
+template <unsigned kTok, unsigned kRow, unsigned kRing>
+struct alignas(1024) LdsWide {
+  _Float16 x[kRing][kTok * kWideK];
+  _Float16 w[2][kRow * kWideK];
+  std::uint8_t nib[kRing][kRow][32];  // Q4_K nibbles of a stage
+  std::uint8_t head[2][kRow][16];     // Q4_K block headers; Q6_K by stage parity, 4 f32 scales
+  float xs[kTok][8];                  // Q4_K activation sums of a block
 };
 
-__device__ __attribute__((always_inline)) inline void gemm_tile_big(const QGemmParams& p,
-                                                                    LdsBig& sm, unsigned m0,
-                                                                    unsigned n0) {
-  constexpr QFormat F = QFormat::Q4K;
-  const unsigned t = threadIdx.x, lane = t % 64, wave = t / 64;
-  const unsigned wt = wave >> 1, wr = wave & 1u, kq = lane / 32;
-  unsigned ar[2], br[2];  // the lane's token rows and weight rows in the tile, per MFMA block
+template <QFormat F, unsigned kTok, unsigned kRow, unsigned WM, unsigned WN, unsigned kRing>
+__device__ __attribute__((always_inline)) inline void gemm_tile_wide(
+    const QGemmParams& p, LdsWide<kTok, kRow, kRing>& sm, unsigned m0, unsigned n0) {
+  constexpr bool kQ4 = F == QFormat::Q4K;
+  constexpr unsigned kWaves = WM * WN, MB = kTok / 32 / WM, NB = kRow / 32 / WN;
+  constexpr unsigned kXInstr = kTok / 8 / kWaves;  // activation DMAs per wave and stage
+  static_assert(kRow * 4 == 64 * kWaves, "four threads expand a row's stage");
+  static_assert(kTok / 32 <= kWaves && kXInstr >= 1 && MB >= 1 && NB >= 1);
+  static_assert(kRing == 2 || kRing == 3);
+  const unsigned t = threadIdx.x, lane = t % 64;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(t / 64);
+  const unsigned wt = wave / WN, wr = wave % WN, col = lane % 32, kq = lane / 32;
+  const unsigned n_stages = p.k / kWideK;
+  const std::size_t row_b = row_bytes<F>(p.k);
+
+  // This lane's sources (rows and tokens past the end read the last one; their results are not
+  // stored). Activations: instruction i of the wave moves tile rows 8 (kXInstr wave + i) .. + 7,
+  // lane l chunk (l % 8) ^ ((row / 2) % 8) of row l / 8.
+  const _Float16* xsrc[kXInstr];
 #pragma unroll
-  for (unsigned i = 0; i < 2; ++i) {
-    ar[i] = 64 * wt + 32 * i + lane % 32;
-    br[i] = 64 * wr + 32 * i + lane % 32;
+  for (unsigned i = 0; i < kXInstr; ++i) {
+    const unsigned r = 8 * (kXInstr * wave + i) + lane / 8;
+    const unsigned tok = m0 + r < p.n_tok ? m0 + r : p.n_tok - 1;
+    xsrc[i] = p.xh + std::size_t{tok} * p.k + 8 * ((lane % 8) ^ ((r / 2) % 8));
   }
-  const unsigned n_stages = p.k / kBK;
-  bool tok_ok[2], row_ok[2];
+  auto w_row = [&](unsigned r) __attribute__((always_inline)) {
+    const unsigned row = n0 + r < p.n_rows ? n0 + r : p.n_rows - 1;
+    return p.w + row * row_b;
+  };
+  const unsigned x_lds = cdna4::lds_offset(sm.x);
+  // Stages and blocks past the end re-read the last one into a buffer that nothing reads again.
+  auto load_x = [&](unsigned s, unsigned slot) __attribute__((always_inline)) {
+    const unsigned at = kWideK * (s < n_stages ? s : n_stages - 1);
 #pragma unroll
-  for (unsigned h = 0; h < 2; ++h) {
-    tok_ok[h] = m0 + 64 * h + t / 4 < p.n_tok;
-    row_ok[h] = n0 + 64 * h + t / 4 < p.n_rows;
+    for (unsigned i = 0; i < kXInstr; ++i)
+      cdna4::lds_load16(xsrc[i] + at,
+                        x_lds + slot * (kTok * kWideK * 2) + 1024 * (kXInstr * wave + i));
+  };
+  auto barrier = []() __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+
+  // Q4_K: nibbles (32 rows an instruction), headers (64 rows) and activation sums (32 tokens) by
+  // the first waves, one instruction each.
+  const bool nib_wave = wave < kRow / 32, head_wave = wave < kRow / 64, xs_wave = wave < kTok / 32;
+  const std::uint8_t* nsrc = w_row(32 * (wave % (kRow / 32)) + lane / 2) + 16 + 16 * (lane % 2);
+  const std::uint8_t* hsrc = w_row(64 * (wave % (kRow / 64)) + lane);
+  const float* ssrc = nullptr;
+  if constexpr (kQ4) {
+    const unsigned r = 32 * (wave % (kTok / 32)) + lane / 2;
+    const unsigned tok = m0 + r < p.n_tok ? m0 + r : p.n_tok - 1;
+    ssrc = p.xs + std::size_t{tok} * (p.k / 32) + 4 * (lane % 2);
   }
-  auto fetch2 = [&](Fetch<F> (&f)[2], unsigned s) __attribute__((always_inline)) {
-    f[0] = fetch<F>(p, n0, m0, s, t);
-    f[1] = fetch<F>(p, n0 + 64, m0 + 64, s, t);
+  const unsigned nib_lds = cdna4::lds_offset(sm.nib), head_lds = cdna4::lds_offset(sm.head);
+  const unsigned xs_lds = cdna4::lds_offset(sm.xs);
+  auto load_nib = [&](unsigned s, unsigned slot) __attribute__((always_inline)) {
+    s = s < n_stages ? s : n_stages - 1;
+    cdna4::lds_load16(nsrc + 144 * (s / 4) + 32 * (s % 4),
+                      nib_lds + slot * (kRow * 32) + 1024 * wave);
   };
-  auto store2 = [&](const Fetch<F> (&f)[2], unsigned s) __attribute__((always_inline)) {
-    store<F, LdsBig>(f[0], sm, s, t, tok_ok[0], row_ok[0], 0);
-    store<F, LdsBig>(f[1], sm, s, t, tok_ok[1], row_ok[1], 64);
+  auto load_head = [&](unsigned b) __attribute__((always_inline)) {
+    const unsigned at = 4 * b < n_stages ? b : n_stages / 4 - 1;
+    cdna4::lds_load16(hsrc + 144 * at, head_lds + (b & 1u) * (kRow * 16) + 1024 * wave);
   };
-  float16_t acc[2][2], c[2][2];
+  auto load_xs = [&](unsigned b) __attribute__((always_inline)) {
+    cdna4::lds_load16(ssrc + 8 * b, xs_lds + 1024 * wave);
+  };
+  // With kRing 3 every DMA of stage s - 2 and before has landed when only those of stage s - 1 are
+  // outstanding (the activations' and `extra` more); with kRing 2 (and Q6_K) all have to be in.
+  auto wait = [&](unsigned extra) __attribute__((always_inline)) {
+    if (kRing == 2 || !kQ4)
+      cdna4::wait_vmcnt<0>();
+    else if (extra == 0)
+      cdna4::wait_vmcnt<kXInstr>();
+    else if (extra == 1)
+      cdna4::wait_vmcnt<kXInstr + 1>();
+    else
+      cdna4::wait_vmcnt<kXInstr + 2>();
+  };
+
+  // Expansion of a stage into weight buffer s % 2 by thread (row er = t / 4, quarter eq = t % 4).
+  const unsigned er = t / 4, eq = t % 4, eswz = (er / 2) % 8;
+  auto put_w = [&](unsigned s, unsigned c, u32x4 v) __attribute__((always_inline)) {
+    *reinterpret_cast<u32x4*>(sm.w[s & 1u] + kWideK * er + 8 * (c ^ eswz)) = v;
+  };
+  // Q4_K: bytes 8 eq .. 8 eq + 7 of the group's 32: weights 8 eq + i (low), 32 + 8 eq + i (high).
+  auto expand_q4 = [&](unsigned s, unsigned slot) __attribute__((always_inline)) {
+    using namespace q4k_gemv_detail;
+    const uint2 raw = *reinterpret_cast<const uint2*>(&sm.nib[slot][er][8 * eq]);
+    const u32x4 head = *reinterpret_cast<const u32x4*>(&sm.head[(s / 4) & 1u][er][0]);
+    const unsigned fld = scale_field(head, s % 4);
+    const float sc_lo = static_cast<float>(fld & 63u), sc_hi = static_cast<float>((fld >> 12) & 63u);
+    const half2_t s_lo = splat(sc_lo), c_lo = splat(-1024.0f * sc_lo);
+    const half2_t s_hi = splat(sc_hi * 0.0625f), c_hi = splat(-64.0f * sc_hi);
+    unsigned lo[4], hi[4];
 #pragma unroll
-  for (unsigned i = 0; i < 2; ++i)
+    for (int d = 0; d < 2; ++d)
 #pragma unroll
-    for (unsigned j = 0; j < 2; ++j)
-      acc[i][j] = c[i][j] = float16_t{};
-  // Two register sets, even and odd stages, each requested two stages before its store.
-  Fetch<F> fa[2], fb[2];
-  fetch2(fa, 0);
-  asm volatile("" : : : "memory");  // stage 0's loads are issued before stage 1's
-  fetch2(fb, 1);
-  store2(fa, 0);
-  fetch2(fa, 2);
-  auto step = [&](Fetch<F> (&fn)[2], unsigned s) __attribute__((always_inline)) {
-    __builtin_amdgcn_sched_barrier(0);
-    // Stage s complete in its buffer, and every wave done with the other one (stage s - 1).
-    __syncthreads();
-    // Also at the last stage (a re-read of it into the buffer and block parity nothing reads
-    // again), so that the store shares one scheduling region with the MFMAs.
-    store2(fn, s + 1);
-    fetch2(fn, s + 3);  // past the last stage: re-reads it
-    const unsigned buf = s & 1u;
-#pragma unroll
-    for (unsigned kk = 0; kk < kBK / 16; ++kk) {
-      half8_t a[2], b[2];
-#pragma unroll
-      for (unsigned i = 0; i < 2; ++i) {
-        a[i] = *reinterpret_cast<const half8_t*>(sm.x[buf] + chunk_at(ar[i], 2 * kk + kq));
-        b[i] = *reinterpret_cast<const half8_t*>(sm.w[buf] + chunk_at(br[i], 2 * kk + kq));
+      for (int i = 0; i < 2; ++i) {
+        const unsigned b = spread_bytes(d == 0 ? raw.x : raw.y, i);
+        lo[2 * d + i] = cdna4::as_uint(int_pair(b, 0x000F000Fu, s_lo, c_lo));
+        hi[2 * d + i] = cdna4::as_uint(int_pair(b, 0x00F000F0u, s_hi, c_hi));
       }
+    put_w(s, eq, u32x4{lo[0], lo[1], lo[2], lo[3]});
+    put_w(s, 4 + eq, u32x4{hi[0], hi[1], hi[2], hi[3]});
+  };
+  // Q6_K: elements 16 eq .. 16 eq + 15 of the set (stage 2 h': low nibbles, 2 h' + 1: high), one
+  // scale group. A block half's bytes serve both of its stages; they are fetched into registers
+  // one half ahead.
+  struct Half {
+    u32x4 ql, qh;
+    unsigned sc[2], d;  // scale bytes of the two sets' groups, f16 d
+  };
+  const std::uint8_t* qrow = w_row(er);
+  const unsigned nb = p.k / 256;
+  auto fetch_half = [&](unsigned h) __attribute__((always_inline)) {
+    h = h < 2 * nb ? h : 2 * nb - 1;
+    Half f;
+    f.ql = *reinterpret_cast<const u32x4*>(qrow + 64 * h + 16 * eq);
+    f.qh = *reinterpret_cast<const u32x4*>(qrow + nb * 128 + 32 * h + 16 * (eq & 1u));
+    const std::uint8_t* sc = qrow + nb * 192 + 8 * h + eq;
+    f.sc[0] = sc[0];
+    f.sc[1] = sc[4];
+    f.d = *reinterpret_cast<const unsigned short*>(qrow + nb * 208 + 2 * (h / 2));
+    return f;
+  };
+  auto expand_q6 = [&](unsigned s, const Half& f) __attribute__((always_inline)) {
+    const unsigned l[4] = {f.ql.x, f.ql.y, f.ql.z, f.ql.w};
+    const unsigned h[4] = {f.qh.x, f.qh.y, f.qh.z, f.qh.w};
+    unsigned v[8];
 #pragma unroll
-      for (unsigned i = 0; i < 2; ++i)
+    for (int d = 0; d < 4; ++d)
 #pragma unroll
-        for (unsigned j = 0; j < 2; ++j)
-          c[i][j] = mfma(a[i], b[j], c[i][j]);
-    }
-    if (s % 2 == 1) {  // the block's last stage: its dmin m term, then its d scale
-      const unsigned bb = (s / 2) & 1u;
+      for (int i = 0; i < 2; ++i) {
+        const q6k_gemv_detail::CodePairs c =
+            q6k_gemv_detail::code_pairs(l[d], h[d], i, 2 * (eq / 2));
+        v[2 * d + i] = cdna4::as_uint((s & 1u) == 0 ? c.lo : c.hi16);
+      }
+    put_w(s, 2 * eq, u32x4{v[0], v[1], v[2], v[3]});
+    put_w(s, 2 * eq + 1, u32x4{v[4], v[5], v[6], v[7]});
+    const float d = q4k_gemv_detail::f16_bits(f.d) * ((s & 1u) == 0 ? 1.0f : 0.0625f);
+    reinterpret_cast<float*>(sm.head[s & 1u][er])[eq] =
+        d * static_cast<float>(static_cast<signed char>(f.sc[s & 1u]));
+  };
+
+  float16_t acc[MB][NB], c[MB][NB];
 #pragma unroll
-      for (unsigned j = 0; j < 2; ++j) {
-        const half8_t bm = *reinterpret_cast<const half8_t*>(&sm.wm[bb][br[j]][8 * kq]);
-        const float d = sm.dd[bb][br[j]][0], dmin = sm.dd[bb][br[j]][1];
+  for (unsigned i = 0; i < MB; ++i)
 #pragma unroll
-        for (unsigned i = 0; i < 2; ++i) {
-          const half8_t am = *reinterpret_cast<const half8_t*>(&sm.xm[bb][ar[i]][8 * kq]);
-          const float16_t mins = mfma(am, bm, float16_t{});
+    for (unsigned j = 0; j < NB; ++j)
+      acc[i][j] = c[i][j] = float16_t{};
+
+  Half raw{}, ahead{};
+  if constexpr (kQ4) {
+    if (head_wave)
+      load_head(0);
+    if (nib_wave)
+      for (unsigned s = 0; s < kRing; ++s)
+        load_nib(s, s);
+  } else {
+    raw = fetch_half(0);
+  }
+  for (unsigned s = 0; s + 1 < kRing; ++s)
+    load_x(s, s);
+  cdna4::wait_vmcnt<0>();
+  barrier();
+  if constexpr (kQ4)
+    expand_q4(0, 0);
+  else
+    expand_q6(0, raw);
+
+  // Operand addresses: row 32 i + col of a tile, chunk 2 kk + kq.
+  unsigned at[4];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            acc[i][j][r] = __builtin_fmaf(d, c[i][j][r], acc[i][j][r]);
-            acc[i][j][r] = __builtin_fmaf(-dmin, mins[r], acc[i][j][r]);
+  for (unsigned kk = 0; kk < 4; ++kk)
+    at[kk] = kWideK * col + 8 * ((2 * kk + kq) ^ ((col / 2) % 8));
+  unsigned cur = 0, nxt = 1, spare = kRing - 1;  // ring slots of stages s, s + 1, s + kRing - 1
+  for (unsigned s4 = 0; s4 < n_stages; s4 += 4) {
+#pragma unroll
+    for (unsigned j = 0; j < 4; ++j) {
+      const unsigned s = s4 + j;
+      // What stage s - 1 issued besides its activations (everything of the prologue is in).
+      wait((nib_wave ? 1u : 0u) + (j == 1 && xs_wave ? 1u : 0u) + (j == 2 && head_wave ? 1u : 0u));
+      barrier();  // stage s complete for every wave, and every wave done with stage s - 1
+      load_x(s + kRing - 1, spare);
+      if constexpr (kQ4) {
+        if (nib_wave)
+          load_nib(s + kRing, cur);  // slot of stage s, expanded in stage s - 1
+        if (j == 0 && xs_wave)
+          load_xs(s4 / 4);  // read at j == 3; the last block's were read before this barrier
+        if (j == 1 && head_wave)
+          load_head(s4 / 4 + 1);  // expanded from at j == 3
+      } else if (j % 2 == 0) {
+        ahead = fetch_half(s / 2 + 1);
+      }
+      const _Float16* xt = sm.x[0] + cur * (kTok * kWideK) + 32 * kWideK * MB * wt;
+      const _Float16* wtile = sm.w[j & 1u] + 32 * kWideK * NB * wr;
+      float4 scale[NB];
+      if constexpr (!kQ4)
+#pragma unroll
+        for (unsigned n = 0; n < NB; ++n)
+          scale[n] =
+              *reinterpret_cast<const float4*>(sm.head[j & 1u][32 * (NB * wr + n) + col]);
+#pragma unroll
+      for (unsigned kk = 0; kk < 4; ++kk) {
+        half8_t a[MB], b[NB];
+#pragma unroll
+        for (unsigned i = 0; i < MB; ++i)
+          a[i] = *reinterpret_cast<const half8_t*>(xt + 32 * kWideK * i + at[kk]);
+#pragma unroll
+        for (unsigned i = 0; i < NB; ++i)
+          b[i] = *reinterpret_cast<const half8_t*>(wtile + 32 * kWideK * i + at[kk]);
+#pragma unroll
+        for (unsigned i = 0; i < MB; ++i)
+#pragma unroll
+          for (unsigned n = 0; n < NB; ++n) {
+            if constexpr (kQ4) {
+              c[i][n] = mfma(a[i], b[n], c[i][n]);
+            } else {  // one scale group per k-step
+              const float16_t g = mfma(a[i], b[n], float16_t{});
+              const float sc = kk == 0   ? scale[n].x
+                               : kk == 1 ? scale[n].y
+                               : kk == 2 ? scale[n].z
+                                         : scale[n].w;
+#pragma unroll
+              for (int r = 0; r < 16; ++r)
+                acc[i][n][r] = __builtin_fmaf(sc, g[r], acc[i][n][r]);
+            }
           }
-          c[i][j] = float16_t{};
+      }
+      // Past the last stage: into the buffer that nothing reads again.
+      if constexpr (kQ4) {
+        expand_q4(s + 1, nxt);
+      } else {
+        if (j % 2 == 1)
+          raw = ahead;
+        expand_q6(s + 1, raw);
+      }
+      if (kQ4 && j == 3) {  // the block's dmin m term, then its d scale
+#pragma unroll
+        for (unsigned n = 0; n < NB; ++n) {
+          const u32x4 head = *reinterpret_cast<const u32x4*>(
+              &sm.head[(s4 / 4) & 1u][32 * (NB * wr + n) + col][0]);
+          half8_t bm;
+#pragma unroll
+          for (unsigned g = 0; g < 2; ++g) {
+            const unsigned f = q4k_gemv_detail::scale_field(head, 2 * kq + g);
+            const float me = static_cast<float>((f >> 6) & 63u), mo = static_cast<float>(f >> 18);
+            bm[4 * g] = static_cast<_Float16>(me);
+            bm[4 * g + 1] = static_cast<_Float16>(me * 0x1p-11f);
+            bm[4 * g + 2] = static_cast<_Float16>(mo);
+            bm[4 * g + 3] = static_cast<_Float16>(mo * 0x1p-11f);
+          }
+          const float d = q4k_gemv_detail::f16_bits(head.x & 0xFFFFu);
+          const float dmin = q4k_gemv_detail::f16_bits(head.x >> 16) * 0x1p6f;
+#pragma unroll
+          for (unsigned i = 0; i < MB; ++i) {
+            const float4 v =
+                *reinterpret_cast<const float4*>(&sm.xs[32 * (MB * wt + i) + col][4 * kq]);
+            const half2_t h[4] = {split(v.x), split(v.y), split(v.z), split(v.w)};
+            const half8_t am = {h[0][0], h[0][1], h[1][0], h[1][1],
+                                h[2][0], h[2][1], h[3][0], h[3][1]};
+            const float16_t mins = mfma(am, bm, float16_t{});
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              acc[i][n][r] = __builtin_fmaf(d, c[i][n][r], acc[i][n][r]);
+              acc[i][n][r] = __builtin_fmaf(-dmin, mins[r], acc[i][n][r]);
+            }
+            c[i][n] = float16_t{};
+          }
         }
       }
+      const unsigned tmp = cur;
+      cur = nxt;
+      nxt = kRing == 2 ? tmp : spare;
+      spare = kRing == 2 ? nxt : tmp;
     }
-  };
-  for (unsigned s = 0; s < n_stages; s += 2) {  // n_stages is even (k % 256 == 0)
-    step(fb, s);
-    step(fa, s + 1);
   }
-  // Lane (row br[j], half kq) holds tokens 8 (r / 4) + 4 kq + r % 4 of token block i.
+  // Lane (row col of block n, half kq) holds tokens 8 (r / 4) + 4 kq + r % 4 of token block i.
 #pragma unroll
-  for (unsigned j = 0; j < 2; ++j) {
-    const unsigned n = n0 + br[j];
+  for (unsigned n = 0; n < NB; ++n) {
+    const unsigned row = n0 + 32 * (NB * wr + n) + col;
 #pragma unroll
-    for (unsigned i = 0; i < 2; ++i)
+    for (unsigned i = 0; i < MB; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const unsigned tok = m0 + 64 * wt + 32 * i + 8 * (r / 4) + 4 * kq + r % 4;
-        if (tok < p.n_tok && n < p.n_rows)
-          p.y[std::size_t{tok} * p.ldy + n] = acc[i][j][r];
+        const unsigned tok = m0 + 32 * (MB * wt + i) + 8 * (r / 4) + 4 * kq + r % 4;
+        if (tok < p.n_tok && row < p.n_rows)
+          p.y[std::size_t{tok} * p.ldy + row] = acc[i][n][r];
       }
   }
+  cdna4::wait_vmcnt<0>();  // every DMA has landed before the workgroup's LDS is given away
 }
 
 // The 64 x 64 tiles [first, first + count), in grouped_tile's order.
@@ -550,31 +758,88 @@ __global__ void __launch_bounds__(qgemm_detail::kThreads) qgemm_kernel(QGemmPara
   qgemm_op<F>(p, 0, qgemm_tiles(p.n_rows, p.n_tok));
 }
 
-// Workgroups for a Q4_K product in 128 x 128 tiles, or 0 where 64 x 64 tiles are faster (at most
-// 64 tokens, or fewer 128 x 128 tiles than the 256 CUs: the 64 x 64 kernel then runs two
-// workgroups per CU). No reference counterpart: callers that know it launch
-// qgemm_q4k_big_kernel on this many workgroups of 256 threads, else qgemm_kernel<Q4K>.
-__host__ __device__ inline unsigned qgemm_big_tiles(unsigned n_rows, unsigned n_tok) {
+// Up to three products over one prepared chunk (the q, k and v projections) in one launch: the
+// same xh, xs, k and n_tok, each its own weights, format, rows and output.
+struct QGemmBatch {
+  QGemmParams m[3];
+  QFormat format[3];
+  unsigned count;
+};
+
+// One workgroup per kTok x kRow tile of every product. The row tiles of products 1 and 2 are
+// spread evenly among product 0's, so every XCD (a contiguous part of the tile order, see xcd_tile)
+// gets its share of each format.
+template <unsigned kTok, unsigned kRow, unsigned WM, unsigned WN, unsigned kRing,
+          unsigned kWavesPerSimd, unsigned kGroup>
+__global__ void __launch_bounds__(64 * WM * WN, kWavesPerSimd) qgemm_wide_kernel(QGemmBatch p) {
   using namespace qgemm_detail;
-  const unsigned tiles = (n_rows + kBig - 1) / kBig * ((n_tok + kBig - 1) / kBig);
-  return n_tok > kBM && tiles >= 256 ? tiles : 0;
+  __shared__ LdsWide<kTok, kRow, kRing> sm;
+  const unsigned n_tok = p.m[0].n_tok;
+  unsigned rt[3], all = 0;
+#pragma unroll
+  for (unsigned i = 0; i < 3; ++i) {
+    rt[i] = i < p.count ? (p.m[i].n_rows + kRow - 1) / kRow : 0;
+    all += rt[i];
+  }
+  const unsigned n_ttiles = (n_tok + kTok - 1) / kTok;
+  unsigned ttile, r;
+  grouped_tile<kGroup>(xcd_tile(blockIdx.x, n_ttiles * all), n_ttiles, all, ttile, r);
+  unsigned which = 0;
+#pragma unroll
+  for (unsigned i = 2; i > 0; --i) {  // is place r of `all` one of product i's rt[i]?
+    if (which == 0 && rt[i] != 0) {
+      const unsigned before = r * rt[i] / all;
+      if ((r + 1) * rt[i] / all > before)
+        which = i, r = before;
+      else
+        r -= before, all -= rt[i];
+    }
+  }
+  const QGemmParams q = which == 0 ? p.m[0] : which == 1 ? p.m[1] : p.m[2];
+  const QFormat f = which == 0 ? p.format[0] : which == 1 ? p.format[1] : p.format[2];
+  if (f == QFormat::Q4K)
+    gemm_tile_wide<QFormat::Q4K, kTok, kRow, WM, WN, kRing>(q, sm, ttile * kTok, r * kRow);
+  else
+    gemm_tile_wide<QFormat::Q6K, kTok, kRow, WM, WN, kRing>(q, sm, ttile * kTok, r * kRow);
 }
 
-// The whole Q4_K product in 128 x 128 tiles (grid-stride over qgemm_big_tiles' tile count, in
-// grouped_tile's order with groups of 4 token tiles). A template, so several translation units
-// may include this header.
-template <int = 0>
-__global__ void __launch_bounds__(qgemm_detail::kThreads) qgemm_q4k_big_kernel(QGemmParams p) {
-  using namespace qgemm_detail;
-  __shared__ LdsBig sm;
-  const unsigned n_ttiles = (p.n_tok + kBig - 1) / kBig, n_rtiles = (p.n_rows + kBig - 1) / kBig;
-  const unsigned count = n_ttiles * n_rtiles;
-  for (unsigned i = blockIdx.x; i < count; i += gridDim.x) {
-    const unsigned tile = gridDim.x == count ? xcd_tile(i, count) : i;
-    unsigned ttile, rtile;
-    grouped_tile<kBigGroupTok>(tile, n_ttiles, n_rtiles, ttile, rtile);
-    gemm_tile_big(p, sm, ttile * kBig, rtile * kBig);
-    __syncthreads();  // the next tile's first stores reuse buffer 0
+// The tile shape with the least estimated time: a CU's tiles, in rounds of as many workgroups as
+// fit on it together. Times of a round by workgroups per CU, in us per 2048 of k (one MI355X,
+// Q4_K, HBM-resident weights):
+//   64 x 64     13, 18, 24 (three together)     128 x 64    17, 28
+//   128 x 128   24, 50                          256 x 128   48 (one fills the CU)
+// so small launches take small tiles (more CUs, shorter stages) and full chips large ones (fewer
+// LDS bytes and expansions per MFMA): 512 tokens x 8192 rows 38 / 34 / 33 / 40 us in this order,
+// 200 tokens 22 / 20 / 27 / 37, 4096 tokens 263 / 229 / 199 / 196.
+// kGroup (token tiles swept across the row tiles) keeps the ~32 to 96 tiles an XCD runs at once
+// within its 4 MiB of L2 also at k = 4096: 2048 rows x 4096, 512 tokens in 64 x 64 tiles 36 us
+// in groups of 8, 31 in groups of 4.
+inline void qgemm_launch(const QGemmBatch& p, hipStream_t stream) {
+  auto tiles = [&](unsigned tok, unsigned row) {
+    unsigned rows = 0;
+    for (unsigned i = 0; i < p.count; ++i)
+      rows += (p.m[i].n_rows + row - 1) / row;
+    return rows * ((p.m[0].n_tok + tok - 1) / tok);
+  };
+  constexpr unsigned kShapes = 4;
+  const unsigned count[kShapes] = {tiles(64, 64), tiles(128, 64), tiles(128, 128),
+                                   tiles(256, 128)};
+  constexpr unsigned kTogether[kShapes] = {3, 2, 2, 1};
+  constexpr unsigned kRound[kShapes][4] = {{0, 13, 18, 24}, {0, 17, 28}, {0, 24, 50}, {0, 48}};
+  unsigned best = 0;
+  std::uint64_t least = ~std::uint64_t{0};
+  for (unsigned i = 0; i < kShapes; ++i) {
+    const unsigned per_cu = (count[i] + 255) / 256, full = per_cu / kTogether[i];
+    const std::uint64_t t = std::uint64_t{full} * kRound[i][kTogether[i]] +
+                            kRound[i][per_cu % kTogether[i]];
+    if (t < least)
+      best = i, least = t;
+  }
+  switch (best) {
+    case 0: qgemm_wide_kernel<64, 64, 2, 2, 2, 2, 4><<<count[0], 256, 0, stream>>>(p); break;
+    case 1: qgemm_wide_kernel<128, 64, 2, 2, 2, 2, 2><<<count[1], 256, 0, stream>>>(p); break;
+    case 2: qgemm_wide_kernel<128, 128, 2, 4, 2, 4, 2><<<count[2], 512, 0, stream>>>(p); break;
+    default: qgemm_wide_kernel<256, 128, 4, 2, 3, 2, 4><<<count[3], 512, 0, stream>>>(p); break;
   }
 }
 

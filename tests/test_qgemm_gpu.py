@@ -201,3 +201,24 @@ def test_python_layer_reference_errors(attn, torch_mod):
         attn.gemm(w, "q4_k", 8, 4096, inp, y, 8)
     with pytest.raises(RuntimeError, match="gemm: unsupported type"):
         attn.gemm(w, "q8_0", 8, 2048, inp, y, 8)
+
+
+@pytest.mark.parametrize("k,n,n_tok", [(2048, 8192, 33), (2048, 2000, 700), (2048, 8100, 515),
+                                       (4096, 2048, 4000), (2048, 9216, 1025), (256, 130, 260)])
+def test_wide_tiles_bit_identical(O, attn, torch_mod, k, n, n_tok):
+    """Every tile shape qgemm_launch picks (64 x 64, 128 x 64, 128 x 128, 256 x 128 here, the last
+    token and row tiles partial, and one block of k) against the 64 x 64 kernel's arithmetic: a
+    product of at most 64 tokens takes 64 x 64 tiles, so 64 tokens at a time give the same bits;
+    the first 64 also meet the reference test's bound."""
+    torch = torch_mod
+    rng = np.random.default_rng(k + n + n_tok)
+    for fmt in ("q4_k", "q6_k"):
+        if fmt == "q6_k" and n_tok > 700:
+            continue
+        blocks = random_blocks(rng, n, k) if fmt == "q4_k" else random_q6k_blocks(rng, n, k)
+        x = xs_normal(rng, n_tok, k)
+        whole = run_gemm(O, attn, torch, fmt, blocks, n, k, x, n + 3)
+        parts = np.concatenate([run_gemm(O, attn, torch, fmt, blocks, n, k, x[t:t + 64], n + 3)
+                                for t in range(0, n_tok, 64)])
+        assert np.array_equal(whole, parts), fmt
+        check(O, attn, torch, fmt, blocks, n, k, x[:5], "wide")
