@@ -17,6 +17,8 @@
 #include <cstdint>
 #include <type_traits>
 
+#include <type_traits>
+
 #include "cdna4_wave.hpp"
 
 namespace miso::kernels {
@@ -880,6 +882,157 @@ __device__ __attribute__((always_inline)) inline void issue_rows8(const void* kt
       : "memory");
 }
 
+// Where a split's queries come from. A pointer: rows [16][256], normalised and rotated. PrepQuery:
+// the projections of the decode step's token at position pos, prepared here (the decode prep of one
+// launch less: attn_prep_head's arithmetic, the rotation read from a table). Every workgroup prepares
+// its KV head's 8 query rows, wave w rows 2 w and 2 w + 1, while its first tiles are in flight.
+// The cache does not hold the token's K and V yet: the wave that copies its row's tile group
+// prepares them, puts them into the tile in LDS (the copy re-read the row before) and stores them.
+struct PrepShared {
+  float norm[kWaves][attn::kDim];
+  float rope[kWaves][attn::kDim];  // cos [32], sin [32], each four times over
+  float token[3][attn::kDim];      // the owner's K row, k_norm, V row
+};
+struct PrepQuery {
+  const float* proj;  // [16][512] query and gate rows, then K [2][256], V [2][256]
+  const float* q_norm;
+  const float* k_norm;
+  const float* rope;  // [64]
+  attn::half_t* k_row;  // this KV head's row pos of the cache
+  attn::half_t* v_row;
+  PrepShared* sh;
+  float eps;
+  unsigned pos;
+};
+
+// The token's row in a split's tiles: tile `tile`, tile row `row` (tile ~0u: not in this split).
+struct TokenPlace {
+  unsigned tile, row;
+};
+__device__ __attribute__((always_inline)) inline TokenPlace token_place(const float*, AttnSpan) {
+  return {~0u, 0};
+}
+__device__ __attribute__((always_inline)) inline TokenPlace token_place(const PrepQuery& qs,
+                                                                       AttnSpan span) {
+  if (qs.pos < span.begin || qs.pos >= span.end)
+    return {~0u, 0};
+  return {(qs.pos - span.begin) / 32, (qs.pos - span.begin) % 32};
+}
+// The last row of a split that the cache holds.
+__device__ __attribute__((always_inline)) inline unsigned last_cached_row(const float*,
+                                                                         AttnSpan span) {
+  return span.end - 1;
+}
+__device__ __attribute__((always_inline)) inline unsigned last_cached_row(const PrepQuery& qs,
+                                                                         AttnSpan span) {
+  return span.end - 1 < qs.pos ? span.end - 1 : qs.pos - 1;  // pos >= 1
+}
+
+// Requests the KV head's query rows into q (wave w: rows 2 w, 2 w + 1) and what the preparation
+// needs, by LDS DMA.
+__device__ __attribute__((always_inline)) inline void issue_queries(const float* src, float (*q)[256],
+                                                                   unsigned kvh, unsigned wave,
+                                                                   unsigned lane, bool) {
+#pragma unroll
+  for (unsigned i = 0; i < 2; ++i) {
+    const unsigned h = 2 * wave + i;
+    cdna4::lds_load16(src + (std::size_t{kvh} * kGroup + h) * attn::kDim + 4 * lane,
+                      cdna4::lds_offset(q[h]));
+  }
+}
+__device__ __attribute__((always_inline)) inline void issue_queries(const PrepQuery& qs,
+                                                                   float (*q)[256], unsigned kvh,
+                                                                   unsigned wave, unsigned lane,
+                                                                   bool owner) {
+#pragma unroll
+  for (unsigned i = 0; i < 2; ++i) {
+    const unsigned h = 2 * wave + i;
+    cdna4::lds_load16(qs.proj + (std::size_t{kvh} * kGroup + h) * 2 * attn::kDim + 4 * lane,
+                      cdna4::lds_offset(q[h]));
+  }
+  cdna4::lds_load16(qs.q_norm + 4 * lane, cdna4::lds_offset(qs.sh->norm[wave]));
+  cdna4::lds_load16(qs.rope + 4 * (lane % 16), cdna4::lds_offset(qs.sh->rope[wave]));
+  if (owner) {  // uniform
+    const float* k = qs.proj + 16 * 2 * attn::kDim + kvh * attn::kDim;
+    cdna4::lds_load16(k + 4 * lane, cdna4::lds_offset(qs.sh->token[0]));
+    cdna4::lds_load16(qs.k_norm + 4 * lane, cdna4::lds_offset(qs.sh->token[1]));
+    cdna4::lds_load16(k + 2 * attn::kDim + 4 * lane, cdna4::lds_offset(qs.sh->token[2]));
+  }
+}
+
+// RMSNorm and NEOX RoPE of a row, lane l holding dimensions 4 l .. 4 l + 3 (rotation partners are
+// 8 lanes apart, lanes 0 .. 15).
+__device__ __attribute__((always_inline)) inline float4 prep_row(float4 x, float4 w, float eps,
+                                                                const float* rope,
+                                                                unsigned lane) {
+  const float ss = cdna4::wave_allsum(
+      __builtin_fmaf(x.w, x.w, __builtin_fmaf(x.z, x.z, __builtin_fmaf(x.y, x.y, x.x * x.x))));
+  const float r = rsqrtf(ss / attn::kDim + eps);
+  float v[4] = {x.x * r * w.x, x.y * r * w.y, x.z * r * w.z, x.w * r * w.w};
+  float partner[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    partner[i] = cdna4::dpp_mov<cdna4::kRowRor8>(v[i]);
+  if (lane < attn::kRopeDim / 4) {
+    const float4 c = *reinterpret_cast<const float4*>(rope + 4 * (lane % 8));
+    const float4 s = *reinterpret_cast<const float4*>(rope + 32 + 4 * (lane % 8));
+    const float cs[4] = {c.x, c.y, c.z, c.w}, sn[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      v[i] = lane < 8 ? v[i] * cs[i] - partner[i] * sn[i] : v[i] * cs[i] + partner[i] * sn[i];
+  }
+  return float4{v[0], v[1], v[2], v[3]};
+}
+
+// The prepared token row of the owner wave: lane l holds dimensions 4 l .. 4 l + 3.
+struct TokenRow {
+  cdna4::half4_t k, v;
+};
+
+// Prepares this wave's query rows in place once its copies of them have landed (and the token's
+// row, for the owner).
+__device__ __attribute__((always_inline)) inline void prepare_queries(const float*, float (*)[256],
+                                                                     unsigned, unsigned, bool,
+                                                                     TokenRow&) {}
+__device__ __attribute__((always_inline)) inline void prepare_queries(const PrepQuery& qs,
+                                                                     float (*q)[256],
+                                                                     unsigned wave, unsigned lane,
+                                                                     bool owner, TokenRow& row) {
+  const float* rope = qs.sh->rope[wave];
+  const float4 w = *reinterpret_cast<const float4*>(&qs.sh->norm[wave][4 * lane]);
+#pragma unroll
+  for (unsigned i = 0; i < 2; ++i) {
+    float4* at = reinterpret_cast<float4*>(&q[2 * wave + i][4 * lane]);
+    *at = prep_row(*at, w, qs.eps, rope, lane);
+  }
+  if (owner) {  // uniform
+    const float4 k = prep_row(*reinterpret_cast<const float4*>(&qs.sh->token[0][4 * lane]),
+                              *reinterpret_cast<const float4*>(&qs.sh->token[1][4 * lane]), qs.eps,
+                              rope, lane);
+    const float4 v = *reinterpret_cast<const float4*>(&qs.sh->token[2][4 * lane]);
+    row.k = cdna4::half4_t{static_cast<_Float16>(k.x), static_cast<_Float16>(k.y),
+                           static_cast<_Float16>(k.z), static_cast<_Float16>(k.w)};
+    row.v = cdna4::half4_t{static_cast<_Float16>(v.x), static_cast<_Float16>(v.y),
+                           static_cast<_Float16>(v.z), static_cast<_Float16>(v.w)};
+  }
+}
+
+// Puts the token's K or V row (4 dimensions per lane) into tile row r of a slot, whose 16-byte
+// chunks are swizzled.
+__device__ __attribute__((always_inline)) inline void put_token(unsigned char* slot, unsigned r,
+                                                               unsigned pos,
+                                                               cdna4::half4_t x, unsigned lane) {
+  *reinterpret_cast<cdna4::half4_t*>(slot + 512 * r + 16 * pos + 8 * (lane & 1u)) = x;
+}
+__device__ __attribute__((always_inline)) inline void store_token(const float*, const TokenRow&,
+                                                                 unsigned) {}
+__device__ __attribute__((always_inline)) inline void store_token(const PrepQuery& qs,
+                                                                 const TokenRow& row,
+                                                                 unsigned lane) {
+  *reinterpret_cast<cdna4::half4_t*>(qs.k_row + 4 * lane) = row.k;
+  *reinterpret_cast<cdna4::half4_t*>(qs.v_row + 4 * lane) = row.v;
+}
+
 // Where the rows of a split lie, for the tile copies: k_at(row) / v_at(row) is the address of K /
 // V row `row`, valid for the 8-row group (aligned to 8) that holds it.
 struct LinearTiles {
@@ -1177,16 +1330,20 @@ __device__ __attribute__((always_inline)) inline void tile_rescale(TileSoftmax& 
 // kCoherent: the partial is stored with agent-coherent accesses (cache policy sc1, what a relaxed
 // agent-scope atomic access compiles to on gfx950), so a workgroup on another XCD can read it
 // after a counter hand-off (attn_decode_fused_kernel); `part_floats` bounds those stores.
-template <class Tiles, bool kCoherent = false>
+template <class Tiles, bool kCoherent = false, class Query = const float*>
 __device__ __attribute__((always_inline)) inline void split_partial_tiles(
-    const float* __restrict__ q, const Tiles& tl, AttnSpan span, unsigned kvh, float* part_m,
+    const Query& q, const Tiles& tl, AttnSpan span, unsigned kvh, float* part_m,
     float* part_l, float* part_o, std::size_t base, TileShared& sh, bool more,
     unsigned part_floats = 0) {
   using cdna4::half8_t;
   const unsigned t = threadIdx.x, lane = t & 63u, g = lane >> 4, c = lane & 15u;
   const unsigned wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const unsigned n_tiles = (span.end - span.begin + kTileKeys - 1) / kTileKeys;
-  const unsigned last_row = span.end - 1;  // unused when n_tiles == 0
+  const unsigned last_row = last_cached_row(q, span);  // unused when n_tiles == 0
+  constexpr bool kPrep = std::is_same_v<Query, PrepQuery>;
+  const TokenPlace place = token_place(q, span);
+  const bool owner = kPrep && place.tile != ~0u && place.row / 8 == wave;
+  TokenRow token{};
   const unsigned k_lds0 = cdna4::lds_offset(sh.k[0]) + 4096 * wave;
   const unsigned v_lds0 = cdna4::lds_offset(sh.v[0]) + 4096 * wave;
 
@@ -1206,12 +1363,7 @@ __device__ __attribute__((always_inline)) inline void split_partial_tiles(
   };
 
   // The KV head's 8 query rows (wave w: rows 2 w, 2 w + 1), then the first three tiles.
-#pragma unroll
-  for (unsigned i = 0; i < 2; ++i) {
-    const unsigned h = 2 * wave + i;
-    cdna4::lds_load16(q + (std::size_t{kvh} * kGroup + h) * attn::kDim + 4 * lane,
-                      cdna4::lds_offset(sh.q[h]));
-  }
+  issue_queries(q, sh.q, kvh, wave, lane, owner);
 #pragma unroll
   for (unsigned ti = 0; ti < kTileStages - 1; ++ti)
     if (ti < n_tiles)
@@ -1246,8 +1398,23 @@ __device__ __attribute__((always_inline)) inline void split_partial_tiles(
   f32x4 s_cur[2] = {f32x4{}, f32x4{}};
   const TileLane tln = tile_lane(lane);
 
+  auto patch = [&](unsigned ti) __attribute__((always_inline)) {  // tile ti's copy has landed
+    if (kPrep && owner && ti == place.tile) {
+      put_token(sh.k[ti % kTileStages], place.row, tile_swz_k(place.row, lane / 2), token.k, lane);
+      put_token(sh.v[ti % kTileStages], place.row, tile_swz_v(place.row, lane / 2), token.v, lane);
+    }
+  };
   if (n_tiles > 0) {
+    if constexpr (kPrep) {
+      switch (n_tiles) {  // everything before the first tiles' 8 copies each has landed
+        case 1: cdna4::wait_vmcnt<8>(); break;
+        case 2: cdna4::wait_vmcnt<16>(); break;
+        default: cdna4::wait_vmcnt<24>(); break;
+      }
+      prepare_queries(q, sh.q, wave, lane, owner, token);
+    }
     wait_tiles_after(n_tiles - 1 < 2 ? n_tiles - 1 : 2);  // tile 0 and the queries landed
+    patch(0);
     tile_barrier();
     // Query pairs: head c % 8, dimensions 8 (4 s + g) .. + 7, x log2(e)/16 (1/sqrt(256) in
     // log2 units), hi half in columns 0-7, lo half in columns 8-15 (pair_half's split).
@@ -1297,6 +1464,7 @@ __device__ __attribute__((always_inline)) inline void split_partial_tiles(
   for (unsigned ti = 0; ti + 1 < n_tiles; ++ti) {
     const unsigned ahead = n_tiles - 2 - ti;  // copies issued after tile ti + 1's
     wait_tiles_after(ahead < 1 ? ahead : 1);
+    patch(ti + 1);
     tile_barrier();
     if (ti + kTileStages - 1 < n_tiles)
       issue(ti + kTileStages - 1);  // into tile ti - 1's stage
@@ -1333,6 +1501,8 @@ __device__ __attribute__((always_inline)) inline void split_partial_tiles(
     softmax_pv(va, sm, moved, ti == 0);
   }
 
+  if (kPrep && owner)
+    store_token(q, token, lane);
   // Relative to the true max; l summed over the lanes g of the column; the (hi, lo) columns of
   // O joined in the lanes c < 8, which store this wave's 64 dimensions of head c.
   const bool empty = n_tiles == 0;
@@ -1713,15 +1883,19 @@ __device__ __attribute__((always_inline)) inline void wave_merge_ml_out(const Wa
 // four results merge at the end through the K slots (wave w's result in its own slot, which no
 // other wave reads before the merge barrier). `more`: the workgroup runs another item
 // afterwards (its LDS is then reused).
-template <class Tiles>
+template <class Tiles, class Query = const float*>
 __device__ __attribute__((always_inline)) inline void split_partial_waves(
-    const float* __restrict__ q, const Tiles& tl, AttnSpan span, unsigned kvh, float* part_m,
+    const Query& q, const Tiles& tl, AttnSpan span, unsigned kvh, float* part_m,
     float* part_l, float* part_o, std::size_t base, TileShared& sh, bool more) {
   using cdna4::half8_t;
   const unsigned t = threadIdx.x, lane = t & 63u;
   const unsigned wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const unsigned n_tiles = (span.end - span.begin + kTileKeys - 1) / kTileKeys;
-  const unsigned last_row = span.end - 1;  // unused when n_tiles == 0
+  const unsigned last_row = last_cached_row(q, span);  // unused when n_tiles == 0
+  constexpr bool kPrep = std::is_same_v<Query, PrepQuery>;
+  const TokenPlace place = token_place(q, span);
+  const bool owner = kPrep && place.tile != ~0u && place.tile % 4 == wave;
+  TokenRow token{};
   const unsigned nw = n_tiles > wave ? (n_tiles - wave + 3) / 4 : 0;  // this wave's tiles
   const unsigned k_lds = cdna4::lds_offset(sh.k[wave]), v_lds = cdna4::lds_offset(sh.v[wave]);
   const WaveCopy cp = wave_copy_offsets(lane);
@@ -1733,18 +1907,19 @@ __device__ __attribute__((always_inline)) inline void split_partial_waves(
   };
 
   // The KV head's 8 query rows (wave w: rows 2 w, 2 w + 1), then the wave's first tile.
-#pragma unroll
-  for (unsigned i = 0; i < 2; ++i) {
-    const unsigned h = 2 * wave + i;
-    cdna4::lds_load16(q + (std::size_t{kvh} * kGroup + h) * attn::kDim + 4 * lane,
-                      cdna4::lds_offset(sh.q[h]));
-  }
+  issue_queries(q, sh.q, kvh, wave, lane, owner);
   if (nw > 0) {
     issue_k(wave);
     issue_v(wave);
+    if constexpr (kPrep) {
+      cdna4::wait_vmcnt<32>();
+      prepare_queries(q, sh.q, wave, lane, owner, token);
+    }
     cdna4::wait_vmcnt<16>();  // the queries and K landed; V may be in flight
   } else {
     cdna4::wait_vmcnt<0>();
+    if constexpr (kPrep)
+      prepare_queries(q, sh.q, wave, lane, owner, token);
   }
   tile_barrier();
   const TileLane tln = tile_lane(lane);
@@ -1758,6 +1933,10 @@ __device__ __attribute__((always_inline)) inline void split_partial_waves(
   for (unsigned j = 0; j < nw; ++j) {
     const unsigned ti = wave + 4 * j;
     const bool next = j + 1 < nw;
+    if (kPrep && owner && ti == place.tile) {  // the tile's K has landed
+      put_token(sh.k[wave], place.row, tile_swz_k(place.row, lane / 2), token.k, lane);
+      asm volatile("" ::: "memory");
+    }
     half8_t ka[2][8];
     read_k(ka, k_lds + op.kl);
     __builtin_amdgcn_sched_barrier(0);  // every K read in flight before the MFMAs
@@ -1769,6 +1948,10 @@ __device__ __attribute__((always_inline)) inline void split_partial_waves(
       cdna4::wait_vmcnt<16>();  // V of tile ti
     } else {
       cdna4::wait_vmcnt<0>();
+    }
+    if (kPrep && owner && ti == place.tile) {  // and its V
+      put_token(sh.v[wave], place.row, tile_swz_v(place.row, lane / 2), token.v, lane);
+      asm volatile("" ::: "memory");
     }
     half8_t va[16];
     read_v_all(va, v_lds, op.vl);
@@ -1784,6 +1967,8 @@ __device__ __attribute__((always_inline)) inline void split_partial_waves(
       cdna4::wait_vmcnt<16>();  // K of the next tile
   }
 
+  if (kPrep && owner)
+    store_token(q, token, lane);
   // The merge through the K slots: wave w's result in its own slot (O in the first 8 KiB, mt and
   // l after it), which only it has used.
   {
@@ -1894,6 +2079,42 @@ __device__ void attn_split_op(const AttnSplitParams& p, unsigned first, unsigned
 template <int kBlock>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(1, 1))) attn_split_kernel(AttnSplitParams p) {
   attn_split_op<kBlock>(p, 0, attn::kKvHeads * p.n_splits);
+}
+
+// The split of a decode step straight from the token's projections (no reference counterpart: the
+// engine launches the prep first): keys [0, pos] of which the cache holds [0, pos), pos >= 1; the
+// partials of attn_prep_kernel + attn_split_kernel over pos + 1 keys, and the token's K and V
+// stored at pos. The preparation runs under the first tiles' latency. Grid (n_splits, 2) x 256,
+// n_splits = s.n_splits, s.len = pos + 1 (s.q is not used).
+struct AttnPrepSplitParams {
+  AttnSplitParams s;
+  const float* proj;  // [16][512] | k [2][256] | v [2][256]
+  const float* q_norm;
+  const float* k_norm;
+  const float* rope;  // cos [32], sin [32] of the position
+  attn::half_t* k_cache;
+  attn::half_t* v_cache;
+  float eps;
+};
+template <int kBlock>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(1, 1)))
+attn_prep_split_kernel(AttnPrepSplitParams p) {
+  using namespace decode_detail;
+  static_assert(kBlock == 256, "four waves per split workgroup");
+  __shared__ TileShared sh;
+  __shared__ __attribute__((aligned(16))) PrepShared ps;
+  const unsigned split = blockIdx.x, kvh = blockIdx.y;
+  const std::size_t head = std::size_t{kvh} * p.s.max_ctx * attn::kDim;
+  const std::size_t row = head + std::size_t{p.s.len - 1} * attn::kDim;
+  const AttnSpan span = attn_split_span(p.s.len, p.s.n_splits, split);
+  const LinearTiles tl{p.s.k_cache + head, p.s.v_cache + head};
+  const std::size_t base = std::size_t{kvh} * p.s.n_splits + split;
+  const PrepQuery q{p.proj, p.q_norm, p.k_norm, p.rope, p.k_cache + row, p.v_cache + row,
+                    &ps,    p.eps,    p.s.len - 1};
+  if (span.end - span.begin > kSplitWavesMinKeys)
+    split_partial_waves(q, tl, span, kvh, p.s.part_m, p.s.part_l, p.s.part_o, base, sh, false);
+  else
+    split_partial_tiles(q, tl, span, kvh, p.s.part_m, p.s.part_l, p.s.part_o, base, sh, false);
 }
 
 // The same split and arithmetic on wave64 VALU (no reference counterpart; same launch shape and

@@ -59,4 +59,53 @@ __global__ void __launch_bounds__(kBlock) qkv_gemv_kernel(Q4kGemvParams q, Q4kGe
     q4k_gemv_op<ActFormat::Fp16, 2048, kBlock, 2>(q, 0, q.n_rows, b - kVGrid - kKGrid, kQGrid);
 }
 
+// The decode step's input in one launch: qkv_gemv_kernel on the residual row itself. Every workgroup
+// forms RMSNorm(h + delta) weight while its weights are in flight (24 KiB of rows from L2 and one
+// barrier more) instead of waiting for a launch that wrote it: 7.0 us against 2.1 + 5.8 us in two
+// launches. h itself is not updated here (every workgroup reads it). The
+// last workgroup tabulates the token's rotation: rope[i], rope[32 + i] = cos, sin of
+// pos inv_freq[i].
+struct QkvNormParams {
+  const float* h;
+  const float* delta;   // or nullptr
+  const float* weight;  // [2048]
+  float eps;
+  const float* inv_freq;  // [32]
+  float* rope;            // [64]
+  unsigned pos;
+};
+
+template <unsigned kQGrid, unsigned kKGrid, unsigned kVGrid>
+__global__ void __launch_bounds__(256) qkv_norm_gemv_kernel(Q4kGemvParams q, Q4kGemvParams k,
+                                                            Q6kGemvParams v, QkvNormParams n) {
+  constexpr unsigned K = 2048;
+  using S4 = q4k_gemv_detail::Q4kSlab<K, 2>;
+  using S6 = q6k_gemv_detail::Q6kSlab<K, 1>;
+  // One LDS for both formats: three workgroups per CU keep the whole launch resident.
+  __shared__ __attribute__((aligned(16)))
+  std::uint8_t slabs[4 * (S4::alloc > S6::alloc ? S4::alloc : S6::alloc)];
+  __shared__ __attribute__((aligned(16))) q4k_gemv_detail::XArea<ActFormat::Fp16, K> x_lds;
+  __shared__ __attribute__((aligned(16))) float rest[2 * K + 4];
+  const unsigned b = blockIdx.x;
+  if (b == kVGrid + kKGrid + kQGrid) {
+    if (threadIdx.x < 32) {
+      float s, c;
+      sincosf(static_cast<float>(n.pos) * n.inv_freq[threadIdx.x], &s, &c);
+      n.rope[threadIdx.x] = c;
+      n.rope[32 + threadIdx.x] = s;
+    }
+    return;
+  }
+  const q4k_gemv_detail::NormX src{n.h, n.delta, n.weight, rest, n.eps};
+  if (b < kVGrid) {
+    q6k_gemv_detail::q6k_gemv_rows<K, 256, 1>(v, src, 0, v.n_rows, b, kVGrid, slabs, x_lds);
+  } else {
+    const bool is_k = b < kVGrid + kKGrid;
+    const Q4kGemvParams p = is_k ? k : q;
+    q4k_gemv_detail::q4k_gemv_rows<ActFormat::Fp16, K, 256, 2>(
+        p, src, 0, p.n_rows, is_k ? b - kVGrid : b - kVGrid - kKGrid, is_k ? kKGrid : kQGrid,
+        slabs, x_lds);
+  }
+}
+
 }  // namespace miso::kernels

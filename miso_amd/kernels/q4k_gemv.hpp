@@ -40,6 +40,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include <type_traits>
+
 #include "cdna4_wave.hpp"
 
 namespace miso::kernels {
@@ -138,21 +140,43 @@ union XArea {
   XStage<A, K> s;
 };
 
-// Requests the K floats of x into xa.f with LDS DMA, instruction i (256 floats) from wave
-// i % (kBlock / 64). Issued before the weights, so the weights' own waits cover it.
-template <ActFormat A, unsigned K, int kBlock>
-__device__ __attribute__((always_inline)) inline void issue_x(const float* x, XArea<A, K>& xa,
+// Where the K activations come from. PlainX: the K floats of x. NormX: RMSNorm(h + delta) weight
+// of a residual row (delta may be null), eps added to the mean square; the rows of delta and weight
+// wait in `rest` (2 K + 4 floats of LDS), and the sum of squares is the one of a 256-thread
+// workgroup with 8 consecutive elements per thread.
+struct PlainX {
+  const float* x;
+};
+struct NormX {
+  const float* x;  // h
+  const float* delta;
+  const float* weight;
+  float* rest;
+  float eps;
+};
+
+// Requests the K floats of the source into xa.f (and src.rest) with LDS DMA, instruction i (256
+// floats) from wave i % (kBlock / 64). Issued before the weights, so the weights' own waits cover it.
+template <ActFormat A, unsigned K, int kBlock, class Src>
+__device__ __attribute__((always_inline)) inline void issue_x(const Src& src, XArea<A, K>& xa,
                                                               unsigned wave, unsigned lane) {
   const unsigned base = cdna4::lds_offset(xa.f);
-  for (unsigned i = wave; i < K / 256; i += kBlock / 64)
-    cdna4::lds_load16(x + 256 * i + 4 * lane, base + 1024 * i);
+  for (unsigned i = wave; i < K / 256; i += kBlock / 64) {
+    cdna4::lds_load16(src.x + 256 * i + 4 * lane, base + 1024 * i);
+    if constexpr (std::is_same_v<Src, NormX>) {
+      const unsigned rest = cdna4::lds_offset(src.rest);
+      if (src.delta != nullptr)  // uniform
+        cdna4::lds_load16(src.delta + 256 * i + 4 * lane, rest + 1024 * i);
+      cdna4::lds_load16(src.weight + 256 * i + 4 * lane, rest + 4 * K + 1024 * i);
+    }
+  }
 }
 
 // Converts xa.f in place with the kBlock threads of the workgroup, once every wave's share has
 // landed (each wave waits for its own DMA before calling). Thread t owns the 8-element slices
 // 8 (t + kBlock s); a quad of threads covers one sub-block.
-template <ActFormat A, unsigned K, int kBlock>
-__device__ inline void convert_x(XArea<A, K>& xa) {
+template <ActFormat A, unsigned K, int kBlock, class Src>
+__device__ inline void convert_x(const Src& src, XArea<A, K>& xa) {
   constexpr unsigned kSlices = (K + 8 * kBlock - 1) / (8 * kBlock);
   static_assert(kSlices <= 4, "at most 32 activations per thread (K <= 32 kBlock)");
   const half2_t one{static_cast<_Float16>(1.0f), static_cast<_Float16>(1.0f)};
@@ -166,7 +190,31 @@ __device__ inline void convert_x(XArea<A, K>& xa) {
       v[sl][1] = *reinterpret_cast<const float4*>(&xa.f[e + 4]);
     }
   }
-  __syncthreads();  // every float is read before the converted form overwrites the area
+  if constexpr (std::is_same_v<Src, NormX>) {
+    static_assert(K == 8 * kBlock && kBlock == 256, "one slice of 8 elements per thread");
+    const unsigned e = 8 * threadIdx.x;
+    float* f = reinterpret_cast<float*>(v[0]);
+    if (src.delta != nullptr)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        f[i] += src.rest[e + i];
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      ss = __builtin_fmaf(f[i], f[i], ss);
+    ss = cdna4::wave_allsum(ss);
+    float* sums = src.rest + 2 * K;
+    if (threadIdx.x % 64 == 0)
+      sums[threadIdx.x / 64] = ss;
+    __syncthreads();  // also: every float of xa is read before the converted form overwrites it
+    const float total = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+    const float r = 1.0f / __builtin_sqrtf(total * (1.0f / K) + src.eps);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      f[i] = f[i] * r * src.rest[K + e + i];
+  } else {
+    __syncthreads();  // every float is read before the converted form overwrites the area
+  }
 #pragma unroll
   for (unsigned sl = 0; sl < kSlices; ++sl) {
     // Whole quads drop out together (K is a multiple of 32), so the quad DPP stays in-quad.
@@ -401,21 +449,21 @@ __host__ __device__ constexpr unsigned q4k_gemv_wave_rows() {
   return q4k_gemv_detail::Geometry<K>::rows * static_cast<unsigned>(kRows);
 }
 
-// Rows [first, first + count) over logical_grid workgroups of kBlock threads (fused callers pass
-// their own block index and grid; K <= 32 kBlock). Each wave takes q4k_gemv_wave_rows<K, kRows>()
-// consecutive rows per step and strides by the number of waves; each next slab is requested as
-// soon as the current one has been read out of LDS.
-template <ActFormat A, unsigned K, int kBlock, int kRows = 1>
-__device__ void q4k_gemv_op(const Q4kGemvParams& p, unsigned first, unsigned count,
-                            unsigned logical_block = blockIdx.x,
-                            unsigned logical_grid = gridDim.x) {
-  using namespace q4k_gemv_detail;
+namespace q4k_gemv_detail {
+
+template <unsigned K, int kRows>
+using Q4kSlab = Slab<Geometry<K>::row_bytes, Geometry<K>::rows, kRows>;
+
+// q4k_gemv_op over activations from src, in the caller's LDS: one slab per wave and the activation
+// area.
+template <ActFormat A, unsigned K, int kBlock, int kRows, class Src>
+__device__ __attribute__((always_inline)) inline void q4k_gemv_rows(
+    const Q4kGemvParams& p, const Src& src, unsigned first, unsigned count, unsigned logical_block,
+    unsigned logical_grid, std::uint8_t* slabs, XArea<A, K>& x_lds) {
   using G = Geometry<K>;
-  using S = Slab<G::row_bytes, G::rows, kRows>;
+  using S = Q4kSlab<K, kRows>;
   static_assert(kBlock % 64 == 0 && kRows >= 1, "whole waves, at least one pass");
   constexpr unsigned kStep = q4k_gemv_wave_rows<K, kRows>();
-  __shared__ __attribute__((aligned(16))) std::uint8_t slab[kBlock / 64][S::alloc];
-  __shared__ __attribute__((aligned(16))) XArea<A, K> x_lds;
   const unsigned lane = threadIdx.x % 64;
   const unsigned wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const unsigned wave = logical_block * (kBlock / 64) + wv;
@@ -423,7 +471,7 @@ __device__ void q4k_gemv_op(const Q4kGemvParams& p, unsigned first, unsigned cou
   const unsigned slot = lane % G::lanes, sub = lane / G::lanes;
   const unsigned j = slot & 3u;  // the lane's group index inside its blocks (lanes % 4 == 0)
   const unsigned end = first + count;
-  const std::uint8_t* mine = slab[wv];
+  const std::uint8_t* mine = slabs + wv * S::alloc;
   const unsigned mine_lds = cdna4::lds_offset(mine);
   auto issue = [&](unsigned r0) __attribute__((always_inline)) {
     const unsigned rows = end - r0 < kStep ? end - r0 : kStep;
@@ -433,7 +481,7 @@ __device__ void q4k_gemv_op(const Q4kGemvParams& p, unsigned first, unsigned cou
 
   // Activations first, then the first slab; the wait for everything but the slab covers the
   // activations, and each pass below waits only for the slab instructions holding its rows.
-  issue_x<A, K, kBlock>(p.x, x_lds, wv, lane);
+  issue_x<A, K, kBlock>(src, x_lds, wv, lane);
   unsigned r0 = first + wave * kStep;
   if (r0 < end) {
     issue(r0);
@@ -441,7 +489,7 @@ __device__ void q4k_gemv_op(const Q4kGemvParams& p, unsigned first, unsigned cou
   } else {
     cdna4::wait_vmcnt<0>();
   }
-  convert_x<A, K, kBlock>(x_lds);
+  convert_x<A, K, kBlock>(src, x_lds);
   GroupX<A> xs[G::per_lane];
 #pragma unroll
   for (unsigned v = 0; v < G::per_lane; ++v)
@@ -472,6 +520,23 @@ __device__ void q4k_gemv_op(const Q4kGemvParams& p, unsigned first, unsigned cou
         p.y[r] = s;
     }
   }
+}
+
+}  // namespace q4k_gemv_detail
+
+// Rows [first, first + count) over logical_grid workgroups of kBlock threads (fused callers pass
+// their own block index and grid; K <= 32 kBlock). Each wave takes q4k_gemv_wave_rows<K, kRows>()
+// consecutive rows per step and strides by the number of waves; each next slab is requested as
+// soon as the current one has been read out of LDS.
+template <ActFormat A, unsigned K, int kBlock, int kRows = 1>
+__device__ void q4k_gemv_op(const Q4kGemvParams& p, unsigned first, unsigned count,
+                            unsigned logical_block = blockIdx.x,
+                            unsigned logical_grid = gridDim.x) {
+  using namespace q4k_gemv_detail;
+  __shared__ __attribute__((aligned(16))) std::uint8_t slabs[kBlock / 64 * Q4kSlab<K, kRows>::alloc];
+  __shared__ __attribute__((aligned(16))) XArea<A, K> x_lds;
+  q4k_gemv_rows<A, K, kBlock, kRows>(p, PlainX{p.x}, first, count, logical_block, logical_grid,
+                                     slabs, x_lds);
 }
 
 template <ActFormat A, unsigned K, int kBlock, int kRows = 1>

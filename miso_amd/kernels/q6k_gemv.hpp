@@ -161,28 +161,28 @@ __host__ __device__ constexpr unsigned q6k_gemv_wave_rows() {
   return q6k_gemv_detail::Geometry<K>::rows * static_cast<unsigned>(kRows);
 }
 
-// Rows [first, first + count) over logical_grid workgroups of kBlock threads (K <= 32 kBlock); each
-// wave takes q6k_gemv_wave_rows<K, kRows>() consecutive rows per step, the same pipeline as
-// q4k_gemv_op.
-template <unsigned K, int kBlock, int kRows = 1>
-__device__ void q6k_gemv_op(const Q6kGemvParams& p, unsigned first, unsigned count,
-                            unsigned logical_block = blockIdx.x,
-                            unsigned logical_grid = gridDim.x) {
-  using namespace q6k_gemv_detail;
-  using q4k_gemv_detail::XArea;
+namespace q6k_gemv_detail {
+
+template <unsigned K, int kRows>
+using Q6kSlab = q4k_gemv_detail::Slab<Geometry<K>::row_bytes, Geometry<K>::rows, kRows>;
+
+// q6k_gemv_op over activations from src, in the caller's LDS (as q4k_gemv_rows).
+template <unsigned K, int kBlock, int kRows, class Src>
+__device__ __attribute__((always_inline)) inline void q6k_gemv_rows(
+    const Q6kGemvParams& p, const Src& src, unsigned first, unsigned count, unsigned logical_block,
+    unsigned logical_grid, std::uint8_t* slabs,
+    q4k_gemv_detail::XArea<ActFormat::Fp16, K>& x_lds) {
   using G = Geometry<K>;
-  using S = q4k_gemv_detail::Slab<G::row_bytes, G::rows, kRows>;
+  using S = Q6kSlab<K, kRows>;
   static_assert(kBlock % 64 == 0 && kRows >= 1, "whole waves, at least one pass");
   constexpr unsigned kStep = q6k_gemv_wave_rows<K, kRows>();
-  __shared__ __attribute__((aligned(16))) std::uint8_t slab[kBlock / 64][S::alloc];
-  __shared__ __attribute__((aligned(16))) XArea<ActFormat::Fp16, K> x_lds;
   const unsigned lane = threadIdx.x % 64;
   const unsigned wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const unsigned wave = logical_block * (kBlock / 64) + wv;
   const unsigned waves = logical_grid * (kBlock / 64);
   const unsigned slot = lane % G::lanes, sub = lane / G::lanes;
   const unsigned end = first + count;
-  const std::uint8_t* mine = slab[wv];
+  const std::uint8_t* mine = slabs + wv * S::alloc;
   const unsigned mine_lds = cdna4::lds_offset(mine);
   auto issue = [&](unsigned r0) __attribute__((always_inline)) {
     const unsigned rows = end - r0 < kStep ? end - r0 : kStep;
@@ -190,7 +190,7 @@ __device__ void q6k_gemv_op(const Q6kGemvParams& p, unsigned first, unsigned cou
                                           rows * static_cast<unsigned>(G::row_bytes), lane);
   };
 
-  q4k_gemv_detail::issue_x<ActFormat::Fp16, K, kBlock>(p.x, x_lds, wv, lane);
+  q4k_gemv_detail::issue_x<ActFormat::Fp16, K, kBlock>(src, x_lds, wv, lane);
   unsigned r0 = first + wave * kStep;
   if (r0 < end) {
     issue(r0);
@@ -198,7 +198,7 @@ __device__ void q6k_gemv_op(const Q6kGemvParams& p, unsigned first, unsigned cou
   } else {
     cdna4::wait_vmcnt<0>();
   }
-  q4k_gemv_detail::convert_x<ActFormat::Fp16, K, kBlock>(x_lds);
+  q4k_gemv_detail::convert_x<ActFormat::Fp16, K, kBlock>(src, x_lds);
   UnitX xs[G::per_lane];
 #pragma unroll
   for (unsigned v = 0; v < G::per_lane; ++v)
@@ -229,6 +229,22 @@ __device__ void q6k_gemv_op(const Q6kGemvParams& p, unsigned first, unsigned cou
         p.y[r] = s;
     }
   }
+}
+
+}  // namespace q6k_gemv_detail
+
+// Rows [first, first + count) over logical_grid workgroups of kBlock threads (K <= 32 kBlock); each
+// wave takes q6k_gemv_wave_rows<K, kRows>() consecutive rows per step, the same pipeline as
+// q4k_gemv_op.
+template <unsigned K, int kBlock, int kRows = 1>
+__device__ void q6k_gemv_op(const Q6kGemvParams& p, unsigned first, unsigned count,
+                            unsigned logical_block = blockIdx.x,
+                            unsigned logical_grid = gridDim.x) {
+  using namespace q6k_gemv_detail;
+  __shared__ __attribute__((aligned(16))) std::uint8_t slabs[kBlock / 64 * Q6kSlab<K, kRows>::alloc];
+  __shared__ __attribute__((aligned(16))) q4k_gemv_detail::XArea<ActFormat::Fp16, K> x_lds;
+  q6k_gemv_rows<K, kBlock, kRows>(p, q4k_gemv_detail::PlainX{p.x}, first, count, logical_block,
+                                  logical_grid, slabs, x_lds);
 }
 
 template <unsigned K, int kBlock, int kRows = 1>

@@ -220,3 +220,65 @@ def test_layer_core_after_each_call(O, attn, torch_mod, layer_case):
     attn.layer_decode(layer, kc, vc, MAX_CTX, 36, rows(h, 36, 37), None, rows(y, 36, 37), EPS, ws)
     torch.cuda.synchronize()
     check(ws.decode_core, 36, 37, 1e-3, "decode")
+
+
+@pytest.mark.parametrize("pos", [1, 7, 31, 32, 33, 1000, 4095, 4096, 5001, 32766, 32767, 32800, 40011])
+def test_layer_decode_lengths(O, attn, torch_mod, layer_case, pos):
+    """The decode step's fused launches (RMSNorm in the projection, prep in the split) where the
+    token's row meets every kind of tile: first and last tile row, its own tile, each copying wave,
+    shared-ring and per-wave splits; against the same step composed of the single operators
+    (attn_prep, attn_decode, the GEMVs), each tested against the oracle by itself, on the normed row
+    that a layer of another format mix leaves in its workspace (one launch per operator; the same
+    row bit for bit). Gates: core differs by the order of the 256-term sums of squares (1e-7) and
+    where one of the new K row's 512 values rounds apart (2^-11 of it in one score of pos + 1): the
+    reference's 1e-5; y also where one of core's 4096 values rounds apart (2^-11 / 64 = 8e-6
+    each): 5e-5. Cache rows as above; h exact; nothing else in the cache touched."""
+    torch = torch_mod
+    layer, deq, norms = layer_case
+    rng = np.random.default_rng(pos)
+    max_ctx = pos + 3
+    h0 = rng.standard_normal(2048).astype(np.float32)
+    delta = (0.5 * rng.standard_normal(2048)).astype(np.float32)
+    gen = torch.Generator(device="cuda").manual_seed(pos)
+    kc = torch.randn(2 * max_ctx * 256, generator=gen, dtype=torch.float16, device="cuda")
+    vc = torch.randn(2 * max_ctx * 256, generator=gen, dtype=torch.float16, device="cuda")
+    k_ref, v_ref = kc.clone(), vc.clone()
+    ws = attn.LayerWorkspace(max_tok=1)
+    wq, wk, wv, wo = (layer._keep[i][0] for i in range(4))
+    attn_norm, q_norm, k_norm, inv_freq = layer._keep[4:]
+    other = attn.Layer(layer._keep[0], layer._keep[1], layer._keep[1], layer._keep[3],
+                       *layer._keep[4:])
+    other_ws = attn.LayerWorkspace(max_tok=1)
+    for d in (delta, None):
+        h = to_dev(torch, h0)
+        y = torch.full((2048,), -1234.5, dtype=torch.float32, device="cuda")
+        attn.layer_decode(layer, kc, vc, max_ctx, pos, h, None if d is None else to_dev(torch, d),
+                          y, EPS, ws)
+        want_h = h0 if d is None else h0 + d
+        assert np.array_equal(to_host(h), want_h)
+        attn.layer_decode(other, k_ref, v_ref, max_ctx, pos, to_dev(torch, h0),
+                          None if d is None else to_dev(torch, d), y.clone(), EPS, other_ws)
+        xn = other_ws.decode[2 * 128 * 8 * 256:][:2048]
+        proj = torch.zeros(9216, device="cuda")
+        attn.qkv_gemv(wq, 8192, proj[:8192], wk, 512, proj[8192:8704], wv, 512, proj[8704:], xn)
+        q = torch.zeros(4096, device="cuda")
+        attn.attn_prep(proj[:8192], proj[8192:8704], proj[8704:], q_norm, k_norm, inv_freq, k_ref,
+                       v_ref, q, pos, max_ctx, EPS)
+        core = torch.zeros(4096, device="cuda")
+        attn.attn_decode(q, proj[:8192], k_ref, v_ref, core, attn.DecodeScratch(128), pos + 1,
+                         max_ctx)
+        y_ref = torch.zeros(2048, device="cuda")
+        attn.q4k_gemv(wo, core, y_ref, 2048, 4096)
+        torch.cuda.synchronize()
+        for got, ref, gate, what in ((ws.decode_core, core, 1e-5, "core"), (y, y_ref, 5e-5, "y")):
+            g, r = to_host(got).astype(np.float64), to_host(ref).astype(np.float64)
+            err = np.sqrt(((g - r) ** 2).sum() / (r ** 2).sum())
+            print(f"[layer decode] pos {pos} {what} rel-L2 {err:.2e}", flush=True)
+            assert np.isfinite(g).all() and err <= gate, what
+        for got, ref in ((kc, k_ref), (vc, v_ref)):
+            g, r = (O.f16_to_f32(to_host(t)).reshape(2, max_ctx, 256) for t in (got, ref))
+            others = np.arange(max_ctx) != pos
+            assert np.array_equal(g[:, others], r[:, others])
+            a, b = g[:, pos].astype(np.float64), r[:, pos].astype(np.float64)
+            ulp = np.spacing(np.abs(b).astype(np.float16)).astype(np.float64)
+            assert (np.abs(a - b) <= ulp + 1e-4 * np.abs(b).max(axis=1, keepdims=True)).all()
