@@ -208,6 +208,18 @@ int miso_attn_decode_ragged(const float* q, const float* gate, const uint16_t* k
                             const uint32_t* lens, uint32_t batch, uint32_t max_len, float* core,
                             float* part_m, float* part_l, float* part_o, void* stream);
 
+/* The same with balanced spans for small batches: part_m and part_l hold `partials` floats and
+ * part_o 256 times as many. With partials >= miso_attn_ragged_balanced_partials(batch, max_len),
+ * batches whose spans miso_attn_ragged_chunk keeps at 512 keys take the span that fills the CUs
+ * evenly for their lengths (128 keys or more; the last 4 floats of part_m carry it to the merge);
+ * otherwise the call is miso_attn_decode_ragged. */
+uint64_t miso_attn_ragged_balanced_partials(uint32_t batch, uint32_t max_len);
+int miso_attn_decode_ragged_ws(const float* q, const float* gate, const uint16_t* k_cache,
+                               const uint16_t* v_cache, const uint64_t* kv_offsets,
+                               const uint32_t* lens, uint32_t batch, uint32_t max_len,
+                               float* core, float* part_m, float* part_l, float* part_o,
+                               uint64_t partials, void* stream);
+
 /* Paged batched decode (no reference counterpart; the reference's KV cache is one contiguous
  * [2][max_ctx][256] f16 buffer per layer, src/engine/attention.hpp:35-41). Same semantics, splits
  * and partial scratch as miso_attn_decode_ragged (and bit-identical outputs on the same keys), with
@@ -225,6 +237,13 @@ int miso_attn_decode_paged(const float* q, const float* gate, const uint16_t* k_
                            uint32_t page_size, const uint32_t* lens, uint32_t batch,
                            uint32_t max_len, float* core, float* part_m, float* part_l,
                            float* part_o, void* stream);
+
+/* miso_attn_decode_paged with balanced spans (miso_attn_decode_ragged_ws). */
+int miso_attn_decode_paged_ws(const float* q, const float* gate, const uint16_t* k_pages,
+                              const uint16_t* v_pages, const int32_t* page_table,
+                              uint32_t max_pages, uint32_t page_size, const uint32_t* lens,
+                              uint32_t batch, uint32_t max_len, float* core, float* part_m,
+                              float* part_l, float* part_o, uint64_t partials, void* stream);
 
 /* fp8 KV cache (no reference counterpart; the reference's cache is f16 [2][max_ctx][256],
  * src/engine/attention.hpp:35-41, kernels/attention_decode.hpp:26-27). Row (KV head, position)

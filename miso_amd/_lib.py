@@ -41,6 +41,11 @@ SIGNATURES = {
     "miso_attn_decode_ragged": (c_int, [P, P, P, P, P, P, c_uint32, c_uint32, P, P, P, P, P]),
     "miso_attn_decode_paged": (c_int, [P, P, P, P, P, c_uint32, c_uint32, P, c_uint32, c_uint32,
                                        P, P, P, P, P]),
+    "miso_attn_ragged_balanced_partials": (c_uint64, [c_uint32, c_uint32]),
+    "miso_attn_decode_ragged_ws": (c_int, [P, P, P, P, P, P, c_uint32, c_uint32, P, P, P, P,
+                                           c_uint64, P]),
+    "miso_attn_decode_paged_ws": (c_int, [P, P, P, P, P, c_uint32, c_uint32, P, c_uint32, c_uint32,
+                                          P, P, P, P, c_uint64, P]),
     "miso_attn_kv_encode_fp8": (c_int, [P, P, P, P, P, P, c_uint32, c_uint32, c_uint32, P]),
     "miso_attn_prep_fp8": (c_int, [P, P, P, P, P, P, P, P, P, P, P, c_uint32, c_uint32, c_float,
                                    P]),

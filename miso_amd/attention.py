@@ -232,8 +232,12 @@ def ragged_chunk(batch: int, max_len: int) -> int:
 
 
 class RaggedScratch:
+    """Split partials of the ragged / paged decode of up to `batch` sequences of max_len keys, with
+    room for balanced spans (miso_attn_decode_ragged_ws)."""
+
     def __init__(self, batch: int, max_len: int, device="cuda"):
-        n = ragged_partials(batch, max_len)
+        n = max(ragged_partials(batch, max_len),
+                int(_lib.load().miso_attn_ragged_balanced_partials(batch, max_len)))
         self.batch, self.max_len = batch, max_len
         self.part_m = torch.empty(n, dtype=torch.float32, device=device)
         self.part_l = torch.empty(n, dtype=torch.float32, device=device)
@@ -254,10 +258,10 @@ def attn_decode_ragged(q, gate, k_cache, v_cache, kv_offsets, lens, core,
     for name, t in (("k_cache", k_cache), ("v_cache", v_cache)):
         if not t.is_cuda or t.dtype not in (torch.float16, torch.int16):
             raise ValueError(f"{name} must be a float16 device tensor")
-    _lib.check(_lib.load().miso_attn_decode_ragged(
+    _lib.check(_lib.load().miso_attn_decode_ragged_ws(
         _ptr(q), _ptr(gate), _ptr(k_cache), _ptr(v_cache), _ptr(kv_offsets), _ptr(lens), batch,
         max_len, _ptr(core), _ptr(scratch.part_m), _ptr(scratch.part_l), _ptr(scratch.part_o),
-        _stream(stream)))
+        scratch.part_m.numel(), _stream(stream)))
 
 
 def attn_decode_paged(q, gate, k_pages, v_pages, page_table, page_size: int, lens, core,
@@ -278,10 +282,11 @@ def attn_decode_paged(q, gate, k_pages, v_pages, page_table, page_size: int, len
     for name, t in (("k_pages", k_pages), ("v_pages", v_pages)):
         if not t.is_cuda or t.dtype not in (torch.float16, torch.int16):
             raise ValueError(f"{name} must be a float16 device tensor")
-    _lib.check(_lib.load().miso_attn_decode_paged(
+    _lib.check(_lib.load().miso_attn_decode_paged_ws(
         _ptr(q), _ptr(gate), _ptr(k_pages), _ptr(v_pages), _ptr(page_table),
         int(page_table.shape[1]), page_size, _ptr(lens), batch, max_len, _ptr(core),
-        _ptr(scratch.part_m), _ptr(scratch.part_l), _ptr(scratch.part_o), _stream(stream)))
+        _ptr(scratch.part_m), _ptr(scratch.part_l), _ptr(scratch.part_o), scratch.part_m.numel(),
+        _stream(stream)))
 
 
 # ------------------------------------------------------------------------------------------------

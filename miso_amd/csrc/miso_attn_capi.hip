@@ -418,40 +418,128 @@ uint64_t miso_attn_ragged_partials(uint32_t batch, uint32_t max_len) {
          (k::attn::kQHeads / k::attn::kKvHeads);
 }
 
-int miso_attn_decode_ragged(const float* q, const float* gate, const uint16_t* k_cache,
-                            const uint16_t* v_cache, const uint64_t* kv_offsets,
-                            const uint32_t* lens, uint32_t batch, uint32_t max_len, float* core,
-                            float* part_m, float* part_l, float* part_o, void* stream) {
+uint64_t miso_attn_ragged_balanced_partials(uint32_t batch, uint32_t max_len) {
+  return uint64_t{batch} * k::attn::kKvHeads * k::attn_ragged_balanced_splits(batch, max_len) *
+             (k::attn::kQHeads / k::attn::kKvHeads) +
+         4;
+}
+
+// The scratch rows per (sequence, KV head) that `partials` floats of part_m hold beside the span
+// word in its last 4 (0: the caller's scratch is miso_attn_ragged_partials', no balanced spans).
+static unsigned balanced_s_max(uint32_t batch, uint32_t max_len, uint64_t partials) {
+  return partials >= miso_attn_ragged_balanced_partials(batch, max_len)
+             ? k::attn_ragged_balanced_splits(batch, max_len)
+             : 0;
+}
+
+static int decode_ragged(const char* fn, const float* q, const float* gate,
+                         const uint16_t* k_cache, const uint16_t* v_cache,
+                         const uint64_t* kv_offsets, const uint32_t* lens, uint32_t batch,
+                         uint32_t max_len, float* core, float* part_m, float* part_l,
+                         float* part_o, uint64_t partials, void* stream) {
   if (any_bad(q, gate, k_cache, v_cache, core, part_o) || bad_scalars(part_m) ||
       bad_scalars(part_l) ||
       kv_offsets == nullptr || lens == nullptr)
-    return fail("miso_attn_decode_ragged", kBadPtr);
+    return fail(fn, kBadPtr);
   if (batch == 0)
-    return fail("miso_attn_decode_ragged", "batch must be >= 1");
+    return fail(fn, "batch must be >= 1");
   if (max_len == 0)
-    return fail("miso_attn_decode_ragged", "max_len must be >= 1");
-  const unsigned s_max = k::attn_ragged_splits(max_len);
+    return fail(fn, "max_len must be >= 1");
   const unsigned cus = device_cus();
-  const k::AttnRaggedParams p{q,     gate,  as_half(k_cache), as_half(v_cache), kv_offsets,
-                              lens,  core,  part_m,           part_l,           part_o,
-                              batch, s_max, 0xFFFFFFFFu, k::attn_ragged_chunk(batch, max_len, cus)};
+  const unsigned fine = balanced_s_max(batch, max_len, partials);
+  const unsigned s_max = fine != 0 ? fine : k::attn_ragged_splits(max_len);
+  k::AttnRaggedParams p{q,     gate,  as_half(k_cache), as_half(v_cache), kv_offsets,
+                        lens,  core,  part_m,           part_l,           part_o,
+                        batch, s_max, 0xFFFFFFFFu, k::attn_ragged_chunk(batch, max_len, cus),
+                        nullptr};
   const uint64_t items = uint64_t{batch} * k::attn::kKvHeads * s_max;
   if (items > 0x7FFFFFFFull)
-    return fail("miso_attn_decode_ragged", "batch x splits too large for one grid");
+    return fail(fn, "batch x splits too large for one grid");
   // One streaming workgroup per CU where the batch fits its item list; else one workgroup per
   // (sequence, KV head, split) slot. Same partials either way.
   const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(cus, items));
-  if (cus > 0 && k::attn_ragged_stream_fits(batch, s_max, grid))
+  if (fine != 0 && cus > 0 && k::attn_ragged_balanced(batch, max_len, cus, grid))
+    p.balanced = reinterpret_cast<unsigned*>(part_m + (partials - 4));
+  if (p.balanced != nullptr || (cus > 0 && k::attn_ragged_stream_fits(batch, s_max, grid)))
     k::attn_ragged_stream_kernel<256><<<grid, 256, 0, as_stream(stream)>>>(p);
   else
     k::attn_ragged_split_kernel<256>
         <<<static_cast<unsigned>(items), 256, 0, as_stream(stream)>>>(p);
-  int rc = launched("miso_attn_decode_ragged(split)");
+  int rc = launched(fn);
   if (rc != 0)
     return rc;
   const unsigned tiles = batch * k::attn::kQHeads * (k::attn::kDim / 64);
   k::attn_ragged_combine_kernel<<<tiles, 64, 0, as_stream(stream)>>>(p);
-  return launched("miso_attn_decode_ragged(combine)");
+  return launched(fn);
+}
+
+int miso_attn_decode_ragged(const float* q, const float* gate, const uint16_t* k_cache,
+                            const uint16_t* v_cache, const uint64_t* kv_offsets,
+                            const uint32_t* lens, uint32_t batch, uint32_t max_len, float* core,
+                            float* part_m, float* part_l, float* part_o, void* stream) {
+  return decode_ragged("miso_attn_decode_ragged", q, gate, k_cache, v_cache, kv_offsets, lens,
+                       batch, max_len, core, part_m, part_l, part_o, 0, stream);
+}
+
+int miso_attn_decode_ragged_ws(const float* q, const float* gate, const uint16_t* k_cache,
+                               const uint16_t* v_cache, const uint64_t* kv_offsets,
+                               const uint32_t* lens, uint32_t batch, uint32_t max_len,
+                               float* core, float* part_m, float* part_l, float* part_o,
+                               uint64_t partials, void* stream) {
+  return decode_ragged("miso_attn_decode_ragged_ws", q, gate, k_cache, v_cache, kv_offsets, lens,
+                       batch, max_len, core, part_m, part_l, part_o, partials, stream);
+}
+
+static int decode_paged(const char* fn, const float* q, const float* gate,
+                        const uint16_t* k_pages, const uint16_t* v_pages,
+                        const int32_t* page_table, uint32_t max_pages, uint32_t page_size,
+                        const uint32_t* lens, uint32_t batch, uint32_t max_len, float* core,
+                        float* part_m, float* part_l, float* part_o, uint64_t partials,
+                        void* stream) {
+  if (any_bad(q, gate, k_pages, v_pages, core, part_o) || bad_scalars(part_m) ||
+      bad_scalars(part_l) || page_table == nullptr || lens == nullptr)
+    return fail(fn, kBadPtr);
+  if (batch == 0)
+    return fail(fn, "batch must be >= 1");
+  if (max_len == 0)
+    return fail(fn, "max_len must be >= 1");
+  if (max_pages == 0)
+    return fail(fn, "max_pages must be >= 1");
+  if (page_size < 8 || page_size > 65536 || (page_size & (page_size - 1)) != 0)
+    return fail(fn, "page_size must be a power of two in [8, 65536]");
+  if (uint64_t{max_pages} * page_size < max_len)
+    return fail(fn, "max_pages * page_size < max_len");
+  const unsigned fine = balanced_s_max(batch, max_len, partials);
+  const unsigned s_max = fine != 0 ? fine : k::attn_ragged_splits(max_len);
+  const uint64_t items = uint64_t{batch} * k::attn::kKvHeads * s_max;
+  if (items > 0x7FFFFFFFull)
+    return fail(fn, "batch x splits too large for one grid");
+  const unsigned cus = device_cus();
+  const unsigned chunk = k::attn_ragged_chunk(batch, max_len, cus);
+  k::AttnPagedParams p{q,      as_half(k_pages), as_half(v_pages), page_table,
+                       lens,   part_m,           part_l,           part_o,
+                       batch,  s_max,            max_pages,
+                       static_cast<unsigned>(__builtin_ctz(page_size)), chunk, nullptr};
+  // As the ragged decode: one streaming workgroup per CU where the batch fits its item list.
+  const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(cus, items));
+  if (fine != 0 && cus > 0 && k::attn_ragged_balanced(batch, max_len, cus, grid))
+    p.balanced = reinterpret_cast<unsigned*>(part_m + (partials - 4));
+  if (p.balanced != nullptr || (cus > 0 && k::attn_ragged_stream_fits(batch, s_max, grid)))
+    k::attn_paged_stream_kernel<256><<<grid, 256, 0, as_stream(stream)>>>(p);
+  else
+    k::attn_paged_split_kernel<256>
+        <<<static_cast<unsigned>(items), 256, 0, as_stream(stream)>>>(p);
+  int rc = launched(fn);
+  if (rc != 0)
+    return rc;
+  // The merge reads only the partials, lens, gate and core of the ragged parameters.
+  const k::AttnRaggedParams r{q,     gate,   nullptr, nullptr, nullptr,
+                              lens,  core,   part_m,  part_l,  part_o,
+                              batch, s_max,  k::attn_paged_len_cap(max_pages, p.log2_page), chunk,
+                              p.balanced};
+  const unsigned tiles = batch * k::attn::kQHeads * (k::attn::kDim / 64);
+  k::attn_ragged_combine_kernel<<<tiles, 64, 0, as_stream(stream)>>>(r);
+  return launched(fn);
 }
 
 int miso_attn_decode_paged(const float* q, const float* gate, const uint16_t* k_pages,
@@ -459,46 +547,18 @@ int miso_attn_decode_paged(const float* q, const float* gate, const uint16_t* k_
                            uint32_t page_size, const uint32_t* lens, uint32_t batch,
                            uint32_t max_len, float* core, float* part_m, float* part_l,
                            float* part_o, void* stream) {
-  if (any_bad(q, gate, k_pages, v_pages, core, part_o) || bad_scalars(part_m) ||
-      bad_scalars(part_l) || page_table == nullptr || lens == nullptr)
-    return fail("miso_attn_decode_paged", kBadPtr);
-  if (batch == 0)
-    return fail("miso_attn_decode_paged", "batch must be >= 1");
-  if (max_len == 0)
-    return fail("miso_attn_decode_paged", "max_len must be >= 1");
-  if (max_pages == 0)
-    return fail("miso_attn_decode_paged", "max_pages must be >= 1");
-  if (page_size < 8 || page_size > 65536 || (page_size & (page_size - 1)) != 0)
-    return fail("miso_attn_decode_paged", "page_size must be a power of two in [8, 65536]");
-  if (uint64_t{max_pages} * page_size < max_len)
-    return fail("miso_attn_decode_paged", "max_pages * page_size < max_len");
-  const unsigned s_max = k::attn_ragged_splits(max_len);
-  const uint64_t items = uint64_t{batch} * k::attn::kKvHeads * s_max;
-  if (items > 0x7FFFFFFFull)
-    return fail("miso_attn_decode_paged", "batch x splits too large for one grid");
-  const unsigned cus = device_cus();
-  const unsigned chunk = k::attn_ragged_chunk(batch, max_len, cus);
-  const k::AttnPagedParams p{q,      as_half(k_pages), as_half(v_pages), page_table,
-                             lens,   part_m,           part_l,           part_o,
-                             batch,  s_max,            max_pages,
-                             static_cast<unsigned>(__builtin_ctz(page_size)), chunk};
-  // As the ragged decode: one streaming workgroup per CU where the batch fits its item list.
-  const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(cus, items));
-  if (cus > 0 && k::attn_ragged_stream_fits(batch, s_max, grid))
-    k::attn_paged_stream_kernel<256><<<grid, 256, 0, as_stream(stream)>>>(p);
-  else
-    k::attn_paged_split_kernel<256>
-        <<<static_cast<unsigned>(items), 256, 0, as_stream(stream)>>>(p);
-  int rc = launched("miso_attn_decode_paged(split)");
-  if (rc != 0)
-    return rc;
-  // The merge reads only the partials, lens, gate and core of the ragged parameters.
-  const k::AttnRaggedParams r{q,     gate,   nullptr, nullptr, nullptr,
-                              lens,  core,   part_m,  part_l,  part_o,
-                              batch, s_max,  k::attn_paged_len_cap(max_pages, p.log2_page), chunk};
-  const unsigned tiles = batch * k::attn::kQHeads * (k::attn::kDim / 64);
-  k::attn_ragged_combine_kernel<<<tiles, 64, 0, as_stream(stream)>>>(r);
-  return launched("miso_attn_decode_paged(combine)");
+  return decode_paged("miso_attn_decode_paged", q, gate, k_pages, v_pages, page_table, max_pages,
+                      page_size, lens, batch, max_len, core, part_m, part_l, part_o, 0, stream);
+}
+
+int miso_attn_decode_paged_ws(const float* q, const float* gate, const uint16_t* k_pages,
+                              const uint16_t* v_pages, const int32_t* page_table,
+                              uint32_t max_pages, uint32_t page_size, const uint32_t* lens,
+                              uint32_t batch, uint32_t max_len, float* core, float* part_m,
+                              float* part_l, float* part_o, uint64_t partials, void* stream) {
+  return decode_paged("miso_attn_decode_paged_ws", q, gate, k_pages, v_pages, page_table,
+                      max_pages, page_size, lens, batch, max_len, core, part_m, part_l, part_o,
+                      partials, stream);
 }
 
 int miso_attn_kv_encode_fp8(const uint16_t* k_cache, const uint16_t* v_cache, uint8_t* k8,

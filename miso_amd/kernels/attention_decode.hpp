@@ -2495,7 +2495,30 @@ struct AttnRaggedParams {
   unsigned len_cap;  // keys a sequence can hold (the paged layout's pages x page size); lens
                      // past it count as len_cap. ~0u for the contiguous ragged layout.
   unsigned chunk;    // keys per split (attn_ragged_chunk), the same in the split and the merge
+  unsigned* balanced;  // device word for balanced spans (attn_ragged_balanced), or nullptr
 };
+
+// Balanced spans: batches whose 512-key spans make less than about four items per CU (where
+// attn_ragged_chunk keeps 512) leave the last round of a streaming launch mostly empty, and short
+// batches most CUs. With scratch for it the streaming kernel picks the span itself from the batch's
+// lengths, which only the device knows (ragged_balanced_tiles), and leaves it in a word for the
+// merge. 13 sequences of 301 .. 9001 keys over 16-row pages: 330 spans of 512 keys on 256 CUs, two
+// rounds, 42.4 us; 256 of 21 tiles, one round, 36.5 us. Scratch rows per (sequence, KV head) for spans
+// of at least kAttnBalancedMinTiles tiles (a tile per wave), about two per CU over the batch.
+constexpr unsigned kAttnBalancedMinTiles = 4;
+__host__ __device__ constexpr unsigned attn_ragged_balanced_splits(unsigned batch,
+                                                                   unsigned max_len) {
+  const unsigned keys = 32 * kAttnBalancedMinTiles;
+  const unsigned fine = max_len / keys + (max_len % keys != 0), share = 1 + 256 / (batch ? batch : 1);
+  const unsigned n = fine < share ? fine : share, least = attn_ragged_splits(max_len);
+  return n > least ? n : least;
+}
+// Whether a streaming launch of `grid` workgroups on `cus` CUs balances its spans.
+__host__ __device__ constexpr bool attn_ragged_balanced(unsigned batch, unsigned max_len,
+                                                        unsigned cus, unsigned grid) {
+  return batch <= 512 && batch <= 2 * grid &&
+         attn_ragged_chunk(batch, max_len, cus) == kAttnRaggedChunk;
+}
 
 // Splits of a sequence of len keys: one per `chunk` keys, at most s_max.
 __host__ __device__ inline unsigned attn_ragged_seq_splits(unsigned len, unsigned s_max,
@@ -2568,7 +2591,53 @@ struct StreamBatch {
   float* part_o;
   const uint32_t* lens;
   unsigned batch, s_max, len_cap, chunk;
+  unsigned* balanced;
 };
+
+// Tiles per span of a balanced launch, by one whole wave: with m spans per workgroup, T tiles in all
+// make about T / R + batch spans of R tiles (half a span wasted per sequence and KV head), and a
+// round costs its tiles and about 3 more (query rows, merge). The m <= 4 with the least m (R + 3),
+// and from that estimate the first R whose spans fit m G. batch <= 2 G, so enough spans fit.
+__device__ __attribute__((always_inline)) inline unsigned ragged_balanced_tiles(
+    const StreamBatch& p, unsigned G, unsigned lane) {
+  constexpr unsigned kPerLane = kRaggedStreamMaxBatch / cdna4::kLanes;
+  unsigned tiles[kPerLane];  // of sequences lane, lane + 64, ...
+  float all = 0.0f;
+#pragma unroll
+  for (unsigned i = 0; i < kPerLane; ++i) {
+    const unsigned s_ = cdna4::kLanes * i + lane;
+    unsigned len = s_ < p.batch ? p.lens[s_] : 0u;
+    len = len < p.len_cap ? len : p.len_cap;
+    tiles[i] = len / kTileKeys + (len % kTileKeys != 0);
+    all += static_cast<float>(tiles[i]);
+  }
+  all = 2.0f * cdna4::wave_allsum(all);
+  const float batch = static_cast<float>(p.batch);
+  unsigned m = 0, R = 0;
+  float least = 0.0f;
+#pragma unroll
+  for (unsigned i = 1; i <= 4; ++i) {
+    const float room = static_cast<float>(i * G) - batch;
+    if (2 * p.batch > i * G)
+      continue;
+    const float est = all / room, cost = static_cast<float>(i) * (est + 3.0f);
+    if (m == 0 || cost < least)
+      m = i, least = cost, R = static_cast<unsigned>(est);
+  }
+  R = R > kAttnBalancedMinTiles ? R : kAttnBalancedMinTiles;
+  for (;; R += R / 32 + 1) {
+    float spans = 0.0f;  // counts below 2^24: exact
+#pragma unroll
+    for (unsigned i = 0; i < kPerLane; ++i) {
+      if (cdna4::kLanes * i >= p.batch)  // uniform
+        break;
+      const unsigned n = (tiles[i] + R - 1) / R;
+      spans += static_cast<float>(n < p.s_max ? n : p.s_max);
+    }
+    if (2.0f * cdna4::wave_allsum(spans) <= static_cast<float>(m * G))
+      return __builtin_amdgcn_readfirstlane(R);
+  }
+}
 
 __device__ __attribute__((always_inline)) inline unsigned lane_value(unsigned v, unsigned j) {
   return static_cast<unsigned>(
@@ -2673,15 +2742,20 @@ __device__ __attribute__((always_inline)) inline void stream_items(const StreamB
 
   // Sequence offsets of the item list (wave 0: 64 sequences per step, an inclusive scan).
   if (wave == 0) {
-    unsigned run = 0;
+    unsigned run = 0, chunk = p.chunk;
     if (lane == 0)
       prefix[0] = 0;
+    if (p.balanced != nullptr) {  // uniform
+      chunk = kTileKeys * ragged_balanced_tiles(p, G, lane);
+      if (w == 0 && lane == 0)
+        *p.balanced = chunk;
+    }
     for (unsigned base = 0; base < p.batch; base += cdna4::kLanes) {
       const unsigned s_ = base + lane;
       unsigned cnt = 0;
       if (s_ < p.batch) {
         const unsigned len = p.lens[s_] < p.len_cap ? p.lens[s_] : p.len_cap;
-        cnt = attn::kKvHeads * attn_ragged_seq_splits(len, p.s_max, p.chunk);
+        cnt = attn::kKvHeads * attn_ragged_seq_splits(len, p.s_max, chunk);
       }
       unsigned incl = cnt;
 #pragma unroll
@@ -2885,7 +2959,7 @@ attn_ragged_stream_kernel(AttnRaggedParams p) {
   decode_detail::RaggedStreamSource src{p.k_cache, p.v_cache, p.kv_offsets};
   decode_detail::stream_items(
       decode_detail::StreamBatch{p.q, p.part_m, p.part_l, p.part_o, p.lens, p.batch, p.s_max,
-                                 p.len_cap, p.chunk},
+                                 p.len_cap, p.chunk, p.balanced},
       src, sh);
 }
 
@@ -2901,7 +2975,8 @@ __global__ void __launch_bounds__(64) attn_ragged_combine_kernel(AttnRaggedParam
     return;
   const std::size_t out = (std::size_t{seq} * attn::kQHeads + h) * attn::kDim + d;
   const unsigned len = p.lens[seq] < p.len_cap ? p.lens[seq] : p.len_cap;
-  const unsigned n_splits = attn_ragged_seq_splits(len, p.s_max, p.chunk);
+  const unsigned chunk = p.balanced != nullptr ? *p.balanced : p.chunk;
+  const unsigned n_splits = attn_ragged_seq_splits(len, p.s_max, chunk);
   if (n_splits == 0) {
     p.core[out] = 0.0f;
     return;
@@ -2934,6 +3009,7 @@ struct AttnPagedParams {
   float* part_o;                 // [batch][2][s_max][8][256]
   unsigned batch, s_max, max_pages, log2_page;
   unsigned chunk;                // keys per split (attn_ragged_chunk)
+  unsigned* balanced;            // as in AttnRaggedParams
 };
 
 // Keys a paged sequence can hold: a longer lens[s] attends to its first max_pages pages only
@@ -2983,7 +3059,8 @@ attn_paged_stream_kernel(AttnPagedParams p) {
                                        p.log2_page};
   decode_detail::stream_items(
       decode_detail::StreamBatch{p.q, p.part_m, p.part_l, p.part_o, p.lens, p.batch, p.s_max,
-                                 attn_paged_len_cap(p.max_pages, p.log2_page), p.chunk},
+                                 attn_paged_len_cap(p.max_pages, p.log2_page), p.chunk,
+                                 p.balanced},
       src, sh);
 }
 

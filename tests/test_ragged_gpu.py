@@ -128,3 +128,32 @@ def test_ragged_chunk_policy(attn, torch_mod):
     assert attn.ragged_chunk(64, 16384) == (1024 if 2 * 64 * 16 >= 4 * cus else 512)
     assert attn.ragged_chunk(1, 65536) == 512
     assert attn.ragged_chunk(9, 2049) == 512
+
+
+@pytest.mark.parametrize("lens,max_len", [([1], 1), ([129, 128], 300), ([4000, 33, 0, 1000], 4096),
+                                          ([9001] + list(range(301, 9000, 725)), 9001),
+                                          ([700] * 64, 1024), ([1500, 20] * 100, 2048),
+                                          ([9000, 31], 512), (list(range(1, 512)), 600)])
+def test_ragged_balanced_spans(O, attn, torch_mod, lens, max_len):
+    """Small batches with scratch for balanced spans (one sequence, empty ones, equal ones, more
+    sequences than fit one round, lengths past max_len) against the oracle, and against the
+    512-key spans of the same call with scratch for those only."""
+    torch = torch_mod
+    lens = np.array(lens, np.uint32)
+    r, got = run(O, attn, torch, lens, len(lens) + max_len, max_len)
+    ref = O.ragged_f64(r["q"], r["gate"], r["k"], r["v"], r["offsets"], lens)
+    live = lens > 0
+    st = O.compare(got[live], ref[live])
+    report(f"balanced spans batch={lens.size} max_len={max_len}", st)
+    assert st["ok"] and st["rel_l2_head"] <= REF_REL_L2, st
+    assert not got[~live].any()
+    sc = attn.RaggedScratch(lens.size, max_len)
+    sc.part_m = sc.part_m[:attn.ragged_partials(lens.size, max_len)]
+    core = torch.full((lens.size * H * D,), -9123.5, device="cuda")
+    attn.attn_decode_ragged(to_dev(torch, r["q"]), to_dev(torch, r["gate"]), to_dev(torch, r["k"]),
+                            to_dev(torch, r["v"]), to_dev(torch, r["offsets"]),
+                            to_dev(torch, r["lens"]), core, sc)
+    torch.cuda.synchronize()
+    fixed = to_host(core).reshape(lens.size, H, D)
+    st = O.compare(fixed[live], ref[live])
+    assert st["ok"] and st["rel_l2_head"] <= REF_REL_L2, st
