@@ -25,8 +25,16 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+# The current device's current stream as an integer: torch.cuda.current_stream() makes a Stream object
+# for it, 2.6 us of the 11.8 a short decode call takes on the host (0.15 us this way).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream(stream) -> Optional[int]:
     if stream is None:
+        if _raw_stream is not None and _device is not None and torch.cuda.is_initialized():
+            return _raw_stream(_device())
         stream = torch.cuda.current_stream()
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
