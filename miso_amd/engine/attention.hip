@@ -100,7 +100,7 @@ void attention_prefill(const AttentionLayer& w, AttentionCache& cache, Attention
   (void)sc;  // the prefill wiring has its own workspace
   auto* kc = reinterpret_cast<kernels::attn::half_t*>(cache.k.data());
   auto* vc = reinterpret_cast<kernels::attn::half_t*>(cache.v.data());
-  const L::PrefillWorkspace ws{ps.xn.data(),   ps.proj.data(), ps.q.data(),
+  const L::PrefillWorkspace ws{ps.proj.data(), ps.q.data(),
                                ps.core.data(), ps.in.xs.data(), ps.in.xh.data(),
                                reinterpret_cast<char*>(ps.balance.data())};
   check("attention_prefill", L::prefill_step(weights(w, rope), kc, vc, cache.len, n,

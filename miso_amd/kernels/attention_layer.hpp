@@ -16,14 +16,14 @@
 //                                                                     n tokens beats n decode
 //                                                                     steps from n = 12
 //
-// Decode step (one token at position len): residual add + RMSNorm of h, the q / k / v projections
-// of the normed row in one launch (qkv_gemv_kernel: Q4_K q and k, Q6_K v, K = 2048; any other
-// format mix falls back to one GEMV per matrix), the per-head norms, RoPE and the K/V append
-// (attn_prep), split-K attention over len + 1 keys with the LSE merge and the gate (attn_split +
-// attn_combine), and the output projection. Prefill step (n tokens at pos0): the same with the
-// prefill GEMMs (qgemm_act + qgemm_wide, q / k / v in one launch) for the projections, attn_prep_batch, and the causal
-// attn_prefill. ingest() applies the engine's policy to a run of n tokens: below the threshold one
-// decode step per token, otherwise prefill chunks of at most the chunk size.
+// Decode step (one token at position len): residual add + RMSNorm of h, the q / k / v projections,
+// the per-head norms, RoPE and the K/V append, split-K attention over len + 1 keys with the LSE
+// merge and the gate, and the output projection: four launches for the model's formats (Q4_K q and
+// k, Q6_K v), one per operator for any other mix. Prefill step (n tokens at pos0): the norm straight
+// into the GEMM input, the prefill GEMMs (qgemm_wide, q / k / v in one launch), the batched prep
+// and the causal attention (attn_prefill_launch). ingest() applies the engine's policy to a run of
+// n tokens: below the threshold one decode step per token, otherwise prefill chunks of at most the
+// chunk size.
 //
 // Every routine returns nullptr on success or a message naming the rejected argument; the C ABI
 // returns it as an error code, an engine front end can throw it.
@@ -79,11 +79,16 @@ struct AddRmsNormParams {
   float* h;            // [tokens][2048], updated in place when delta is set
   const float* delta;  // [tokens][2048] or nullptr
   const float* weight;  // [2048]
-  float* out;           // [tokens][2048]
+  float* out;           // [tokens][2048] (the normed rows), or nullptr:
+  _Float16* xh;         // [tokens][2048] and
+  float* xs;            // [tokens][64], the normed rows as GEMM input (qgemm_act)
   float eps;
 };
 
-template <int = 0>  // a template: header-defined kernels must not clash across translation units
+// One workgroup per token. kGemm: the normed row goes out as the GEMM's f16 input and its group
+// sums, so that it is neither written nor read back in f32: bound by its bytes (4096 tokens, 117 MB
+// in 28 us against 28 + 9 us with the row through memory and qgemm_act).
+template <bool kGemm>
 __global__ void __launch_bounds__(256) add_rmsnorm_kernel(AddRmsNormParams p) {
   __shared__ float wave_ss[4];
   const std::size_t row = std::size_t{blockIdx.x} * kHidden;
@@ -112,9 +117,75 @@ __global__ void __launch_bounds__(256) add_rmsnorm_kernel(AddRmsNormParams p) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const float4 w = *reinterpret_cast<const float4*>(p.weight + e + 4 * i);
-    *reinterpret_cast<float4*>(p.out + row + e + 4 * i) =
-        float4{v[4 * i] * r * w.x, v[4 * i + 1] * r * w.y, v[4 * i + 2] * r * w.z,
-               v[4 * i + 3] * r * w.w};
+    v[4 * i] = v[4 * i] * r * w.x;
+    v[4 * i + 1] = v[4 * i + 1] * r * w.y;
+    v[4 * i + 2] = v[4 * i + 2] * r * w.z;
+    v[4 * i + 3] = v[4 * i + 3] * r * w.w;
+  }
+  if constexpr (kGemm) {
+    _Float16 h[8];
+    const float sum = qgemm_act_group(v, h);
+    *reinterpret_cast<uint4*>(p.xh + row + e) = __builtin_bit_cast(uint4, h);
+    if (threadIdx.x % 4 == 0)
+      p.xs[(row + e) / 32] = sum;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      *reinterpret_cast<float4*>(p.out + row + e + 4 * i) =
+          float4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+  }
+}
+
+// The batched prep of a chunk (attn_prep_batch's results up to the order of the sums of squares):
+// one workgroup per token, a wave per head row (16 bytes per lane), the token's 32 rotations
+// tabulated once. attn_prep_batch_kernel's workgroup per head holds one float per thread and waits
+// at two barriers for it; this is bound by its bytes (4096 tokens, 160 MB).
+template <int = 0>
+__global__ void __launch_bounds__(256) prep_tokens_kernel(AttnPrepBatchParams p) {
+  using namespace attn;
+  __shared__ __attribute__((aligned(16))) float rope[64];
+  const unsigned t = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const std::size_t src = std::size_t{t} * p.proj_stride;
+  const unsigned pos = p.tok0.pos + t;
+  constexpr unsigned kHeads = kQHeads + kKvHeads, kPer = (kHeads + 3) / 4;
+  float4 x[kPer];
+#pragma unroll
+  for (unsigned i = 0; i < kPer; ++i) {
+    const unsigned head = wave + 4 * i < kHeads ? wave + 4 * i : kHeads - 1;
+    const float* row = head < kQHeads ? p.tok0.qg + head * 2 * kDim
+                                      : p.tok0.k + (head - kQHeads) * kDim;
+    x[i] = *reinterpret_cast<const float4*>(row + src + 4 * lane);
+  }
+  const float4 wq = *reinterpret_cast<const float4*>(p.tok0.q_norm + 4 * lane);
+  if (threadIdx.x < 32) {
+    float s, c;
+    sincosf(static_cast<float>(pos) * p.tok0.inv_freq[threadIdx.x], &s, &c);
+    rope[threadIdx.x] = c;
+    rope[32 + threadIdx.x] = s;
+  }
+  __syncthreads();
+#pragma unroll
+  for (unsigned i = 0; i < kPer; ++i) {
+    const unsigned head = wave + 4 * i;
+    if (head >= kHeads)  // uniform
+      break;
+    if (head < kQHeads) {
+      const float4 y = decode_detail::prep_row(x[i], wq, p.tok0.eps, rope, lane);
+      *reinterpret_cast<float4*>(p.tok0.q + (std::size_t{t} * kQHeads + head) * kDim + 4 * lane) =
+          y;
+    } else {
+      const unsigned kvh = head - kQHeads;
+      const float4 wk = *reinterpret_cast<const float4*>(p.tok0.k_norm + 4 * lane);
+      const float4 v = *reinterpret_cast<const float4*>(p.tok0.v + src + kvh * kDim + 4 * lane);
+      const float4 y = decode_detail::prep_row(x[i], wk, p.tok0.eps, rope, lane);
+      const std::size_t at = (std::size_t{kvh} * p.tok0.max_ctx + pos) * kDim + 4 * lane;
+      *reinterpret_cast<cdna4::half4_t*>(p.tok0.k_cache + at) =
+          cdna4::half4_t{static_cast<_Float16>(y.x), static_cast<_Float16>(y.y),
+                         static_cast<_Float16>(y.z), static_cast<_Float16>(y.w)};
+      *reinterpret_cast<cdna4::half4_t*>(p.tok0.v_cache + at) =
+          cdna4::half4_t{static_cast<_Float16>(v.x), static_cast<_Float16>(v.y),
+                         static_cast<_Float16>(v.z), static_cast<_Float16>(v.w)};
+    }
   }
 }
 
@@ -310,7 +381,6 @@ inline DecodeWorkspace decode_workspace(float* ws) {
 // chunk, so the whole prefill workspace is zero-filled once when it is allocated (every chunk
 // leaves the counters zero).
 struct PrefillWorkspace {
-  float* xn;     // [max_tok][2048]
   float* proj;   // [max_tok][9216]
   float* q;      // [max_tok][16][256]
   float* core;   // [max_tok][16][256]
@@ -326,19 +396,18 @@ inline constexpr std::size_t prefill_balance_floats(unsigned max_tok) {
 }
 
 inline constexpr std::size_t prefill_workspace_floats(unsigned max_tok) {
-  return std::size_t{max_tok} * (kHidden + kProj + 2 * kCore + kCore / 32 + kCore / 2) +
+  return std::size_t{max_tok} * (kProj + 2 * kCore + kCore / 32 + kCore / 2) +
          prefill_balance_floats(max_tok);
 }
 
-// Float offset of core in a prefill workspace (after xn, proj and q).
+// Float offset of core in a prefill workspace (after proj and q).
 inline constexpr std::size_t prefill_core_offset(unsigned max_tok) {
-  return std::size_t{max_tok} * (kHidden + kProj + kCore);
+  return std::size_t{max_tok} * (kProj + kCore);
 }
 
 inline PrefillWorkspace prefill_workspace(float* ws, unsigned max_tok) {
   PrefillWorkspace w;
-  w.xn = ws;
-  w.proj = w.xn + std::size_t{max_tok} * kHidden;
+  w.proj = ws;
   w.q = w.proj + std::size_t{max_tok} * kProj;
   w.core = ws + prefill_core_offset(max_tok);
   w.xs = w.core + std::size_t{max_tok} * kCore;
@@ -382,7 +451,8 @@ inline const char* decode_step(const Weights& w, attn::half_t* k_cache, attn::ha
     combine_add_kernel<><<<64 + (delta != nullptr ? 8 : 0), 64, 0, stream>>>(comb, h, delta);
     return gemv(w.o, ws.core, y, stream);
   }
-  add_rmsnorm_kernel<<<1, 256, 0, stream>>>(AddRmsNormParams{h, delta, w.attn_norm, ws.xn, eps});
+  add_rmsnorm_kernel<false><<<1, 256, 0, stream>>>(
+      AddRmsNormParams{h, delta, w.attn_norm, ws.xn, nullptr, nullptr, eps});
   if (const char* err = project_qkv(w, ws.xn, ws.proj, stream))
     return err;
   const AttnPrepParams prep{ws.proj,  ws.proj + 8192, ws.proj + 8704, w.q_norm, w.k_norm,
@@ -407,8 +477,8 @@ inline const char* prefill_step(const Weights& w, attn::half_t* k_cache, attn::h
     return "chunk does not fit the prefill workspace";
   if (std::size_t{pos0} + n > max_ctx)
     return "KV cache is full";
-  add_rmsnorm_kernel<<<n, 256, 0, stream>>>(AddRmsNormParams{h, delta, w.attn_norm, ws.xn, eps});
-  gemm_input(ws.xn, kHidden, n, ws.xh, ws.xs, stream);
+  add_rmsnorm_kernel<true><<<n, 256, 0, stream>>>(
+      AddRmsNormParams{h, delta, w.attn_norm, nullptr, ws.xh, ws.xs, eps});
   if (const char* err = gemm(ws.xh, ws.xs, n, kProj, stream, GemmOut{w.q, ws.proj},
                              GemmOut{w.k, ws.proj + 8192}, GemmOut{w.v, ws.proj + 8704}))
     return err;
@@ -416,7 +486,7 @@ inline const char* prefill_step(const Weights& w, attn::half_t* k_cache, attn::h
                                   w.inv_freq, k_cache, v_cache, ws.q, pos0, max_ctx, eps},
                                  n,
                                  kProj};
-  attn_prep_batch_kernel<256><<<n * 18, 256, 0, stream>>>(prep);
+  prep_tokens_kernel<><<<n, 256, 0, stream>>>(prep);
   const AttnPrefillParams ap{ws.q, ws.proj, k_cache, v_cache, ws.core, pos0, n, max_ctx, kProj};
   attn_prefill_launch(ap, ws.balance, prefill_balance_floats(max_tok) * sizeof(float), stream);
   gemm_input(ws.core, kCore, n, ws.xh, ws.xs, stream);

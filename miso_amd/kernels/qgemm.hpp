@@ -62,46 +62,54 @@ struct QGemmParams {
   unsigned k, n_rows, n_tok, ldy;
 };
 
+// 8 consecutive elements of a thread, the four threads of a quad holding one 32-element group: f16
+// into h, the group's sum of the rounded values returned. The sum is the reference's association
+// (tests/test_qgemm.hip:92-104): the chunk sums ((h0 + h1) + h2) + h3 of the 8 four-element chunks
+// added in order to 0; every lane gathers the quad's chunk sums by DPP broadcast.
+__device__ __attribute__((always_inline)) inline float qgemm_act_group(const float (&x)[8],
+                                                                      _Float16 (&h)[8]) {
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    h[j] = static_cast<_Float16>(x[j]);
+    v[j] = static_cast<float>(h[j]);
+  }
+  const float c0 = ((v[0] + v[1]) + v[2]) + v[3];
+  const float c1 = ((v[4] + v[5]) + v[6]) + v[7];
+  // Chunk sums 2 l and 2 l + 1 come from quad lane l (DPP quad_perm broadcasts of lane l).
+  using cdna4::as_float;
+  using cdna4::as_uint;
+  auto from = [](float y, auto ctrl) {
+    return as_float(__builtin_amdgcn_update_dpp(0u, as_uint(y), decltype(ctrl)::value, 0xF, 0xF,
+                                                true));
+  };
+  using L0 = std::integral_constant<int, 0x00>;
+  using L1 = std::integral_constant<int, 0x55>;
+  using L2 = std::integral_constant<int, 0xAA>;
+  using L3 = std::integral_constant<int, 0xFF>;
+  float sum = 0.0f + from(c0, L0{});
+  sum += from(c1, L0{});
+  sum += from(c0, L1{});
+  sum += from(c1, L1{});
+  sum += from(c0, L2{});
+  sum += from(c1, L2{});
+  sum += from(c0, L3{});
+  sum += from(c1, L3{});
+  return sum;
+}
+
 // Groups [first, first + count) of n_tok k / 32 (group g: elements 32 g .. 32 g + 31 of x, row
 // major), grid-stride: thread i of the launch takes elements 8 (i % 4) .. + 7 of group
-// first + i / 4. A group's sum is the reference's association (tests/test_qgemm.hip:92-104): the
-// chunk sums ((h0 + h1) + h2) + h3 of its 8 four-element chunks added in order to 0, so xs is
-// bit-identical to it; the quad's first lane gathers the other lanes' chunk sums by DPP broadcast.
+// first + i / 4. xs is bit-identical to the reference's (qgemm_act_group).
 __device__ inline void qgemm_act_op(const QGemmActParams& p, unsigned first, unsigned count) {
   const unsigned stride = gridDim.x * blockDim.x;  // a multiple of 4: quads stay whole
   for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i / 4 < count; i += stride) {
     const std::size_t e = (std::size_t{first} + i / 4) * 32 + 8 * (i % 4);
     const float4 a = *reinterpret_cast<const float4*>(p.x + e);
     const float4 b = *reinterpret_cast<const float4*>(p.x + e + 4);
-    const _Float16 h[8] = {static_cast<_Float16>(a.x), static_cast<_Float16>(a.y),
-                           static_cast<_Float16>(a.z), static_cast<_Float16>(a.w),
-                           static_cast<_Float16>(b.x), static_cast<_Float16>(b.y),
-                           static_cast<_Float16>(b.z), static_cast<_Float16>(b.w)};
-    float v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      v[j] = static_cast<float>(h[j]);
-    const float c0 = ((v[0] + v[1]) + v[2]) + v[3];
-    const float c1 = ((v[4] + v[5]) + v[6]) + v[7];
-    // Chunk sums 2 l and 2 l + 1 come from quad lane l (DPP quad_perm broadcasts of lane l).
-    using cdna4::as_float;
-    using cdna4::as_uint;
-    auto from = [](float x, auto ctrl) {
-      return as_float(__builtin_amdgcn_update_dpp(0u, as_uint(x), decltype(ctrl)::value, 0xF, 0xF,
-                                                  true));
-    };
-    using L0 = std::integral_constant<int, 0x00>;
-    using L1 = std::integral_constant<int, 0x55>;
-    using L2 = std::integral_constant<int, 0xAA>;
-    using L3 = std::integral_constant<int, 0xFF>;
-    float sum = 0.0f + from(c0, L0{});
-    sum += from(c1, L0{});
-    sum += from(c0, L1{});
-    sum += from(c1, L1{});
-    sum += from(c0, L2{});
-    sum += from(c1, L2{});
-    sum += from(c0, L3{});
-    sum += from(c1, L3{});
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    _Float16 h[8];
+    const float sum = qgemm_act_group(x, h);
     *reinterpret_cast<uint4*>(p.xh + e) = __builtin_bit_cast(uint4, h);
     if (i % 4 == 0)
       p.xs[first + i / 4] = sum;
