@@ -1507,6 +1507,13 @@ inline bool attn_prefill_in_parts(const AttnPrefillParams& a, void* workspace, s
   return true;
 }
 
+// Largest launch that one workgroup per block runs faster than balanced pairs: with few blocks the
+// halves of the longest one save less than handing a partial over and merging it costs. Measured on
+// one MI355X (one workgroup per block against pairs, us): 16 tokens after 0 9.8 / 10.8, 277 after 0
+// 17.3 / 21.8, 277 after 64 19.1 / 23.6, 512 after 0 24.5 / 26.5, 600 after 0 26.7 / 27.4; 720 after
+// 0 30.8 / 29.8, 720 after 64 32.5 / 31.3, 1024 after 0 39.3 / 34.9.
+constexpr unsigned kAttnPairsMinTokens = 640;
+
 // The causal prefill with a workspace: in parts, in balanced pairs, or one workgroup per block,
 // whichever the launch's size asks for. The workspace holds the balanced form's where
 // attn_prefill_balanced(n) (the caller checks); a larger one also lets the launch run in parts.
@@ -1514,7 +1521,7 @@ inline void attn_prefill_launch(const AttnPrefillParams& a, void* workspace, std
                                 hipStream_t stream) {
   if (attn_prefill_in_parts(a, workspace, bytes, stream))
     return;
-  if (!attn_prefill_balanced(a.n)) {
+  if (!attn_prefill_balanced(a.n) || a.n <= kAttnPairsMinTokens) {
     attn_prefill_kernel<256><<<attn_prefill_items(a.n), 256, 0, stream>>>(a);
     return;
   }

@@ -244,3 +244,19 @@ def test_prefill_parts_small_workspace(O, attn, torch_mod):
     small.nbytes = 0
     assert np.array_equal(run_prefill(attn, torch, wide, scratch=small),
                           run_prefill(attn, torch, wide))
+
+
+@pytest.mark.parametrize("pos0,n", [(0, 16), (0, 277), (64, 640), (0, 640)])
+def test_prefill_short_launch_is_plain(O, attn, torch_mod, prefill_scratch, pos0, n):
+    """Up to 640 tokens a launch that gains nothing in parts runs one workgroup per block, bit for
+    bit; one token more runs balanced pairs (rounded differently), inside the same gate."""
+    def both(n):
+        p = O.prefill_inputs(n, pos0, n, pos0 + n, q_scale=2.0)
+        return (run_prefill(attn, torch_mod, p, scratch=prefill_scratch),
+                run_prefill(attn, torch_mod, p))
+    assert np.array_equal(*both(n))
+    if n == 640:
+        pairs, plain = both(n + 1)
+        assert not np.array_equal(pairs, plain)
+        st = O.compare(pairs, plain.astype(np.float64))
+        assert st["ok"], st
