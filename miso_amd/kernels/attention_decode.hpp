@@ -17,8 +17,6 @@
 #include <cstdint>
 #include <type_traits>
 
-#include <type_traits>
-
 #include "cdna4_wave.hpp"
 
 namespace miso::kernels {
@@ -2594,24 +2592,38 @@ struct StreamBatch {
   unsigned* balanced;
 };
 
-// Tiles per span of a balanced launch, by one whole wave: with m spans per workgroup, T tiles in all
+constexpr unsigned kStreamSeqsPerLane = kRaggedStreamMaxBatch / cdna4::kLanes;
+
+// Tiles per span of a balanced launch, by one whole wave, lane l holding the lengths of sequences l,
+// l + 64, ... (0 past the batch): with m spans per workgroup, T tiles in all
 // make about T / R + batch spans of R tiles (half a span wasted per sequence and KV head), and a
 // round costs its tiles and about 3 more (query rows, merge). The m <= 4 with the least m (R + 3),
 // and from that estimate the first R whose spans fit m G. batch <= 2 G, so enough spans fit.
+// The 512-key spans stay where others would only add partials to merge: they cost no more by that
+// estimate (short sequences of one length), R tiles give a wave as many as 16 do (57 sequences of
+// 782 .. 3217 keys), or they run in one round of at least 10 tiles per CU, when the memory sets the
+// pace whatever the span (6 of 3532 .. 9803 keys). Forming the choice costs such a batch 0.6 us.
 __device__ __attribute__((always_inline)) inline unsigned ragged_balanced_tiles(
-    const StreamBatch& p, unsigned G, unsigned lane) {
-  constexpr unsigned kPerLane = kRaggedStreamMaxBatch / cdna4::kLanes;
-  unsigned tiles[kPerLane];  // of sequences lane, lane + 64, ...
+    const StreamBatch& p, unsigned G, const unsigned (&lens)[kStreamSeqsPerLane]) {
+  unsigned tiles[kStreamSeqsPerLane];
   float all = 0.0f;
 #pragma unroll
-  for (unsigned i = 0; i < kPerLane; ++i) {
-    const unsigned s_ = cdna4::kLanes * i + lane;
-    unsigned len = s_ < p.batch ? p.lens[s_] : 0u;
-    len = len < p.len_cap ? len : p.len_cap;
-    tiles[i] = len / kTileKeys + (len % kTileKeys != 0);
+  for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
+    tiles[i] = lens[i] / kTileKeys + (lens[i] % kTileKeys != 0);
     all += static_cast<float>(tiles[i]);
   }
   all = 2.0f * cdna4::wave_allsum(all);
+  auto spans = [&](unsigned R) __attribute__((always_inline)) {  // counts below 2^24: exact
+    float n = 0.0f;
+#pragma unroll
+    for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
+      if (cdna4::kLanes * i >= p.batch)  // uniform
+        break;
+      const unsigned k = (tiles[i] + R - 1) / R;
+      n += static_cast<float>(k < p.s_max ? k : p.s_max);
+    }
+    return 2.0f * cdna4::wave_allsum(n);
+  };
   const float batch = static_cast<float>(p.batch);
   unsigned m = 0, R = 0;
   float least = 0.0f;
@@ -2624,19 +2636,16 @@ __device__ __attribute__((always_inline)) inline unsigned ragged_balanced_tiles(
     if (m == 0 || cost < least)
       m = i, least = cost, R = static_cast<unsigned>(est);
   }
+  constexpr unsigned kPlain = kAttnRaggedChunk / kTileKeys;
+  const unsigned plain = static_cast<unsigned>(spans(kPlain)), rounds = (plain + G - 1) / G;
+  bool keep = rounds <= kRaggedStreamMaxItems &&  // more: lengths beyond the caller's max_len
+              (static_cast<float>(rounds * (kPlain + 3)) <= least ||
+               (rounds == 1 && all >= 10.0f * static_cast<float>(G)));
   R = R > kAttnBalancedMinTiles ? R : kAttnBalancedMinTiles;
-  for (;; R += R / 32 + 1) {
-    float spans = 0.0f;  // counts below 2^24: exact
-#pragma unroll
-    for (unsigned i = 0; i < kPerLane; ++i) {
-      if (cdna4::kLanes * i >= p.batch)  // uniform
-        break;
-      const unsigned n = (tiles[i] + R - 1) / R;
-      spans += static_cast<float>(n < p.s_max ? n : p.s_max);
-    }
-    if (2.0f * cdna4::wave_allsum(spans) <= static_cast<float>(m * G))
-      return __builtin_amdgcn_readfirstlane(R);
-  }
+  while (!keep && spans(R) > static_cast<float>(m * G))
+    R += R / 32 + 1;
+  keep = keep || (rounds <= m && R > kPlain - kWaves && R <= kPlain);
+  return __builtin_amdgcn_readfirstlane(keep ? kPlain : R);
 }
 
 __device__ __attribute__((always_inline)) inline unsigned lane_value(unsigned v, unsigned j) {
@@ -2742,21 +2751,28 @@ __device__ __attribute__((always_inline)) inline void stream_items(const StreamB
 
   // Sequence offsets of the item list (wave 0: 64 sequences per step, an inclusive scan).
   if (wave == 0) {
-    unsigned run = 0, chunk = p.chunk;
+    unsigned run = 0, chunk = p.chunk, lens[kStreamSeqsPerLane] = {};
+#pragma unroll
+    for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
+      if (cdna4::kLanes * i >= p.batch)  // uniform
+        break;
+      const unsigned s_ = cdna4::kLanes * i + lane;
+      const unsigned len = p.lens[s_ < p.batch ? s_ : p.batch - 1];
+      lens[i] = s_ >= p.batch ? 0u : len < p.len_cap ? len : p.len_cap;
+    }
     if (lane == 0)
       prefix[0] = 0;
     if (p.balanced != nullptr) {  // uniform
-      chunk = kTileKeys * ragged_balanced_tiles(p, G, lane);
+      chunk = kTileKeys * ragged_balanced_tiles(p, G, lens);
       if (w == 0 && lane == 0)
         *p.balanced = chunk;
     }
-    for (unsigned base = 0; base < p.batch; base += cdna4::kLanes) {
-      const unsigned s_ = base + lane;
-      unsigned cnt = 0;
-      if (s_ < p.batch) {
-        const unsigned len = p.lens[s_] < p.len_cap ? p.lens[s_] : p.len_cap;
-        cnt = attn::kKvHeads * attn_ragged_seq_splits(len, p.s_max, chunk);
-      }
+#pragma unroll
+    for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
+      if (cdna4::kLanes * i >= p.batch)  // uniform
+        break;
+      const unsigned s_ = cdna4::kLanes * i + lane;
+      const unsigned cnt = attn::kKvHeads * attn_ragged_seq_splits(lens[i], p.s_max, chunk);
       unsigned incl = cnt;
 #pragma unroll
       for (unsigned d = 1; d < cdna4::kLanes; d *= 2) {

@@ -157,3 +157,33 @@ def test_ragged_balanced_spans(O, attn, torch_mod, lens, max_len):
     fixed = to_host(core).reshape(lens.size, H, D)
     st = O.compare(fixed[live], ref[live])
     assert st["ok"] and st["rel_l2_head"] <= REF_REL_L2, st
+
+
+@pytest.mark.parametrize("lens,kept", [
+    ([512] * 243, True),  # 486 spans in two rounds; halves would take four
+    ([3217, 782] * 28, True),  # 15 tiles a span, four per wave as of 16
+    ([4096] * 24, False),  # two rounds of 512 keys, one of 26 tiles
+    ([8192] * 5, True), ([8192] * 4 + [8160], False),  # one round of 10 tiles per CU, and less
+])
+def test_ragged_balanced_keeps_512_key_spans(O, attn, torch_mod, lens, kept):
+    """On 256 CUs: spans of 512 keys stay where they are estimated no slower, where others would
+    give a wave as many tiles, and in one round of 10 tiles per CU (bitwise the call with scratch
+    for those only); any others are balanced."""
+    torch = torch_mod
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes are those of 256 CUs")
+    lens = np.array(lens, np.uint32)
+    max_len = int(lens.max())
+    r = O.ragged_inputs(lens.size, lens)
+    at = [to_dev(torch, r[x]) for x in ("q", "gate", "k", "v", "offsets", "lens")]
+    out = []
+    for full in (True, False):
+        sc = attn.RaggedScratch(lens.size, max_len)
+        if not full:
+            sc.part_m = sc.part_m[:attn.ragged_partials(lens.size, max_len)]
+        core = torch.full((lens.size * H * D,), -9123.5, device="cuda")
+        attn.attn_decode_ragged(*at, core, sc)
+        out.append(to_host(core).reshape(lens.size, H, D))
+    assert np.array_equal(*out) == kept
+    st = O.compare(out[0], out[1].astype(np.float64))
+    assert st["ok"] and st["rel_l2_head"] <= REF_REL_L2, st
