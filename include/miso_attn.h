@@ -163,7 +163,7 @@ int miso_attn_prefill(const float* q, const float* qg, const uint16_t* k_cache,
  * 16-token block, kernels/attention_prefill.hpp:42-161, so under the causal mask the last block
  * sets the time). Same arguments, contract and output as miso_attn_prefill (within the prefill
  * tolerance, not bitwise: the heavy blocks' keys are summed in two parts; bit-equal from call to
- * call). For n <= 2048 (16-token blocks) and for 3841 <= n <= 4096 (32-token blocks) token
+ * call). For 640 < n <= 2048 (16-token blocks) and for 3841 <= n <= 4096 (32-token blocks) token
  * block B-1-j of the B blocks is paired with block j and the pair's tiles are shared by two
  * workgroups (at most 256, one per CU); the two parts of a split block meet in `workspace`:
  * miso_attn_prefill_workspace_bytes(n) bytes of device memory, 16-byte aligned, zero-filled once
@@ -177,7 +177,10 @@ int miso_attn_prefill(const float* q, const float* qg, const uint16_t* k_cache,
  * balanced form's for n <= 2048; same zero fill), launches of n <= max_n tokens up to 3072 that
  * leave the chip idle otherwise -- few tokens after a prefix -- run in parts: the keys of every
  * token block are split between workgroups and a second kernel joins the parts (two launches,
- * bit-equal from call to call). A smaller workspace keeps the forms above. */
+ * bit-equal from call to call). A smaller workspace keeps the forms above.
+ *
+ * Launches of up to 640 tokens that gain nothing in parts run miso_attn_prefill's layout, which is
+ * the faster one there (the workspace is checked all the same). */
 uint64_t miso_attn_prefill_workspace_bytes(uint32_t n);
 uint64_t miso_attn_prefill_parts_workspace_bytes(uint32_t max_n);
 int miso_attn_prefill_ws(const float* q, const float* qg, const uint16_t* k_cache,

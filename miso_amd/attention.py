@@ -198,7 +198,7 @@ def prefill_workspace_bytes(n: int) -> int:
 
 class PrefillScratch:
     """Workspace of miso_attn_prefill_ws for launches of up to max_n tokens (balanced pairs:
-    n <= 2048 and 3841 <= n <= 4096; parts: up to 3072 tokens after a prefix), its pair counters
+    640 < n <= 2048 and 3841 <= n <= 4096; parts: up to 3072 tokens after a prefix), its pair counters
     (the first 1 KiB) zeroed once; every call leaves it reusable."""
 
     def __init__(self, max_n: int = 4096, device="cuda"):
