@@ -217,10 +217,10 @@ constexpr unsigned kAttnPartsJobTiles = 12;
 // Largest launch in parts, and the row blocks per wave it takes: 0 where the other forms are as
 // fast. Measured on one MI355X (parts against the form it replaces, N(0,1) inputs, us):
 //   - Up to 2048 tokens the balanced pairs fill 2 of every 256 CUs per token block. Parts fill all
-//     of them and cost a merge launch and a job's prologue more: 10 tiles and an eighth of a
-//     pair's run. 203 tokens after 12001: 69 against 346; 37 after 1000: 19 against 39; 512 after
-//     1536: 41 against 68; 1300 after 2000: 91 both; 1024 after 0: 37 against 35 (pairs kept);
-//     2000 after 4000: 202 against 182 (pairs kept).
+//     of them and cost a merge launch and a job's prologue more: 10 tiles, an eighth of a pair's
+//     run and a sixteenth of a worker's. 203 tokens after 12001: 69 against 346; 37 after 1000: 19
+//     against 39; 512 after 1536: 41 against 68; 1300 after 2000: 91 both; 1024 after 0: 37 against
+//     35, 1485 after 1289: 79.9 against 76.1, 2000 after 4000: 202 against 182 (pairs kept).
 //   - 2049 to 3072 tokens leave the last round of one-block workgroups half empty, which a long
 //     prefix makes costly: 2100 after 8000 336 against 506, 3001 after 5003 363 against 388; 3001
 //     after 0 112 against 104 and 3300 after 4000 352 against 343 (one workgroup per block kept).
@@ -237,7 +237,9 @@ inline unsigned attn_prefill_parts_row_blocks(unsigned pos0, unsigned n) {
   for (unsigned b = 0; b < blocks; ++b)
     total += attn_prefill_block_tiles(pos0, n, kAttnQBlock, b);
   const std::uint64_t per_block = total / blocks, per_worker = total / kAttnPartsMaxWorkers;
-  const bool pays = n <= 2048 ? per_block >= per_worker + 10 + per_block / 8 : pos0 >= n;
+  const bool pays = n <= 2048
+                        ? per_block >= per_worker + per_worker / 16 + 10 + per_block / 8
+                        : pos0 >= n;
   return !pays ? 0 : per_worker >= 150 ? 2 : 1;
 }
 
