@@ -2511,10 +2511,11 @@ __host__ __device__ constexpr unsigned attn_ragged_balanced_splits(unsigned batc
   const unsigned n = fine < share ? fine : share, least = attn_ragged_splits(max_len);
   return n > least ? n : least;
 }
-// Whether a streaming launch of `grid` workgroups on `cus` CUs balances its spans.
+// Whether a streaming launch of `grid` workgroups on `cus` CUs balances its spans. Sequences of up to
+// 128 keys are one span each either way (1 of 113: 11.6 us, with a choice 12.5).
 __host__ __device__ constexpr bool attn_ragged_balanced(unsigned batch, unsigned max_len,
                                                         unsigned cus, unsigned grid) {
-  return batch <= 512 && batch <= 2 * grid &&
+  return batch <= 512 && batch <= 2 * grid && max_len > 32 * kAttnBalancedMinTiles &&
          attn_ragged_chunk(batch, max_len, cus) == kAttnRaggedChunk;
 }
 
@@ -2594,63 +2595,139 @@ struct StreamBatch {
 
 constexpr unsigned kStreamSeqsPerLane = kRaggedStreamMaxBatch / cdna4::kLanes;
 
+__device__ __attribute__((always_inline)) inline unsigned lane_value(unsigned v, unsigned j) {
+  return static_cast<unsigned>(
+      __builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(j)));
+}
+
+// Inclusive prefix sum over the wave: within rows of 16 lanes by row shifts, then lane 15 of rows 0
+// and 2 added to the next row and lane 31 to the upper half (row_bcast). Six DPP adds; by
+// ds_bpermute it took a balanced call 0.2 us longer.
+__device__ __attribute__((always_inline)) inline unsigned wave_prefix_sum(unsigned x) {
+  x += __builtin_amdgcn_update_dpp(0u, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0u, x, 0x112, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0u, x, 0x114, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0u, x, 0x118, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0u, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 to rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0u, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 to rows 2, 3
+  return x;
+}
+
+// The item list: where each sequence's items start, for the launch's own spans and, in a balanced
+// launch, for those chosen instead.
+struct StreamLists {
+  unsigned plain[kRaggedStreamMaxBatch + 1], other[kRaggedStreamMaxBatch + 1];
+  unsigned is_other;
+};
+static_assert(sizeof(StreamLists) <= sizeof(StreamShared::merge), "the lists in the merge area");
+
 // Tiles per span of a balanced launch, by one whole wave, lane l holding the lengths of sequences l,
-// l + 64, ... (0 past the batch): with m spans per workgroup, T tiles in all
-// make about T / R + batch spans of R tiles (half a span wasted per sequence and KV head), and a
-// round costs its tiles and about 3 more (query rows, merge). The m <= 4 with the least m (R + 3),
-// and from that estimate the first R whose spans fit m G. batch <= 2 G, so enough spans fit.
-// The 512-key spans stay where others would only add partials to merge: they cost no more by that
-// estimate (short sequences of one length), R tiles give a wave as many as 16 do (57 sequences of
-// 782 .. 3217 keys), or they run in one round of at least 10 tiles per CU, when the memory sets the
-// pace whatever the span (6 of 3532 .. 9803 keys). Forming the choice costs such a batch 0.6 us.
+// l + 64, ... (0 past the batch). With m spans per workgroup, T tiles in all make about T / R +
+// batch spans of R tiles (half a span wasted per sequence and KV head), and a round costs its
+// longest span's tiles and about 3 more (query rows, merge). The m <= 4 with the least m (R + 3), and
+// from that estimate the first R whose spans fit m G. batch <= 2 G, so enough spans fit. The 512-key
+// spans stay where others would only add partials to merge:
+//   - they run in one round of at least 10 tiles per CU, when the memory sets the pace whatever the
+//     span (6 of 3532 .. 9803 keys);
+//   - others give a wave no fewer tiles in no fewer rounds (57 sequences of 782 .. 3217 keys);
+//   - others cost no less at 5 tiles a span beside its own (its partials are merged too), counted
+//     with the tiles the 512-key spans have: the longest's in one round, in more the middle of the
+//     longest's and the mean. 100 sequences of 300 keys, one round of 10 tiles: 25.4 us against 32.9
+//     in two of 5; 238 of 23 .. 447: 51.7 against 54.5.
+// The choice stands before a workgroup's first load and one wave makes it, so its time is its
+// instruction count: quotients of counts by v_rcp_f32 (exact below 2^20: (a + 0.5) / b is at least
+// 0.5 / b from a whole number; one off moves the choice, not the result), and the longest spans only
+// where they can decide.
 __device__ __attribute__((always_inline)) inline unsigned ragged_balanced_tiles(
     const StreamBatch& p, unsigned G, const unsigned (&lens)[kStreamSeqsPerLane]) {
-  unsigned tiles[kStreamSeqsPerLane];
-  float all = 0.0f;
+  constexpr unsigned kPlain = kAttnRaggedChunk / kTileKeys;
+  constexpr float kP = kPlain, kW = kWaves;
+  const float g = static_cast<float>(G), batch = static_cast<float>(p.batch);
+  const float s_max = static_cast<float>(p.s_max);
+  auto ceil_quotient = [](float a, float b) __attribute__((always_inline)) {  // whole numbers
+    return __builtin_floorf((a + (b - 0.5f)) * __builtin_amdgcn_rcpf(b));
+  };
+  float tiles[kStreamSeqsPerLane] = {}, all = 0.0f;
 #pragma unroll
   for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
-    tiles[i] = lens[i] / kTileKeys + (lens[i] % kTileKeys != 0);
-    all += static_cast<float>(tiles[i]);
+    if (cdna4::kLanes * i >= p.batch)  // uniform
+      break;
+    tiles[i] = static_cast<float>(lens[i] / kTileKeys + (lens[i] % kTileKeys != 0));
+    all += tiles[i];
   }
-  all = 2.0f * cdna4::wave_allsum(all);
-  auto spans = [&](unsigned R) __attribute__((always_inline)) {  // counts below 2^24: exact
+  auto spans = [&](float R) __attribute__((always_inline)) {
     float n = 0.0f;
 #pragma unroll
     for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
       if (cdna4::kLanes * i >= p.batch)  // uniform
         break;
-      const unsigned k = (tiles[i] + R - 1) / R;
-      n += static_cast<float>(k < p.s_max ? k : p.s_max);
+      n += fminf(ceil_quotient(tiles[i], R), s_max);
     }
     return 2.0f * cdna4::wave_allsum(n);
   };
-  const float batch = static_cast<float>(p.batch);
-  unsigned m = 0, R = 0;
-  float least = 0.0f;
+  all = 2.0f * cdna4::wave_allsum(all);
+  const float plain = spans(kP), rounds = ceil_quotient(plain, g);
+  // More items than a workgroup's list holds: lengths beyond the caller's max_len.
+  const bool may_stay = rounds <= static_cast<float>(kRaggedStreamMaxItems);
+  if (plain <= g && all >= 10.0f * g)  // uniform, as every branch below
+    return kPlain;
+  float m = 0.0f, least = 0.0f, R = 0.0f;
 #pragma unroll
-  for (unsigned i = 1; i <= 4; ++i) {
-    const float room = static_cast<float>(i * G) - batch;
-    if (2 * p.batch > i * G)
+  for (int i = 1; i <= 4; ++i) {
+    const float mi = static_cast<float>(i);
+    if (2.0f * batch > mi * g)
       continue;
-    const float est = all / room, cost = static_cast<float>(i) * (est + 3.0f);
-    if (m == 0 || cost < least)
-      m = i, least = cost, R = static_cast<unsigned>(est);
+    const float est = all * __builtin_amdgcn_rcpf(mi * g - batch), cost = mi * (est + 3.0f);
+    if (m == 0.0f || cost < least)
+      m = mi, least = cost, R = est;
   }
-  constexpr unsigned kPlain = kAttnRaggedChunk / kTileKeys;
-  const unsigned plain = static_cast<unsigned>(spans(kPlain)), rounds = (plain + G - 1) / G;
-  bool keep = rounds <= kRaggedStreamMaxItems &&  // more: lengths beyond the caller's max_len
-              (static_cast<float>(rounds * (kPlain + 3)) <= least ||
-               (rounds == 1 && all >= 10.0f * static_cast<float>(G)));
-  R = R > kAttnBalancedMinTiles ? R : kAttnBalancedMinTiles;
-  while (!keep && spans(R) > static_cast<float>(m * G))
-    R += R / 32 + 1;
-  keep = keep || (rounds <= m && R > kPlain - kWaves && R <= kPlain);
-  return __builtin_amdgcn_readfirstlane(keep ? kPlain : R);
+  const float mean = all * __builtin_amdgcn_rcpf(fmaxf(plain, 1.0f));
+  // At most 2^29 keys, of which a 32-bit length makes 8.
+  R = fminf(fmaxf(__builtin_floorf(R), static_cast<float>(kAttnBalancedMinTiles)), 0x1p24f);
+  for (; R < 0x1p24f; R += __builtin_floorf(R * 0.03125f) + 1.0f) {
+    if (may_stay && rounds <= m && R > kP - kW && R <= kP)
+      return kPlain;
+    if (may_stay && rounds * (mean + 5.0f) <= m * (R + 8.0f)) {
+      float top = 0.0f, longest = 0.0f;
+#pragma unroll
+      for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
+        if (cdna4::kLanes * i >= p.batch)  // uniform
+          break;
+        const float k = fminf(ceil_quotient(tiles[i], kP), s_max);
+        top = fmaxf(top, ceil_quotient(tiles[i], fmaxf(k, 1.0f)));
+        longest = fmaxf(longest, tiles[i]);
+      }
+      top = cdna4::wave_allmax(top);
+      const float other = fminf(R, cdna4::wave_allmax(longest));
+      const float span = plain <= g ? top : 0.5f * (top + mean);
+      if (rounds * (span + 5.0f) <= m * (other + 5.0f) ||
+          (rounds <= m && ceil_quotient(other, kW) >= ceil_quotient(top, kW)))
+        return kPlain;
+    }
+    if (spans(R) <= m * g)
+      break;
+  }
+  return __builtin_amdgcn_readfirstlane(static_cast<unsigned>(R));
 }
 
-__device__ __attribute__((always_inline)) inline unsigned lane_value(unsigned v, unsigned j) {
-  return static_cast<unsigned>(
-      __builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(j)));
+// Sequence starts for spans of `chunk` keys, by one whole wave (lengths as above).
+__device__ __attribute__((always_inline)) inline void list_items(
+    const StreamBatch& p, const unsigned (&lens)[kStreamSeqsPerLane], unsigned chunk,
+    unsigned* starts, unsigned lane) {
+  unsigned run = 0;
+  if (lane == 0)
+    starts[0] = 0;
+#pragma unroll
+  for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
+    if (cdna4::kLanes * i >= p.batch)  // uniform
+      break;
+    const unsigned s_ = cdna4::kLanes * i + lane;
+    const unsigned incl =
+        wave_prefix_sum(attn::kKvHeads * attn_ragged_seq_splits(lens[i], p.s_max, chunk));
+    if (s_ < p.batch)
+      starts[s_ + 1] = run + incl;
+    run += lane_value(incl, cdna4::kLanes - 1);
+  }
 }
 
 // Where an item's tiles lie. describe() runs in lane j for item j (its sequence, KV head and
@@ -2747,11 +2824,13 @@ __device__ __attribute__((always_inline)) inline void stream_items(const StreamB
   const unsigned t = threadIdx.x, lane = t & 63u;
   const unsigned wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const unsigned G = gridDim.x, w = blockIdx.x;
-  unsigned* prefix = reinterpret_cast<unsigned*>(sh.merge);
+  StreamLists& ls = *reinterpret_cast<StreamLists*>(sh.merge);
 
-  // Sequence offsets of the item list (wave 0: 64 sequences per step, an inclusive scan).
-  if (wave == 0) {
-    unsigned run = 0, chunk = p.chunk, lens[kStreamSeqsPerLane] = {};
+  // Sequence starts of the item list, by wave 0. In a balanced launch wave 1 chooses the span
+  // meanwhile, and if it is another one, lists its items.
+  const bool balanced = p.balanced != nullptr;
+  if (wave == 0 || (balanced && wave == 1)) {
+    unsigned lens[kStreamSeqsPerLane] = {};
 #pragma unroll
     for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
       if (cdna4::kLanes * i >= p.batch)  // uniform
@@ -2760,49 +2839,51 @@ __device__ __attribute__((always_inline)) inline void stream_items(const StreamB
       const unsigned len = p.lens[s_ < p.batch ? s_ : p.batch - 1];
       lens[i] = s_ >= p.batch ? 0u : len < p.len_cap ? len : p.len_cap;
     }
-    if (lane == 0)
-      prefix[0] = 0;
-    if (p.balanced != nullptr) {  // uniform
+    unsigned chunk = p.chunk;
+    if (wave == 1) {
       chunk = kTileKeys * ragged_balanced_tiles(p, G, lens);
+      if (lane == 0)
+        ls.is_other = chunk != p.chunk;
       if (w == 0 && lane == 0)
         *p.balanced = chunk;
     }
-#pragma unroll
-    for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
-      if (cdna4::kLanes * i >= p.batch)  // uniform
-        break;
-      const unsigned s_ = cdna4::kLanes * i + lane;
-      const unsigned cnt = attn::kKvHeads * attn_ragged_seq_splits(lens[i], p.s_max, chunk);
-      unsigned incl = cnt;
-#pragma unroll
-      for (unsigned d = 1; d < cdna4::kLanes; d *= 2) {
-        const unsigned up = __shfl_up(incl, d, cdna4::kLanes);
-        incl += lane >= d ? up : 0u;
-      }
-      if (s_ < p.batch)
-        prefix[s_ + 1] = run + incl;
-      run += __shfl(incl, cdna4::kLanes - 1, cdna4::kLanes);
-    }
+    if (wave == 0 || chunk != p.chunk)
+      list_items(p, lens, chunk, wave == 0 ? ls.plain : ls.other, lane);
   }
   __syncthreads();
+  const unsigned* const prefix = balanced && ls.is_other != 0 ? ls.other : ls.plain;  // uniform
   // Every wave holds the descriptors of the workgroup's items, item j in lane j: key span,
   // partial row group, tile count (0 for an empty span), sequence and KV head (and what Src
   // keeps).
   const unsigned total = prefix[p.batch];
   const unsigned n_items = w < total ? (total - w + G - 1) / G : 0;
   unsigned it_begin = 0, it_end = 0, it_part = 0, it_tiles = 0, it_seq = 0, it_kvh = 0;
+  // Item k lies in the sequence with prefix[s] <= k < prefix[s + 1]: for few items by counting the
+  // sequences that end at or before k (one LDS read; the search below waits for one per step).
+  unsigned lo = 0;
+  if (n_items <= 4) {  // uniform
+    for (unsigned base = 0; base < p.batch; base += cdna4::kLanes) {
+      const unsigned end = base + lane < p.batch ? prefix[base + lane + 1] : ~0u;
+      for (unsigned j = 0; j < n_items; ++j) {
+        const unsigned before = __builtin_popcountll(__builtin_amdgcn_ballot_w64(end <= w + j * G));
+        lo += lane == j ? before : 0u;
+      }
+    }
+  }
   if (lane < n_items) {
     const unsigned k = w + lane * G;
-    unsigned lo = 0, hi = p.batch;  // the sequence s with prefix[s] <= k < prefix[s + 1]
-    while (hi - lo > 1) {
-      const unsigned mid = (lo + hi) / 2;
-      if (prefix[mid] <= k)
-        lo = mid;
-      else
-        hi = mid;
+    if (n_items > 4) {
+      unsigned hi = p.batch;
+      while (hi - lo > 1) {
+        const unsigned mid = (lo + hi) / 2;
+        if (prefix[mid] <= k)
+          lo = mid;
+        else
+          hi = mid;
+      }
     }
     const unsigned r = k - prefix[lo], n = (prefix[lo + 1] - prefix[lo]) / 2;
-    const unsigned kvh = r / n, split = r % n;
+    const unsigned kvh = r >= n ? 1u : 0u, split = r - kvh * n;
     const unsigned len = p.lens[lo] < p.len_cap ? p.lens[lo] : p.len_cap;
     const AttnSpan span = attn_split_span(len, n, split);
     src.describe(lo, kvh, len);

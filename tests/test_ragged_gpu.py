@@ -164,11 +164,13 @@ def test_ragged_balanced_spans(O, attn, torch_mod, lens, max_len):
     ([3217, 782] * 28, True),  # 15 tiles a span, four per wave as of 16
     ([4096] * 24, False),  # two rounds of 512 keys, one of 26 tiles
     ([8192] * 5, True), ([8192] * 4 + [8160], False),  # one round of 10 tiles per CU, and less
+    ([300] * 100, True),  # one round of 10 tiles; two of 5 cost more
+    ([23, 447] * 119, True), ([1240] * 102, False),  # two rounds of 14 at most; two of 20 for three
 ])
 def test_ragged_balanced_keeps_512_key_spans(O, attn, torch_mod, lens, kept):
-    """On 256 CUs: spans of 512 keys stay where they are estimated no slower, where others would
-    give a wave as many tiles, and in one round of 10 tiles per CU (bitwise the call with scratch
-    for those only); any others are balanced."""
+    """On 256 CUs: spans of 512 keys stay where they are estimated no slower (counted with the tiles
+    they really have), where others would give a wave as many tiles, and in one round of 10 tiles
+    per CU (bitwise the call with scratch for those only); any others are balanced."""
     torch = torch_mod
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the sizes are those of 256 CUs")
@@ -187,3 +189,21 @@ def test_ragged_balanced_keeps_512_key_spans(O, attn, torch_mod, lens, kept):
     assert np.array_equal(*out) == kept
     st = O.compare(out[0], out[1].astype(np.float64))
     assert st["ok"] and st["rel_l2_head"] <= REF_REL_L2, st
+
+
+def test_ragged_short_sequences_choose_nothing(O, attn, torch_mod):
+    """Sequences of up to 128 keys are one span either way: the call is the one without room for
+    balanced spans, and the chosen span's word (the last 4 floats of part_m) stays untouched."""
+    torch = torch_mod
+    for max_len, untouched in ((128, True), (129, False)):
+        lens = np.array([max_len, 1, 77], np.uint32)
+        r = O.ragged_inputs(5, lens)
+        sc = attn.RaggedScratch(lens.size, max_len)
+        sc.part_m.fill_(-77.25)
+        core = torch.empty(lens.size * H * D, device="cuda")
+        attn.attn_decode_ragged(*(to_dev(torch, r[x]) for x in ("q", "gate", "k", "v", "offsets",
+                                                                "lens")), core, sc)
+        assert bool((sc.part_m[-4:] == -77.25).all()) == untouched
+        ref = O.ragged_f64(r["q"], r["gate"], r["k"], r["v"], r["offsets"], lens)
+        st = O.compare(to_host(core).reshape(lens.size, H, D), ref)
+        assert st["ok"] and st["rel_l2_head"] <= REF_REL_L2, st
