@@ -896,6 +896,7 @@ struct PrepQuery {
   const float* q_norm;
   const float* k_norm;
   const float* rope;  // [64]
+  float* q_out;         // this KV head's 8 prepared rows, or nullptr
   attn::half_t* k_row;  // this KV head's row pos of the cache
   attn::half_t* v_row;
   PrepShared* sh;
@@ -1002,6 +1003,8 @@ __device__ __attribute__((always_inline)) inline void prepare_queries(const Prep
   for (unsigned i = 0; i < 2; ++i) {
     float4* at = reinterpret_cast<float4*>(&q[2 * wave + i][4 * lane]);
     *at = prep_row(*at, w, qs.eps, rope, lane);
+    if (qs.q_out != nullptr)  // uniform
+      *reinterpret_cast<float4*>(qs.q_out + (2 * wave + i) * attn::kDim + 4 * lane) = *at;
   }
   if (owner) {  // uniform
     const float4 k = prep_row(*reinterpret_cast<const float4*>(&qs.sh->token[0][4 * lane]),
@@ -2081,15 +2084,16 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(1, 
 
 // The split of a decode step straight from the token's projections (no reference counterpart: the
 // engine launches the prep first): keys [0, pos] of which the cache holds [0, pos), pos >= 1; the
-// partials of attn_prep_kernel + attn_split_kernel over pos + 1 keys, and the token's K and V
-// stored at pos. The preparation runs under the first tiles' latency. Grid (n_splits, 2) x 256,
-// n_splits = s.n_splits, s.len = pos + 1 (s.q is not used).
+// partials of attn_prep_kernel + attn_split_kernel over pos + 1 keys, the token's K and V stored at
+// pos and the prepared queries in q. The preparation runs under the first tiles' latency. Grid
+// (n_splits, 2) x 256, n_splits = s.n_splits, s.len = pos + 1 (s.q is not used).
 struct AttnPrepSplitParams {
   AttnSplitParams s;
   const float* proj;  // [16][512] | k [2][256] | v [2][256]
   const float* q_norm;
   const float* k_norm;
   const float* rope;  // cos [32], sin [32] of the position
+  float* q;           // [16][256]
   attn::half_t* k_cache;
   attn::half_t* v_cache;
   float eps;
@@ -2107,8 +2111,9 @@ attn_prep_split_kernel(AttnPrepSplitParams p) {
   const AttnSpan span = attn_split_span(p.s.len, p.s.n_splits, split);
   const LinearTiles tl{p.s.k_cache + head, p.s.v_cache + head};
   const std::size_t base = std::size_t{kvh} * p.s.n_splits + split;
-  const PrepQuery q{p.proj, p.q_norm, p.k_norm, p.rope, p.k_cache + row, p.v_cache + row,
-                    &ps,    p.eps,    p.s.len - 1};
+  const PrepQuery q{p.proj, p.q_norm, p.k_norm, p.rope,
+                    split == 0 ? p.q + std::size_t{kvh} * kGroup * attn::kDim : nullptr,
+                    p.k_cache + row, p.v_cache + row, &ps, p.eps, p.s.len - 1};
   if (span.end - span.begin > kSplitWavesMinKeys)
     split_partial_waves(q, tl, span, kvh, p.s.part_m, p.s.part_l, p.s.part_o, base, sh, false);
   else

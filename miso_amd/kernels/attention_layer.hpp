@@ -282,11 +282,12 @@ inline bool qkv_mix(const Weights& w) {
 
 // qkv_launch on the residual row itself, and the token's rotation table (qkv_norm_gemv_kernel).
 inline void qkv_norm_launch(const Weights& w, const float* h, const float* delta, float eps,
-                            unsigned pos, float* rope, float* proj, hipStream_t stream) {
+                            unsigned pos, float* xn, float* rope, float* proj,
+                            hipStream_t stream) {
   constexpr unsigned kQ = 512, kK = 32, kV = 64;
   const Q4kGemvParams pq{w.q.data, nullptr, proj, w.q.n}, pk{w.k.data, nullptr, proj + 8192, w.k.n};
   const Q6kGemvParams pv{w.v.data, nullptr, proj + 8704, w.v.n};
-  const QkvNormParams pn{h, delta, w.attn_norm, eps, w.inv_freq, rope, pos};
+  const QkvNormParams pn{h, delta, w.attn_norm, xn, eps, w.inv_freq, rope, pos};
   qkv_norm_gemv_kernel<kQ, kK, kV><<<kQ + kK + kV + 1, 256, 0, stream>>>(pq, pk, pv, pn);
 }
 
@@ -442,12 +443,12 @@ inline const char* decode_step(const Weights& w, attn::half_t* k_cache, attn::ha
                               ws.part_o, keys,      max_ctx, n_splits};
   const AttnCombineParams comb{ws.part_m, ws.part_l, ws.part_o, ws.proj, ws.core, n_splits};
   // Four launches where the formats are the model's and the cache holds a key, the rotation table
-  // in ws.q: 21.7 us at 4096 keys against 25.3 us in the six launches below (the small kernels are
+  // in ws.core until the combine writes that: 21.7 us at 4096 keys against 25.3 us in the six launches below (the small kernels are
   // launch- and latency-bound, and the prep hides under the split's first tile).
   if (qkv_mix(w) && len >= 1) {
-    qkv_norm_launch(w, h, delta, eps, len, ws.q, ws.proj, stream);
+    qkv_norm_launch(w, h, delta, eps, len, ws.xn, ws.core, ws.proj, stream);
     attn_prep_split_kernel<256><<<dim3(n_splits, 2), 256, 0, stream>>>(AttnPrepSplitParams{
-        split, ws.proj, w.q_norm, w.k_norm, ws.q, k_cache, v_cache, eps});
+        split, ws.proj, w.q_norm, w.k_norm, ws.core, ws.q, k_cache, v_cache, eps});
     combine_add_kernel<><<<64 + (delta != nullptr ? 8 : 0), 64, 0, stream>>>(comb, h, delta);
     return gemv(w.o, ws.core, y, stream);
   }

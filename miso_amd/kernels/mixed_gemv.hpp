@@ -62,13 +62,14 @@ __global__ void __launch_bounds__(kBlock) qkv_gemv_kernel(Q4kGemvParams q, Q4kGe
 // The decode step's input in one launch: qkv_gemv_kernel on the residual row itself. Every workgroup
 // forms RMSNorm(h + delta) weight while its weights are in flight (24 KiB of rows from L2 and one
 // barrier more) instead of waiting for a launch that wrote it: 7.0 us against 2.1 + 5.8 us in two
-// launches. h itself is not updated here (every workgroup reads it). The
-// last workgroup tabulates the token's rotation: rope[i], rope[32 + i] = cos, sin of
-// pos inv_freq[i].
+// launches. h itself is not updated here (every workgroup reads it); the first workgroup stores the
+// normed row in xn. The last workgroup tabulates the token's rotation: rope[i], rope[32 + i] = cos,
+// sin of pos inv_freq[i].
 struct QkvNormParams {
   const float* h;
   const float* delta;   // or nullptr
   const float* weight;  // [2048]
+  float* xn;            // [2048]
   float eps;
   const float* inv_freq;  // [32]
   float* rope;            // [64]
@@ -96,7 +97,7 @@ __global__ void __launch_bounds__(256) qkv_norm_gemv_kernel(Q4kGemvParams q, Q4k
     }
     return;
   }
-  const q4k_gemv_detail::NormX src{n.h, n.delta, n.weight, rest, n.eps};
+  const q4k_gemv_detail::NormX src{n.h, n.delta, n.weight, rest, b == 0 ? n.xn : nullptr, n.eps};
   if (b < kVGrid) {
     q6k_gemv_detail::q6k_gemv_rows<K, 256, 1>(v, src, 0, v.n_rows, b, kVGrid, slabs, x_lds);
   } else {

@@ -270,7 +270,12 @@ def test_layer_decode_lengths(O, attn, torch_mod, layer_case, pos):
         y_ref = torch.zeros(2048, device="cuda")
         attn.q4k_gemv(wo, core, y_ref, 2048, 4096)
         torch.cuda.synchronize()
-        for got, ref, gate, what in ((ws.decode_core, core, 1e-5, "core"), (y, y_ref, 5e-5, "y")):
+        # the workspace's normed row (bit for bit) and prepared queries, as the six launches leave them
+        at = 2 * 128 * 8 * 256
+        assert torch.equal(ws.decode[at:at + 2048], xn)
+        got_q = ws.decode[at + 2048 + 9216:][:4096]
+        for got, ref, gate, what in ((ws.decode_core, core, 1e-5, "core"), (y, y_ref, 5e-5, "y"),
+                                     (got_q, q, 1e-6, "q")):
             g, r = to_host(got).astype(np.float64), to_host(ref).astype(np.float64)
             err = np.sqrt(((g - r) ** 2).sum() / (r ** 2).sum())
             print(f"[layer decode] pos {pos} {what} rel-L2 {err:.2e}", flush=True)
