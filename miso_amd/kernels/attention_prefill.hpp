@@ -1443,6 +1443,12 @@ __global__ void __launch_bounds__(256) attn_prefill_merge_kernel(AttnPrefillPart
       x[i][0] = *reinterpret_cast<const float4*>(o0 + at * kDim);
       x[i][1] = *reinterpret_cast<const float4*>(o0 + (at + 1) * kDim);
     }
+    // Every row is loaded here, not in the branches below.
+#pragma unroll
+    for (unsigned i = 0; i < kBatch; ++i)
+#pragma unroll
+      for (unsigned h = 0; h < 2; ++h)
+        asm volatile("" : "+v"(x[i][h].x), "+v"(x[i][h].y), "+v"(x[i][h].z), "+v"(x[i][h].w));
 #pragma unroll
     for (unsigned h = 0; h < 2; ++h) {
       float mx = top[h];
@@ -1455,9 +1461,9 @@ __global__ void __launch_bounds__(256) attn_prefill_merge_kernel(AttnPrefillPart
       o[h] = float4{o[h].x * old, o[h].y * old, o[h].z * old, o[h].w * old};
 #pragma unroll
       for (unsigned i = 0; i < kBatch; ++i) {
-        const float e = i0 + i < parts
-                            ? __builtin_amdgcn_exp2f((h == 0 ? ml[i].x : ml[i].z) - mx)
-                            : 0.0f;
+        if (i0 + i >= parts)  // uniform: a repeated row is left out (times 0 an infinity is NaN)
+          break;
+        const float e = __builtin_amdgcn_exp2f((h == 0 ? ml[i].x : ml[i].z) - mx);
         l[h] = __builtin_fmaf(h == 0 ? ml[i].y : ml[i].w, e, l[h]);
         o[h].x = __builtin_fmaf(x[i][h].x, e, o[h].x);
         o[h].y = __builtin_fmaf(x[i][h].y, e, o[h].y);

@@ -260,3 +260,23 @@ def test_prefill_short_launch_is_plain(O, attn, torch_mod, prefill_scratch, pos0
         assert not np.array_equal(pairs, plain)
         st = O.compare(pairs, plain.astype(np.float64))
         assert st["ok"], st
+
+
+def test_prefill_parts_keep_infinities(O, attn, torch_mod, prefill_scratch):
+    """An overflowed V entry of the prefix makes its dimension infinite in every row of its KV head,
+    whatever part it lies in, and nothing else: as in one workgroup per block. 203 tokens after 2000
+    run in 9 .. 10 parts a block, so a batch of the merge ends in rows without weight."""
+    n, pos0 = 203, 2000
+    for key in (3, 700, 1999):
+        p = O.prefill_inputs(n + key, pos0, n, pos0 + n, q_scale=0.5)
+        p["v"][key * D + 77] = 0x7C00  # KV head 0
+        p["v"][(pos0 + n + key) * D + 5] = 0xFC00  # KV head 1
+        parts = run_prefill(attn, torch_mod, p, scratch=prefill_scratch)
+        plain = run_prefill(attn, torch_mod, p)
+        want = np.zeros((n, H, D))
+        want[:, :8, 77], want[:, 8:, 5] = np.inf, -np.inf
+        hit = want != 0
+        assert np.array_equal(plain[hit], want[hit]) and np.isfinite(plain[~hit]).all()
+        assert np.array_equal(parts[hit], want[hit])
+        parts, plain = parts[~hit], plain[~hit]
+        assert (np.abs(parts - plain) <= 2e-3 + 1e-2 * np.abs(plain)).all()
