@@ -262,12 +262,13 @@ def test_prefill_short_launch_is_plain(O, attn, torch_mod, prefill_scratch, pos0
         assert st["ok"], st
 
 
-def test_prefill_parts_keep_infinities(O, attn, torch_mod, prefill_scratch):
+@pytest.mark.parametrize("pos0,n", [(1000, 37), (5000, 100), (12001, 203)])
+def test_prefill_parts_keep_infinities(O, attn, torch_mod, prefill_scratch, pos0, n):
     """An overflowed V entry of the prefix makes its dimension infinite in every row of its KV head,
-    whatever part it lies in, and nothing else: as in one workgroup per block. 203 tokens after 2000
-    run in 9 .. 10 parts a block, so a batch of the merge ends in rows without weight."""
-    n, pos0 = 203, 2000
-    for key in (3, 700, 1999):
+    whatever part it lies in (the first, a middle one, the last), and nothing else: as in one
+    workgroup per block. The blocks run in 4, 18 and 9 parts, so a batch of 8 of the merge ends in
+    rows without weight, which repeat the last part."""
+    for key in (3, pos0 // 2, pos0 - 1):
         p = O.prefill_inputs(n + key, pos0, n, pos0 + n, q_scale=0.5)
         p["v"][key * D + 77] = 0x7C00  # KV head 0
         p["v"][(pos0 + n + key) * D + 5] = 0xFC00  # KV head 1
