@@ -302,6 +302,9 @@ constexpr int kRowBytes = attn::kDim * 2;      // 512: one f16 row
 constexpr int kTileBytes = kKeys * kRowBytes;  // 16 KiB per K or V tile
 constexpr float kLog2e = 1.44269504088896340736f;
 constexpr float kRescaleSlack = 8.0f;  // log2 units: numerators stay <= 2^8 between rescales
+// A row's reference max before its first finite score: with -inf instead, a job whose first tile
+// scores -inf throughout (a part may start anywhere) would form -inf - -inf.
+constexpr float kNoMax = -3.402823466e38f;
 
 // K tiles in the first 48 KiB, V tiles in the next 48 KiB, so every operand address is a per-lane
 // base plus a compile-time offset below 64 KiB (the ring slot is folded into the offset).
@@ -428,7 +431,7 @@ struct TileCopy {
 // 4 c .. 4 c + 3 of the wave's 8, row n = token n / 8, head n % 8; the lane holds row col =
 // lane % 32 of each). q0: block 0's Q^T B operands, dims 16 s + 8 hi + j of the lane's row,
 // x log2(e)/16 (block 1's are in LDS at q1 + 1024 s + 16 lane). m[c]: the reference max in log2
-// units (-inf before the first tile); l[c]: the lane half's share of the running sum.
+// units (kNoMax before the first tile); l[c]: the lane half's share of the running sum.
 struct Rows2 {
   half8_t q0[16];
   unsigned q1;
@@ -481,8 +484,8 @@ __device__ __attribute__((always_inline)) inline void scale_acc(float16_t (&o)[8
 // Softmax decision for one block of one tile. `acc`: the block's S^T accumulator (raw scores in
 // log2 units; element r = key k0 + 8 (r / 4) + 4 hi + r % 4, the lane's row). Keys past `lim` are
 // masked when kMasked. The reference max m moves only when the tile's row max exceeds it by more
-// than the slack (2^8), decided wave-wide so the rescale branch is uniform; on the first tile (m =
-// -inf) it always moves. Writes the f16 numerators 2^(s - m) as the block's two P^T operands,
+// than the slack (2^8), decided wave-wide so the rescale branch is uniform; on the first tile with a
+// finite score (m = kNoMax before it) it always moves. Writes the f16 numerators 2^(s - m) as the block's two P^T operands,
 // updates l = l corr + their sum (the sum of the rounded values the MFMAs use), and returns
 // corr = 2^(m_old - m_new), the factor the block's O must be scaled by (1 if m stayed; `moved`
 // says whether any lane's m moved).
@@ -510,7 +513,7 @@ __device__ __attribute__((always_inline)) inline float decide_block(const float1
   float corr = 1.0f;
   if (moved) {
     const float mn = fmaxf(m, mx);
-    corr = __builtin_amdgcn_exp2f(m - mn);  // 0 on the first tile (m = -inf)
+    corr = __builtin_amdgcn_exp2f(m - mn);  // 0 on the first tile (m = kNoMax)
     m = mn;
   }
   const cdna4::half2_t ones{static_cast<_Float16>(1.0f), static_cast<_Float16>(1.0f)};
@@ -725,7 +728,7 @@ __device__ __attribute__((always_inline)) inline void tile_step2(
     moved[c] = __builtin_amdgcn_ballot_w64(mx > rw.m[c] + kRescaleSlack) != 0;
     if (moved[c]) {
       const float mn = fmaxf(rw.m[c], mx);
-      corr[c] = __builtin_amdgcn_exp2f(rw.m[c] - mn);  // 0 on the first tile (m = -inf)
+      corr[c] = __builtin_amdgcn_exp2f(rw.m[c] - mn);  // 0 on the first tile (m = kNoMax)
       rw.m[c] = mn;
     }
     asm volatile("" : "+v"(rw.m[c]));
@@ -1053,7 +1056,7 @@ __device__ __attribute__((always_inline)) inline void prefill_items(
         for (int st = 0; st < 16; ++st)
           rw.q0[st] = *reinterpret_cast<const __attribute__((address_space(3))) half8_t*>(
               qa + 512 * col + 16 * ((2 * st + hi) ^ (col & 15)));
-        rw.m[0] = -__builtin_inff();
+        rw.m[0] = kNoMax;
         rw.l[0] = 0.0f;
       } else {
 #pragma unroll
@@ -1076,7 +1079,7 @@ __device__ __attribute__((always_inline)) inline void prefill_items(
               *reinterpret_cast<__attribute__((address_space(3))) half8_t*>(rw.q1 + 1024u * st) =
                   v;
           }
-          rw.m[c] = -__builtin_inff();
+          rw.m[c] = kNoMax;
           rw.l[c] = 0.0f;
         }
       }

@@ -281,3 +281,20 @@ def test_prefill_parts_keep_infinities(O, attn, torch_mod, prefill_scratch, pos0
         assert np.array_equal(parts[hit], want[hit])
         parts, plain = parts[~hit], plain[~hit]
         assert (np.abs(parts - plain) <= 2e-3 + 1e-2 * np.abs(plain)).all()
+
+
+@pytest.mark.parametrize("pos0,n", [(2000, 203), (33000, 40), (0, 900)])
+def test_prefill_hidden_keys(O, attn, torch_mod, prefill_scratch, pos0, n):
+    """Keys whose every score is -inf (an overflowed K entry against queries of one sign) weigh
+    nothing, wherever parts and split blocks begin: most of the prefix, or of the chunk, hidden."""
+    p = O.prefill_inputs(n, pos0, n, pos0 + n, q_scale=1.0)
+    p["q"].reshape(n, H, D)[:, :, 9] = np.abs(p["q"].reshape(n, H, D)[:, :, 9]) + 0.25
+    end = pos0 - 70 if pos0 else 700
+    p["k"].reshape(2, pos0 + n, D)[:, 40:end, 9] = 0xFC00
+    rows = np.unique(np.concatenate([np.arange(min(n, 35)), np.arange(0, n, 29), [n - 1]]))
+    ref = O.prefill_f64(p["q"], p["qg"], p["qg_stride"], p["k"], p["v"], pos0, pos0 + n, rows)
+    assert np.isfinite(ref).all()
+    for scratch in (None, prefill_scratch):
+        st = O.compare(run_prefill(attn, torch_mod, p, scratch=scratch)[rows], ref)
+        report(f"hidden keys pos0={pos0} n={n}", st)
+        assert st["ok"], st
