@@ -102,7 +102,7 @@ void attention_prefill(const AttentionLayer& w, AttentionCache& cache, Attention
   auto* vc = reinterpret_cast<kernels::attn::half_t*>(cache.v.data());
   const L::PrefillWorkspace ws{ps.proj.data(), ps.q.data(),
                                ps.core.data(), ps.in.xs.data(), ps.in.xh.data(),
-                               reinterpret_cast<char*>(ps.balance.data())};
+                               reinterpret_cast<char*>(ps.balance.data()), ps.xn.data()};
   check("attention_prefill", L::prefill_step(weights(w, rope), kc, vc, cache.len, n,
                                              cache.max_ctx, h, delta, y, eps, ws, ps.max_tok,
                                              stream));

@@ -60,8 +60,9 @@ struct AttentionScratch {
   float* v() { return proj.data() + 8704; }
 };
 
-// Prefill workspace for chunks of up to max_tok tokens, with the engine's members (`core` holds
-// the last chunk's [n][16][256] attention output) plus `balance`: the balanced prefill's
+// Prefill workspace for chunks of up to max_tok tokens, with the engine's members, as the last
+// chunk left them (the normed rows, the projections, the prepared q, the [n][16][256] attention
+// output `core`), plus `balance`: the balanced prefill's
 // partials and pair counters for chunks of up to min(max_tok, 4096) tokens, zero-filled once here
 // (every chunk leaves the counters zero).
 struct AttentionPrefillScratch {

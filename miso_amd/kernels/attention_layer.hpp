@@ -79,15 +79,15 @@ struct AddRmsNormParams {
   float* h;            // [tokens][2048], updated in place when delta is set
   const float* delta;  // [tokens][2048] or nullptr
   const float* weight;  // [2048]
-  float* out;           // [tokens][2048] (the normed rows), or nullptr:
-  _Float16* xh;         // [tokens][2048] and
+  float* out;           // [tokens][2048], the normed rows (kGemm: may be nullptr)
+  _Float16* xh;         // kGemm: [tokens][2048] and
   float* xs;            // [tokens][64], the normed rows as GEMM input (qgemm_act)
   float eps;
 };
 
 // One workgroup per token. kGemm: the normed row goes out as the GEMM's f16 input and its group
-// sums, so that it is neither written nor read back in f32: bound by its bytes (4096 tokens, 117 MB
-// in 28 us against 28 + 9 us with the row through memory and qgemm_act).
+// sums, so that it is not read back in f32, nor written unless the caller wants it: bound by its
+// bytes (4096 tokens, 117 MB in 28 us against 28 + 9 us with the row through memory and qgemm_act).
 template <bool kGemm>
 __global__ void __launch_bounds__(256) add_rmsnorm_kernel(AddRmsNormParams p) {
   __shared__ float wave_ss[4];
@@ -128,12 +128,12 @@ __global__ void __launch_bounds__(256) add_rmsnorm_kernel(AddRmsNormParams p) {
     *reinterpret_cast<uint4*>(p.xh + row + e) = __builtin_bit_cast(uint4, h);
     if (threadIdx.x % 4 == 0)
       p.xs[(row + e) / 32] = sum;
-  } else {
+  }
+  if (!kGemm || p.out != nullptr)  // uniform
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       *reinterpret_cast<float4*>(p.out + row + e + 4 * i) =
           float4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
-  }
 }
 
 // The batched prep of a chunk (attn_prep_batch's results up to the order of the sums of squares):
@@ -388,6 +388,7 @@ struct PrefillWorkspace {
   float* xs;     // [max_tok][4096 / 32] GEMM input sums
   _Float16* xh;  // [max_tok][4096] GEMM input values
   char* balance;  // prefill_balance_floats(max_tok) floats
+  float* xn = nullptr;  // [max_tok][2048] for the normed rows, where the caller keeps them
 };
 
 inline constexpr std::size_t prefill_balance_floats(unsigned max_tok) {
@@ -479,7 +480,7 @@ inline const char* prefill_step(const Weights& w, attn::half_t* k_cache, attn::h
   if (std::size_t{pos0} + n > max_ctx)
     return "KV cache is full";
   add_rmsnorm_kernel<true><<<n, 256, 0, stream>>>(
-      AddRmsNormParams{h, delta, w.attn_norm, nullptr, ws.xh, ws.xs, eps});
+      AddRmsNormParams{h, delta, w.attn_norm, ws.xn, ws.xh, ws.xs, eps});
   if (const char* err = gemm(ws.xh, ws.xs, n, kProj, stream, GemmOut{w.q, ws.proj},
                              GemmOut{w.k, ws.proj + 8192}, GemmOut{w.v, ws.proj + 8704}))
     return err;

@@ -505,6 +505,29 @@ def rel_l2_rows(got: np.ndarray, ref: np.ndarray) -> float:
 _ref = None
 
 
+_drop_in = None
+
+
+def drop_in():
+    """ctypes handle of oracle/_build/libdrop_in.so (drop_in_capi.hip)."""
+    global _drop_in
+    if _drop_in is None:
+        L = ctypes.CDLL(str(HERE / "_build" / "libdrop_in.so"))
+        V, U = c_void_p, c_uint32
+        sig = {
+            "drop_engine_new": (V, [V, V, V, V, V, V, U, U]),
+            "drop_engine_delete": (None, [V]),
+            "drop_engine_step": (c_int, [V, c_int, V, V, V, U, c_float]),
+            "drop_engine_read": (c_uint64, [V, ctypes.c_char_p, V, c_uint64]),
+        }
+        for name, (res, args) in sig.items():
+            fn = getattr(L, name)
+            fn.restype = res
+            fn.argtypes = args
+        _drop_in = L
+    return _drop_in
+
+
 def ref_kernels():
     """ctypes handle of oracle/_ref/libmiso_ref_kernels.so, or None if it was not built."""
     global _ref
