@@ -174,10 +174,13 @@ int miso_attn_prefill(const float* q, const float* qg, const uint16_t* k_cache,
  * the balanced sizes, a NULL or misaligned workspace or one smaller than required.
  *
  * With a workspace of miso_attn_prefill_parts_workspace_bytes(max_n) bytes (which also holds the
- * balanced form's for n <= 2048; same zero fill), launches of n <= max_n tokens up to 3072 that
- * leave the chip idle otherwise -- few tokens after a prefix -- run in parts: the keys of every
- * token block are split between workgroups and a second kernel joins the parts (two launches,
- * bit-equal from call to call). A smaller workspace keeps the forms above.
+ * balanced form's for n <= 2048), launches of n <= max_n tokens up to 3072 that leave the chip idle
+ * otherwise -- few tokens after a prefix -- run in parts: the keys of every token block are split
+ * between workgroups and a second kernel joins the parts (two launches, bit-equal from call to
+ * call). These partials are large, since any launch may follow a long prefix: 2 MiB for 1 token, 34
+ * MB for 16, 76 for 512, 118 from 3072 on. A launch whose own partials do not fit the workspace it
+ * is given runs in the forms above, so miso_attn_prefill_workspace_bytes keeps the small ones.
+ * Only the pair counters, the first 1024 bytes, have to start at zero.
  *
  * Launches of up to 640 tokens that gain nothing in parts run miso_attn_prefill's layout, which is
  * the faster one there (the workspace is checked all the same). */
@@ -392,10 +395,12 @@ typedef struct miso_attn_layer {
 /* Device floats of the decode / prefill workspaces (the engine's AttentionScratch and
  * AttentionPrefillScratch, src/engine/attention.hpp:44-69), for chunks of up to max_tok tokens.
  * The prefill workspace ends with the causal prefill's (miso_attn_prefill_ws, balanced pairs and
- * parts): zero-fill it once when it is allocated (every call leaves its
- * pair counters zero). */
+ * parts; its sizes there): zero its pair counters, 256 words at float offset
+ * miso_attn_layer_prefill_counters(max_tok), once when it is allocated (every call leaves them
+ * zero; zero-filling the whole workspace does as well). */
 uint64_t miso_attn_layer_decode_ws(void);
 uint64_t miso_attn_layer_prefill_ws(uint32_t max_tok);
+uint64_t miso_attn_layer_prefill_counters(uint32_t max_tok);
 
 /* Where each step leaves the attention output before the output projection, as a float offset
  * into its workspace: the engine's AttentionScratch::core (16 heads x 256 floats, the last decode

@@ -76,8 +76,7 @@ AttentionPrefillScratch::AttentionPrefillScratch(unsigned n)
       core(std::size_t{n} * L::kCore),
       balance(L::prefill_balance_floats(n)) {
   // The balanced prefill's pair counters start at zero (every chunk leaves them so).
-  if (balance.size() != 0)
-    MISO_HIP_CHECK(hipMemset(balance.data(), 0, balance.size() * sizeof(float)));
+  MISO_HIP_CHECK(hipMemset(balance.data(), 0, kernels::kAttnSplitCounterBytes));
 }
 
 void attention_decode(const AttentionLayer& w, AttentionCache& cache, AttentionScratch& sc,

@@ -62,9 +62,9 @@ struct AttentionScratch {
 
 // Prefill workspace for chunks of up to max_tok tokens, with the engine's members, as the last
 // chunk left them (the normed rows, the projections, the prepared q, the [n][16][256] attention
-// output `core`), plus `balance`: the balanced prefill's
-// partials and pair counters for chunks of up to min(max_tok, 4096) tokens, zero-filled once here
-// (every chunk leaves the counters zero).
+// output `core`), plus `balance`: the causal prefill's pair
+// counters, zeroed once here (every chunk leaves them so), and partials (balanced pairs, parts: up
+// to 118 MB, what chunks of max_tok tokens can use after any prefix).
 struct AttentionPrefillScratch {
   explicit AttentionPrefillScratch(unsigned max_tok);
   unsigned max_tok;

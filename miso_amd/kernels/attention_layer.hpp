@@ -378,9 +378,8 @@ inline DecodeWorkspace decode_workspace(float* ws) {
 }
 
 // The prefill workspace ends with the causal prefill's own (attn_prefill_launch: balanced pairs
-// or parts, for chunks of up to max_tok tokens): its pair counters must be zero before the first
-// chunk, so the whole prefill workspace is zero-filled once when it is allocated (every chunk
-// leaves the counters zero).
+// or parts, for chunks of up to max_tok tokens): its pair counters (the first
+// kAttnSplitCounterBytes of it) must be zero before the first chunk; every chunk leaves them so.
 struct PrefillWorkspace {
   float* proj;   // [max_tok][9216]
   float* q;      // [max_tok][16][256]

@@ -175,7 +175,6 @@ __host__ __device__ constexpr std::size_t attn_prefill_split_workspace_bytes(uns
 // ------------------------------------------------------------------------------------------------
 
 constexpr unsigned kAttnPartsMaxWorkers = 128;  // per KV head: 256 CUs, one workgroup each
-constexpr unsigned kAttnPartsMaxBlocks = 256;   // token blocks per KV head (8 bits of a cut)
 
 struct AttnPrefillCuts {
   unsigned workers, blocks;
@@ -185,7 +184,7 @@ struct AttnPrefillCuts {
 
 struct AttnPrefillPartsParams {
   AttnPrefillParams a;
-  float* part_o;   // [slot][rows][256], rows = 128 per row block per wave, relative to 2^m
+  float* part_o;   // [slot][rows][256], rows = attn_prefill_parts_rows, relative to 2^m
   float* part_ml;  // [slot][rows][2]: m (log2 units), l
   AttnPrefillCuts cuts;
 };
@@ -196,11 +195,16 @@ __host__ __device__ constexpr unsigned attn_prefill_parts_slots(unsigned workers
                                                                 unsigned blocks) {
   return attn::kKvHeads * (workers + blocks);
 }
-__host__ __device__ constexpr std::size_t attn_prefill_parts_bytes(unsigned workers,
-                                                                   unsigned blocks,
-                                                                   unsigned row_blocks) {
-  return std::size_t{attn_prefill_parts_slots(workers, blocks)} * 128 * row_blocks *
-         (attn::kDim + 2) * sizeof(float);
+// Rows of a slot: 8 heads x the tokens of a block, or of the launch if those are fewer.
+__host__ __device__ constexpr unsigned attn_prefill_parts_rows(unsigned n, unsigned row_blocks) {
+  const unsigned tokens = kAttnQBlock * row_blocks;
+  return attn::kQHeads / attn::kKvHeads * (n < tokens ? n : tokens);
+}
+// The partials of a launch of n tokens.
+constexpr std::size_t attn_prefill_parts_bytes(unsigned n, unsigned row_blocks) {
+  const unsigned tokens = kAttnQBlock * row_blocks, blocks = (n + tokens - 1) / tokens;
+  return std::size_t{attn_prefill_parts_slots(kAttnPartsMaxWorkers, blocks)} *
+         attn_prefill_parts_rows(n, row_blocks) * (attn::kDim + 2) * sizeof(float);
 }
 
 // Tiles of 32 keys that block b (of `tokens` tokens each) of a launch sees.
@@ -225,10 +229,11 @@ constexpr unsigned kAttnPartsJobTiles = 12;
 //     prefix makes costly: 2100 after 8000 336 against 506, 3001 after 5003 363 against 388; 3001
 //     after 0 112 against 104 and 3300 after 4000 352 against 343 (one workgroup per block kept).
 //   - Two row blocks per wave (half the LDS reads per MFMA, twice the prologue and partial) pay
-//     from about 150 one-block tiles per worker: 512 after 32000 280 against 330 with one, 700
+//     from about 150 one-block tiles per worker (and with tokens for both): 512 after 32000 280 against 330 with one, 700
 //     after 14000 207 against 223; 512 after 4096 (34 tiles) 78 against 65, 2500 after 2500 (145)
 //     206 against 190.
 constexpr unsigned kAttnPartsMaxTokens = 3072;
+static_assert(kAttnPartsMaxTokens / kAttnQBlock < 1u << 9, "a block in the top 9 bits of a place");
 inline unsigned attn_prefill_parts_row_blocks(unsigned pos0, unsigned n) {
   if (n == 0 || n > kAttnPartsMaxTokens || std::uint64_t{pos0} + n >= 1u << 27)
     return 0;
@@ -240,15 +245,17 @@ inline unsigned attn_prefill_parts_row_blocks(unsigned pos0, unsigned n) {
   const bool pays = n <= 2048
                         ? per_block >= per_worker + per_worker / 16 + 10 + per_block / 8
                         : pos0 >= n;
-  return !pays ? 0 : per_worker >= 150 ? 2 : 1;
+  return !pays ? 0 : per_worker >= 150 && n > kAttnQBlock ? 2 : 1;
 }
 
-// Workspace with which every launch of up to max_n tokens can run in parts or in balanced pairs:
-// the pairs' counters, then the parts' (m, l) and O.
+// Workspace with which every launch of up to max_n tokens can run in parts, or in balanced pairs up
+// to 2048 tokens: the pairs' counters, then the parts' (m, l) and O. 2 MiB for 1 token, 34 MB
+// for 16, 68 for 32, 76 for 512, 118 from 3072 on, since any launch may follow a long prefix.
 constexpr std::size_t attn_prefill_parts_workspace_bytes(unsigned max_n) {
   const unsigned n = max_n < kAttnPartsMaxTokens ? max_n : kAttnPartsMaxTokens;
-  return kAttnSplitCounterBytes +
-         attn_prefill_parts_bytes(kAttnPartsMaxWorkers, (n + 31) / 32, 2);
+  const std::size_t one = attn_prefill_parts_bytes(n, 1);
+  const std::size_t two = n > kAttnQBlock ? attn_prefill_parts_bytes(n, 2) : 0;
+  return kAttnSplitCounterBytes + (one > two ? one : two);
 }
 
 // Cuts the tiles of n tokens after pos0 in blocks of 16 row_blocks tokens into at most
@@ -1276,11 +1283,12 @@ __device__ __attribute__((always_inline)) inline void prefill_items(
       if constexpr (kParts) {
         if (jb.part) {  // uniform: (m, l) and the rows of O to the part's slot, for the merge
           store = false;
-          const std::size_t row0 = std::size_t{jb.slot} * kPartRows + 32 * kBlocks * wave;
+          const std::size_t row0 =
+              std::size_t{jb.slot} * attn_prefill_parts_rows(p.n, kBlocks) + 32 * kBlocks * wave;
 #pragma unroll
           for (int c = 0; c < kBlocks; ++c) {
             stage_o(c, 1.0f);
-            if (hi == 0)
+            if (hi == 0 && tw + 4 * c + col / kGroup < p.n)
               *reinterpret_cast<float2*>(sp->part_ml + 2 * (row0 + 32 * c + col)) =
                   float2{rw.m[c], l_row[c]};
             float* out = sp->part_o + (row0 + 32 * c) * kDim + 4 * lane;
@@ -1404,11 +1412,13 @@ __global__ void __launch_bounds__(256) attn_prefill_parts_kernel(AttnPrefillPart
 // 2 w + 1, lane l dimensions 4 l .. 4 l + 3. With M the largest m of a row's parts,
 // O = sum O_i 2^(m_i - M) and L = sum l_i 2^(m_i - M) in tile order; core = O / L * sigmoid(gate).
 // Bound by the partials it reads (1 KiB per row and part, mostly from the memory-side cache), so
-// every part of both rows is in flight before the first is used, eight parts at a time.
-template <int kRowBlocks>
+// every part of both rows is in flight before the first is used, eight parts at a time. kShort: a
+// launch of fewer tokens than a block has (otherwise the parts lie a constant apart, which the
+// loads fold into their offsets: 512 tokens after 1536 38.6 us against 39.4).
+template <int kRowBlocks, bool kShort>
 __global__ void __launch_bounds__(256) attn_prefill_merge_kernel(AttnPrefillPartsParams p) {
   using attn::kDim;
-  constexpr unsigned kTokens = kAttnQBlock * kRowBlocks, kPartRows = 128 * kRowBlocks;
+  constexpr unsigned kTokens = kAttnQBlock * kRowBlocks;
   constexpr unsigned kGroup = attn::kQHeads / attn::kKvHeads, kBatch = 8;
   const unsigned tok = blockIdx.x / attn::kKvHeads, kvh = blockIdx.x % attn::kKvHeads;
   const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -1428,7 +1438,8 @@ __global__ void __launch_bounds__(256) attn_prefill_merge_kernel(AttnPrefillPart
   const unsigned parts = w1 - w0 + 1;
   // Worker w0 - 1 + i, slot + block as attn_prefill_parts_slots says; rows 8 (token in block) + head.
   const std::size_t slot0 = std::size_t{kvh} * (p.cuts.workers + p.cuts.blocks) + w0 - 1 + blk;
-  const std::size_t row0 = slot0 * kPartRows + 8 * (tok % kTokens) + 2 * wave;
+  const unsigned part_rows = attn_prefill_parts_rows(kShort ? p.a.n : kTokens, kRowBlocks);
+  const std::size_t row0 = slot0 * part_rows + 8 * (tok % kTokens) + 2 * wave;
   const float* o0 = p.part_o + row0 * kDim + 4 * lane;
   const float* ml0 = p.part_ml + row0 * 2;
   const std::size_t gate_at =
@@ -1441,7 +1452,7 @@ __global__ void __launch_bounds__(256) attn_prefill_merge_kernel(AttnPrefillPart
     float4 x[kBatch][2], ml[kBatch];
 #pragma unroll
     for (unsigned i = 0; i < kBatch; ++i) {
-      const std::size_t at = std::size_t{i0 + i < parts ? i0 + i : parts - 1} * kPartRows;
+      const std::size_t at = std::size_t{i0 + i < parts ? i0 + i : parts - 1} * part_rows;
       ml[i] = *reinterpret_cast<const float4*>(ml0 + at * 2);  // (m, l) of both rows
       x[i][0] = *reinterpret_cast<const float4*>(o0 + at * kDim);
       x[i][1] = *reinterpret_cast<const float4*>(o0 + (at + 1) * kDim);
@@ -1497,23 +1508,28 @@ inline bool attn_prefill_in_parts(const AttnPrefillParams& a, void* workspace, s
   const unsigned row_blocks = attn_prefill_parts_row_blocks(a.pos0, a.n);
   if (row_blocks == 0)
     return false;
-  const unsigned blocks = (a.n + kAttnQBlock * row_blocks - 1) / (kAttnQBlock * row_blocks);
-  if (bytes < kAttnSplitCounterBytes +
-                  attn_prefill_parts_bytes(kAttnPartsMaxWorkers, blocks, row_blocks))
+  if (bytes < kAttnSplitCounterBytes + attn_prefill_parts_bytes(a.n, row_blocks))
     return false;
   AttnPrefillPartsParams p{a, nullptr, nullptr,
                            attn_prefill_cuts(a.pos0, a.n, row_blocks, kAttnPartsMaxWorkers)};
   p.part_ml =
       reinterpret_cast<float*>(static_cast<char*>(workspace) + kAttnSplitCounterBytes);
-  p.part_o = p.part_ml + std::size_t{attn_prefill_parts_slots(p.cuts.workers, blocks)} * 128 *
-                             row_blocks * 2;
+  p.part_o = p.part_ml + std::size_t{attn_prefill_parts_slots(p.cuts.workers, p.cuts.blocks)} *
+                             attn_prefill_parts_rows(a.n, row_blocks) * 2;
   const unsigned grid = 8 * ((p.cuts.workers + 3) / 4), rows = a.n * attn::kKvHeads;
+  const bool is_short = a.n < kAttnQBlock * row_blocks;
   if (row_blocks == 2) {
     attn_prefill_parts_kernel<2><<<grid, 256, 0, stream>>>(p);
-    attn_prefill_merge_kernel<2><<<rows, 256, 0, stream>>>(p);
+    if (is_short)
+      attn_prefill_merge_kernel<2, true><<<rows, 256, 0, stream>>>(p);
+    else
+      attn_prefill_merge_kernel<2, false><<<rows, 256, 0, stream>>>(p);
   } else {
     attn_prefill_parts_kernel<1><<<grid, 256, 0, stream>>>(p);
-    attn_prefill_merge_kernel<1><<<rows, 256, 0, stream>>>(p);
+    if (is_short)
+      attn_prefill_merge_kernel<1, true><<<rows, 256, 0, stream>>>(p);
+    else
+      attn_prefill_merge_kernel<1, false><<<rows, 256, 0, stream>>>(p);
   }
   return true;
 }

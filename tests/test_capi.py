@@ -234,14 +234,37 @@ def test_prefill_workspace_bytes(lib):
         lib.miso_attn_prefill_workspace_bytes(4096)
 
 
+def test_prefill_parts_workspace_bytes(lib):
+    """Parts: a slot per (worker + block) of both KV heads, at most 128 workers, 8 rows per token of a
+    block or of a shorter launch; two row blocks only with tokens for both. No launch of up to max_n
+    tokens needs more, and the balanced form up to 2048 tokens fits; a single token takes 2 MiB."""
+    def parts(n, rb):
+        tokens = 16 * rb
+        return 2 * (128 + -(-n // tokens)) * 8 * min(n, tokens) * 258 * 4
+    size = lib.miso_attn_prefill_parts_workspace_bytes
+    assert size(0) == 1024
+    most = 0
+    for n in range(1, 3073):
+        need = max(parts(n, 1), parts(n, 2) if n > 16 else 0)
+        most = max(most, need)
+        assert size(n) == 1024 + most, n
+        assert n > 2048 or size(n) >= lib.miso_attn_prefill_workspace_bytes(n)
+    assert size(3073) == size(1 << 31) == size(3072)
+    assert size(1) < 2.2e6 and size(16) < 34.1e6
+
+
 def test_layer_core_offsets(lib):
     """The engine's scratch.core / ps.core inside the layer workspaces: 16-byte aligned, inside
-    the workspace, and not overlapping the balanced prefill's counters at the prefill workspace's
-    end."""
+    the workspace, and before the GEMM input (f16 values and sums of [max_tok][4096]) and the causal
+    prefill's counters and partials (pairs or parts, whichever is larger) that end the prefill
+    workspace."""
     dec = lib.miso_attn_layer_decode_core()
     assert dec % 4 == 0 and dec + 4096 <= lib.miso_attn_layer_decode_ws()
     for max_tok in (1, 16, 512, 4096, 8192):
         at = lib.miso_attn_layer_prefill_core(max_tok)
-        balance = lib.miso_attn_prefill_workspace_bytes(min(max_tok, 4096)) // 4
-        assert at % 4 == 0
-        assert at + max_tok * 4096 <= lib.miso_attn_layer_prefill_ws(max_tok) - balance
+        balance = max(lib.miso_attn_prefill_workspace_bytes(min(max_tok, 4096)),
+                      lib.miso_attn_prefill_parts_workspace_bytes(max_tok)) // 4
+        counters = lib.miso_attn_layer_prefill_counters(max_tok)
+        assert at % 4 == 0 and counters % 4 == 0
+        assert at + max_tok * (4096 + 2048 + 128) <= counters
+        assert counters + balance <= lib.miso_attn_layer_prefill_ws(max_tok)

@@ -298,3 +298,27 @@ def test_prefill_hidden_keys(O, attn, torch_mod, prefill_scratch, pos0, n):
         st = O.compare(run_prefill(attn, torch_mod, p, scratch=scratch)[rows], ref)
         report(f"hidden keys pos0={pos0} n={n}", st)
         assert st["ok"], st
+
+
+@pytest.mark.parametrize("pos0,n", [(20000, 1), (500, 13), (5000, 16), (700, 17), (308000, 20),
+                                    (12001, 203), (4096, 2100)])
+def test_prefill_parts_stay_in_their_workspace(attn, torch_mod, pos0, n):
+    """A workspace sized for n tokens (less than a block's rows a slot up to 16 tokens, up to 31 with
+    two row blocks: 20 tokens after 308000) holds every partial: nothing behind it is touched, and
+    the result is the plain form's inside the prefill gate."""
+    torch = torch_mod
+    g = torch.Generator(device="cuda").manual_seed(n)
+    q = torch.randn(n * H * D, generator=g, device="cuda")
+    qg = torch.randn(n * H * 2 * D, generator=g, device="cuda")
+    k, v = (torch.randn(2 * (pos0 + n) * D, generator=g, dtype=torch.float16, device="cuda")
+            for _ in range(2))
+    sc = attn.PrefillScratch(n)
+    sc.buf = torch.full((sc.nbytes // 4 + (1 << 20),), 0x5A5A5A5A, dtype=torch.int32, device="cuda")
+    sc.buf[:256].zero_()
+    core, plain = torch.empty_like(q), torch.empty_like(q)
+    attn.attn_prefill(q, qg, k, v, core, pos0, n, pos0 + n, scratch=sc)
+    attn.attn_prefill(q, qg, k, v, plain, pos0, n, pos0 + n)
+    assert bool((sc.buf[sc.nbytes // 4:] == 0x5A5A5A5A).all())
+    assert not bool(sc.buf[:256].any())
+    assert bool(((core - plain).abs() <= 2e-3 + 1e-2 * plain.abs()).all())
+    assert not torch.equal(core, plain)  # it did run in parts
