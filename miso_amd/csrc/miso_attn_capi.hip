@@ -379,18 +379,22 @@ uint64_t miso_attn_prefill_parts_workspace_bytes(uint32_t max_n) {
   return k::attn_prefill_parts_workspace_bytes(max_n);
 }
 
-// Checks the workspace of a prefill whose other arguments are good, and launches it.
+// Why a prefill of n tokens cannot use this workspace, or nullptr. A launch that would run one
+// workgroup per block takes any workspace, also none.
+static const char* bad_workspace(uint32_t n, const void* workspace, uint64_t bytes) {
+  if (!k::attn_prefill_balanced(n))
+    return nullptr;
+  if (bad_ptr(workspace))
+    return "workspace must be a non-null, 16-byte aligned device pointer";
+  if (bytes < k::attn_prefill_split_workspace_bytes(n))
+    return "workspace smaller than miso_attn_prefill_workspace_bytes(n)";
+  return nullptr;
+}
+
+// Launches a prefill whose arguments are good.
 static int prefill_with_ws(const char* fn, const k::AttnPrefillParams& a, void* workspace,
                            uint64_t bytes, void* stream) {
-  // A launch that would run one workgroup per block takes any workspace, also none.
-  const bool usable = !bad_ptr(workspace);
-  if (k::attn_prefill_balanced(a.n)) {
-    if (!usable)
-      return fail(fn, "workspace must be a non-null, 16-byte aligned device pointer");
-    if (bytes < k::attn_prefill_split_workspace_bytes(a.n))
-      return fail(fn, "workspace smaller than miso_attn_prefill_workspace_bytes(n)");
-  }
-  k::attn_prefill_launch(a, workspace, usable ? bytes : 0, as_stream(stream));
+  k::attn_prefill_launch(a, workspace, bad_ptr(workspace) ? 0 : bytes, as_stream(stream));
   return launched(fn);
 }
 
@@ -402,6 +406,8 @@ int miso_attn_prefill_ws(const float* q, const float* qg, const uint16_t* k_cach
   if (const int rc =
           prefill_args(fn, q, qg, k_cache, v_cache, core, pos0, n, max_ctx, qg_stride))
     return rc;
+  if (const char* err = bad_workspace(n, workspace, workspace_bytes))
+    return fail(fn, err);
   const k::AttnPrefillParams a{q,    qg, as_half(k_cache), as_half(v_cache), core, pos0,
                                n,    max_ctx, qg_stride};
   return prefill_with_ws(fn, a, workspace, workspace_bytes, stream);
@@ -678,6 +684,9 @@ int miso_attn_prefill_fp8_ws(const float* q, const float* qg, const uint8_t* k8,
                              uint32_t n, uint32_t max_ctx, uint32_t qg_stride, void* workspace,
                              uint64_t workspace_bytes, void* stream) {
   constexpr const char* fn = "miso_attn_prefill_fp8_ws";
+  // Before the widening: a rejected call writes nothing.
+  if (const char* err = bad_workspace(n, workspace, workspace_bytes))
+    return fail(fn, err);
   if (const int rc = prefill_fp8_widen(fn, q, qg, k8, v8, k_scale, v_scale, k_ws, v_ws, core, pos0,
                                        n, max_ctx, qg_stride, stream))
     return rc;

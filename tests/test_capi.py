@@ -79,6 +79,12 @@ def test_host_validation_rejects_bad_arguments(lib):
     need = lib.miso_attn_prefill_workspace_bytes(2000)
     rejected(lib.miso_attn_prefill_ws(P, P, P, P, P, 0, 2000, 2000, 8192, P, need - 1, N), lib,
              "smaller than")
+    # the fp8 prefill too, before its first launch (the widening into k_ws / v_ws)
+    fp8 = lib.miso_attn_prefill_fp8_ws
+    for ws, nbytes, why in ((N, W, "non-null"), (P + 4, W, "aligned"), (P, need - 1, "smaller")):
+        rejected(fp8(P, P, P, P, P, P, P, P, P, 0, 2000, 2000, 8192, ws, nbytes, N), lib, why)
+    rejected(fp8(P, P, P, P, P, P, P, P, P, 0, 0, 10, 8192, P, W, N), lib, "n must be >= 1")
+    rejected(fp8(P, P, P, P, P, P, P, P, P, 8, 3, 10, 8192, P, W, N), lib, "KV cache is full")
     rejected(lib.miso_attn_prep(P, P, P, P, P, P, P, P, P, 10, 10, 1e-6, N), lib, "full")
     rejected(lib.miso_attn_prep_batch(P, P, P, P, P, P, P, P, P, 8, 10, 1e-6, 3, 9216, N), lib,
              "full")
