@@ -425,9 +425,7 @@ uint64_t miso_attn_ragged_partials(uint32_t batch, uint32_t max_len) {
 }
 
 uint64_t miso_attn_ragged_balanced_partials(uint32_t batch, uint32_t max_len) {
-  return uint64_t{batch} * k::attn::kKvHeads * k::attn_ragged_balanced_splits(batch, max_len) *
-             (k::attn::kQHeads / k::attn::kKvHeads) +
-         4;
+  return k::attn_ragged_balanced_rows(batch, max_len) * k::attn::kQHeads + 4;
 }
 
 // The scratch rows per (sequence, KV head) that `partials` floats of part_m hold beside the span

@@ -2516,6 +2516,17 @@ __host__ __device__ constexpr unsigned attn_ragged_balanced_splits(unsigned batc
   const unsigned n = fine < share ? fine : share, least = attn_ragged_splits(max_len);
   return n > least ? n : least;
 }
+// Scratch rows of one KV head over the batch: no less than any smaller batch or shorter max_len takes
+// (the splits above times the batch is not monotone), so scratch for one serves the others.
+__host__ __device__ constexpr std::size_t attn_ragged_balanced_rows(unsigned batch,
+                                                                    unsigned max_len) {
+  const unsigned keys = 32 * kAttnBalancedMinTiles;
+  const std::size_t fine = std::size_t{batch} * (max_len / keys + (max_len % keys != 0));
+  const std::size_t share = std::size_t{batch} + 256;
+  const std::size_t n = fine < share ? fine : share;
+  const std::size_t least = std::size_t{batch} * attn_ragged_splits(max_len);
+  return n > least ? n : least;
+}
 // Whether a streaming launch of `grid` workgroups on `cus` CUs balances its spans. Sequences of up to
 // 128 keys are one span each either way (1 of 113: 11.6 us, with a choice 12.5).
 __host__ __device__ constexpr bool attn_ragged_balanced(unsigned batch, unsigned max_len,

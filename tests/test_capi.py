@@ -224,6 +224,22 @@ def test_ragged_scratch_sizes(lib):
     assert lib.miso_attn_ragged_partials(64, 16384) == 64 * 2 * 32 * 8
 
 
+def test_ragged_balanced_partials(lib):
+    """Room for balanced spans: the plain spans' at least, about two spans per CU over the batch
+    (spans of 128 keys or more) and the chosen span's word, and never less for a larger batch or
+    longer sequences, so that scratch serves every smaller batch."""
+    size = lib.miso_attn_ragged_balanced_partials
+    for max_len in (1, 128, 129, 512, 513, 4096, 9001, 16384, 262144):
+        least, last = (max_len + 511) // 512, 0
+        for batch in range(1, 520):
+            n = size(batch, max_len)
+            fine = min(-(-max_len // 128), 1 + 256 // batch)
+            assert n >= batch * 16 * max(fine, least) + 4
+            assert n <= 16 * max(batch * least, batch + 256) + 4
+            assert n >= last and n >= size(batch, max(1, max_len - 77)), (batch, max_len)
+            last = n
+
+
 def test_prefill_workspace_bytes(lib):
     """The balanced prefill's workspace (n <= 2048, 3841 <= n <= 4096): a fixed 1 KiB of pair
     counters, then (m, l) and O of both parts of each pair (128 rows per part with 16-token
