@@ -422,7 +422,7 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const QGemmParam
 //
 // Stage s: the MFMAs read activations and expanded weights of stage s while the same threads
 // expand stage s + 1 into the other weight buffer. kRing 3 keeps two stages of activations in
-// flight, with counted waits (the waves then have no other loads); kRing 2 one stage.
+// flight, with counted waits (the waves then have no other loads), kRing 4 three; kRing 2 one stage.
 // Per output element the arithmetic is gemm_tile's in the same order: all tile shapes give
 // bit-identical results.
 //
@@ -448,7 +448,7 @@ __device__ __attribute__((always_inline)) inline void gemm_tile_wide(
   constexpr unsigned kXInstr = kTok / 8 / kWaves;  // activation DMAs per wave and stage
   static_assert(kRow * 4 == 64 * kWaves, "four threads expand a row's stage");
   static_assert(kTok / 32 <= kWaves && kXInstr >= 1 && MB >= 1 && NB >= 1);
-  static_assert(kRing == 2 || kRing == 3);
+  static_assert(kRing >= 2 && kRing <= 4);
   const unsigned t = threadIdx.x, lane = t % 64;
   const unsigned wave = __builtin_amdgcn_readfirstlane(t / 64);
   const unsigned wt = wave / WN, wr = wave % WN, col = lane % 32, kq = lane / 32;
@@ -483,8 +483,13 @@ __device__ __attribute__((always_inline)) inline void gemm_tile_wide(
   };
 
   // Q4_K: nibbles (32 rows an instruction), headers (64 rows) and activation sums (32 tokens) by
-  // the first waves, one instruction each.
-  const bool nib_wave = wave < kRow / 32, head_wave = wave < kRow / 64, xs_wave = wave < kTok / 32;
+  // the first waves, one instruction each; with kRing 4 the headers and sums by the last ones, so that
+  // the waves of the nibbles issue the same in every stage.
+  constexpr unsigned kHead0 = kRing == 4 ? kWaves - kRow / 64 : 0;
+  constexpr unsigned kXs0 = kRing == 4 ? kWaves - kTok / 32 : 0;
+  static_assert(kRing != 4 || (kHead0 >= kRow / 32 && kXs0 >= kRow / 32));
+  const bool nib_wave = wave < kRow / 32, head_wave = wave - kHead0 < kRow / 64;
+  const bool xs_wave = wave - kXs0 < kTok / 32;
   const std::uint8_t* nsrc = w_row(32 * (wave % (kRow / 32)) + lane / 2) + 16 + 16 * (lane % 2);
   const std::uint8_t* hsrc = w_row(64 * (wave % (kRow / 64)) + lane);
   const float* ssrc = nullptr;
@@ -502,22 +507,24 @@ __device__ __attribute__((always_inline)) inline void gemm_tile_wide(
   };
   auto load_head = [&](unsigned b) __attribute__((always_inline)) {
     const unsigned at = 4 * b < n_stages ? b : n_stages / 4 - 1;
-    cdna4::lds_load16(hsrc + 144 * at, head_lds + (b & 1u) * (kRow * 16) + 1024 * wave);
+    cdna4::lds_load16(hsrc + 144 * at, head_lds + (b & 1u) * (kRow * 16) + 1024 * (wave - kHead0));
   };
   auto load_xs = [&](unsigned b) __attribute__((always_inline)) {
-    cdna4::lds_load16(ssrc + 8 * b, xs_lds + 1024 * wave);
+    cdna4::lds_load16(ssrc + 8 * b, xs_lds + 1024 * (wave - kXs0));
   };
-  // With kRing 3 every DMA of stage s - 2 and before has landed when only those of stage s - 1 are
-  // outstanding (the activations' and `extra` more); with kRing 2 (and Q6_K) all have to be in.
+  // Stage s needs every DMA of stage s - kRing + 1 and before; outstanding may be those of the
+  // kRing - 2 stages since: their activations' and `extra` more. With kRing 2 (and Q6_K) all have to be
+  // in.
   auto wait = [&](unsigned extra) __attribute__((always_inline)) {
+    constexpr unsigned kX = (kRing - 2) * kXInstr;
     if (kRing == 2 || !kQ4)
       cdna4::wait_vmcnt<0>();
     else if (extra == 0)
-      cdna4::wait_vmcnt<kXInstr>();
+      cdna4::wait_vmcnt<kX>();
     else if (extra == 1)
-      cdna4::wait_vmcnt<kXInstr + 1>();
+      cdna4::wait_vmcnt<kX + 1>();
     else
-      cdna4::wait_vmcnt<kXInstr + 2>();
+      cdna4::wait_vmcnt<kX + 2>();
   };
 
   // Expansion of a stage into weight buffer s % 2 by thread (row er = t / 4, quarter eq = t % 4).
@@ -593,23 +600,34 @@ __device__ __attribute__((always_inline)) inline void gemm_tile_wide(
       acc[i][j] = c[i][j] = float16_t{};
 
   Half raw{}, ahead{};
+  // In the order in which they are waited for: what expands stage 0, stage 0 itself, then what the
+  // stages since would have issued.
   if constexpr (kQ4) {
     if (head_wave)
       load_head(0);
+    if (nib_wave) {
+      load_nib(0, 0);
+      load_nib(1, 1);
+    }
+    for (unsigned s = 0; s + 1 < kRing; ++s) {
+      load_x(s, s);
+      if (s != 0 && nib_wave)
+        load_nib(s + 1, s + 1);
+    }
     if (nib_wave)
-      for (unsigned s = 0; s < kRing; ++s)
-        load_nib(s, s);
+      cdna4::wait_vmcnt<(kRing - 1) * (kXInstr + 1)>();
+    else
+      cdna4::wait_vmcnt<(kRing - 1) * kXInstr>();
+    barrier();
+    expand_q4(0, 0);
   } else {
     raw = fetch_half(0);
-  }
-  for (unsigned s = 0; s + 1 < kRing; ++s)
-    load_x(s, s);
-  cdna4::wait_vmcnt<0>();
-  barrier();
-  if constexpr (kQ4)
-    expand_q4(0, 0);
-  else
+    for (unsigned s = 0; s + 1 < kRing; ++s)
+      load_x(s, s);
+    cdna4::wait_vmcnt<0>();
+    barrier();
     expand_q6(0, raw);
+  }
 
   // Operand addresses: row 32 i + col of a tile, chunk 2 kk + kq.
   unsigned at[4];
@@ -621,8 +639,12 @@ __device__ __attribute__((always_inline)) inline void gemm_tile_wide(
 #pragma unroll
     for (unsigned j = 0; j < 4; ++j) {
       const unsigned s = s4 + j;
-      // What stage s - 1 issued besides its activations (everything of the prologue is in).
-      wait((nib_wave ? 1u : 0u) + (j == 1 && xs_wave ? 1u : 0u) + (j == 2 && head_wave ? 1u : 0u));
+      // What the last kRing - 2 stages (the prologue's among them) issued besides activations; with
+      // kRing 4 not the headers and sums (once a block their waves wait for a little more).
+      if constexpr (kRing == 4)
+        wait(nib_wave ? 2u : 0u);
+      else
+        wait((nib_wave ? 1u : 0u) + (j == 1 && xs_wave ? 1u : 0u) + (j == 2 && head_wave ? 1u : 0u));
       barrier();  // stage s complete for every wave, and every wave done with stage s - 1
       load_x(s + kRing - 1, spare);
       if constexpr (kQ4) {
@@ -630,7 +652,7 @@ __device__ __attribute__((always_inline)) inline void gemm_tile_wide(
           load_nib(s + kRing, cur);  // slot of stage s, expanded in stage s - 1
         if (j == 0 && xs_wave)
           load_xs(s4 / 4);  // read at j == 3; the last block's were read before this barrier
-        if (j == 1 && head_wave)
+        if (j == (kRing == 4 ? 0 : 1) && head_wave)
           load_head(s4 / 4 + 1);  // expanded from at j == 3
       } else if (j % 2 == 0) {
         ahead = fetch_half(s / 2 + 1);
@@ -712,10 +734,14 @@ __device__ __attribute__((always_inline)) inline void gemm_tile_wide(
           }
         }
       }
-      const unsigned tmp = cur;
-      cur = nxt;
-      nxt = kRing == 2 ? tmp : spare;
-      spare = kRing == 2 ? nxt : tmp;
+      if constexpr (kRing == 4) {  // stage s is in slot s % 4
+        cur = (j + 1) % 4, nxt = (j + 2) % 4, spare = j;
+      } else {
+        const unsigned tmp = cur;
+        cur = nxt;
+        nxt = kRing == 2 ? tmp : spare;
+        spare = kRing == 2 ? nxt : tmp;
+      }
     }
   }
   // Lane (row col of block n, half kq) holds tokens 8 (r / 4) + 4 kq + r % 4 of token block i.
@@ -822,6 +848,11 @@ __global__ void __launch_bounds__(64 * WM * WN, kWavesPerSimd) qgemm_wide_kernel
 // kGroup (token tiles swept across the row tiles) keeps the ~32 to 96 tiles an XCD runs at once
 // within its 4 MiB of L2 also at k = 4096: 2048 rows x 4096, 512 tokens in 64 x 64 tiles 36 us
 // in groups of 8, 31 in groups of 4.
+// 64 x 64 tiles, one workgroup per CU: nothing hides a stage's wait, and weights come from memory (a
+// model's layers do not stay in the L2s), so Q4_K takes four stages in the ring. Weights of 80
+// matrices in turn, with two stages and four: 2048 rows x 4096, 13 tokens 30.8 / 26.4 us, 512 tokens
+// 34.8 / 27.3; 8192 rows x 2048, 64 tokens 19.6 / 15.8; a whole layer over 512 tokens 125 / 118. Q6_K
+// waits for its weights' registers at every other stage, and stays with two: 512 rows x 2048 19.5 / 20.9.
 inline void qgemm_launch(const QGemmBatch& p, hipStream_t stream) {
   auto tiles = [&](unsigned tok, unsigned row) {
     unsigned rows = 0;
@@ -844,7 +875,12 @@ inline void qgemm_launch(const QGemmBatch& p, hipStream_t stream) {
       best = i, least = t;
   }
   switch (best) {
-    case 0: qgemm_wide_kernel<64, 64, 2, 2, 2, 2, 4><<<count[0], 256, 0, stream>>>(p); break;
+    case 0:
+      if (count[0] <= 256 && p.format[0] == QFormat::Q4K)
+        qgemm_wide_kernel<64, 64, 2, 2, 4, 2, 4><<<count[0], 256, 0, stream>>>(p);
+      else
+        qgemm_wide_kernel<64, 64, 2, 2, 2, 2, 4><<<count[0], 256, 0, stream>>>(p);
+      break;
     case 1: qgemm_wide_kernel<128, 64, 2, 2, 2, 2, 2><<<count[1], 256, 0, stream>>>(p); break;
     case 2: qgemm_wide_kernel<128, 128, 2, 4, 2, 4, 2><<<count[2], 512, 0, stream>>>(p); break;
     default: qgemm_wide_kernel<256, 128, 4, 2, 3, 2, 4><<<count[3], 512, 0, stream>>>(p); break;
