@@ -225,12 +225,12 @@ __device__ __attribute__((always_inline)) inline half2_t split(float v) {
 // Writes a fetched stage into the stage-parity buffers (and, for Q4_K, its block's min-term
 // operands and scales into the block-parity ones; both stages of a block write the same values,
 // which are read only after the block's second barrier). The thread's token and row go to tile
-// row off + t / 4.
-template <QFormat F, class L = Lds>
-__device__ inline void store(const Fetch<F>& f, L& sm, unsigned s, unsigned t, bool tok_ok,
-                             bool row_ok, unsigned off = 0) {
+// row t / 4.
+template <QFormat F>
+__device__ inline void store(const Fetch<F>& f, Lds& sm, unsigned s, unsigned t, bool tok_ok,
+                             bool row_ok) {
   using q4k_gemv_detail::spread_bytes;
-  const unsigned tok = off + (t >> 2), q = t & 3u, buf = s & 1u;
+  const unsigned tok = t >> 2, q = t & 3u, buf = s & 1u;
   const u32x4 zero{0u, 0u, 0u, 0u};
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -853,7 +853,12 @@ __global__ void __launch_bounds__(64 * WM * WN, kWavesPerSimd) qgemm_wide_kernel
 // matrices in turn, with two stages and four: 2048 rows x 4096, 13 tokens 30.8 / 26.4 us, 512 tokens
 // 34.8 / 27.3; 8192 rows x 2048, 64 tokens 19.6 / 15.8; a whole layer over 512 tokens 125 / 118. Q6_K
 // waits for its weights' registers at every other stage, and stays with two: 512 rows x 2048 19.5 / 20.9.
-inline void qgemm_launch(const QGemmBatch& p, hipStream_t stream) {
+struct QGemmShape {
+  unsigned index;  // 0 .. 3: 64 x 64, 128 x 64, 128 x 128, 256 x 128
+  unsigned tiles;  // the launch's workgroups
+  bool deep;       // four stages in the ring (64 x 64)
+};
+inline QGemmShape qgemm_shape(const QGemmBatch& p) {
   auto tiles = [&](unsigned tok, unsigned row) {
     unsigned rows = 0;
     for (unsigned i = 0; i < p.count; ++i)
@@ -874,16 +879,21 @@ inline void qgemm_launch(const QGemmBatch& p, hipStream_t stream) {
     if (t < least)
       best = i, least = t;
   }
-  switch (best) {
+  return {best, count[best], best == 0 && count[0] <= 256 && p.format[0] == QFormat::Q4K};
+}
+
+inline void qgemm_launch(const QGemmBatch& p, hipStream_t stream) {
+  const QGemmShape s = qgemm_shape(p);
+  switch (s.index) {
     case 0:
-      if (count[0] <= 256 && p.format[0] == QFormat::Q4K)
-        qgemm_wide_kernel<64, 64, 2, 2, 4, 2, 4><<<count[0], 256, 0, stream>>>(p);
+      if (s.deep)
+        qgemm_wide_kernel<64, 64, 2, 2, 4, 2, 4><<<s.tiles, 256, 0, stream>>>(p);
       else
-        qgemm_wide_kernel<64, 64, 2, 2, 2, 2, 4><<<count[0], 256, 0, stream>>>(p);
+        qgemm_wide_kernel<64, 64, 2, 2, 2, 2, 4><<<s.tiles, 256, 0, stream>>>(p);
       break;
-    case 1: qgemm_wide_kernel<128, 64, 2, 2, 2, 2, 2><<<count[1], 256, 0, stream>>>(p); break;
-    case 2: qgemm_wide_kernel<128, 128, 2, 4, 2, 4, 2><<<count[2], 512, 0, stream>>>(p); break;
-    default: qgemm_wide_kernel<256, 128, 4, 2, 3, 2, 4><<<count[3], 512, 0, stream>>>(p); break;
+    case 1: qgemm_wide_kernel<128, 64, 2, 2, 2, 2, 2><<<s.tiles, 256, 0, stream>>>(p); break;
+    case 2: qgemm_wide_kernel<128, 128, 2, 4, 2, 4, 2><<<s.tiles, 512, 0, stream>>>(p); break;
+    default: qgemm_wide_kernel<256, 128, 4, 2, 3, 2, 4><<<s.tiles, 512, 0, stream>>>(p); break;
   }
 }
 

@@ -1,6 +1,7 @@
 // Test infrastructure: extern "C" launchers for what the product's own library does not launch: the
-// engine drop-in (miso_amd/engine/attention.{hpp,hip} against engine_stub/). Used only by GPU
-// tests; never linked into the product.
+// engine drop-in (miso_amd/engine/attention.{hpp,hip} against engine_stub/), the 64 x 64 GEMM kernel
+// that the engine's own gemm() launches, and GEMM batches of any mix. Used only by GPU tests; never
+// linked into the product.
 
 #include "engine/attention.hip"
 
@@ -87,6 +88,50 @@ std::uint64_t drop_engine_read(void* e_, const char* name, float* out, std::uint
       return m.b.size();
     }
   return 0;
+}
+
+// qgemm_kernel<F> as the engine launches it (src/engine/weights.hip:306-330); format 0 Q4_K, 1 Q6_K.
+int drop_qgemm_kernel(int format, const std::uint8_t* w, const void* xh, const float* xs, float* y,
+                      unsigned k, unsigned n_rows, unsigned n_tok, unsigned ldy) {
+  namespace K = miso::kernels;
+  const K::QGemmParams p{w, static_cast<const _Float16*>(xh), xs, y, k, n_rows, n_tok, ldy};
+  const unsigned tiles = K::qgemm_tiles(n_rows, n_tok);
+  if (format == 0)
+    K::qgemm_kernel<K::QFormat::Q4K><<<tiles, 256>>>(p);
+  else
+    K::qgemm_kernel<K::QFormat::Q6K><<<tiles, 256>>>(p);
+  return static_cast<int>(hipGetLastError());
+}
+
+namespace {
+miso::kernels::QGemmBatch batch(unsigned count, const int* format, const std::uint8_t* const* w,
+                                const void* xh, const float* xs, float* const* y, unsigned k,
+                                const unsigned* n_rows, unsigned n_tok, unsigned ldy) {
+  namespace K = miso::kernels;
+  K::QGemmBatch b{};
+  b.count = count;
+  for (unsigned i = 0; i < count; ++i) {
+    b.m[i] = {w ? w[i] : nullptr, static_cast<const _Float16*>(xh), xs, y ? y[i] : nullptr, k,
+              n_rows[i], n_tok, ldy};
+    b.format[i] = format[i] == 0 ? K::QFormat::Q4K : K::QFormat::Q6K;
+  }
+  return b;
+}
+}  // namespace
+
+// qgemm_launch of up to three products, and the tile shape it takes for them (10 + the shape's index
+// where the ring is deep; host only).
+int drop_qgemm_batch(unsigned count, const int* format, const std::uint8_t* const* w, const void* xh,
+                     const float* xs, float* const* y, unsigned k, const unsigned* n_rows,
+                     unsigned n_tok, unsigned ldy) {
+  miso::kernels::qgemm_launch(batch(count, format, w, xh, xs, y, k, n_rows, n_tok, ldy), nullptr);
+  return static_cast<int>(hipGetLastError());
+}
+unsigned drop_qgemm_shape(unsigned count, const int* format, const unsigned* n_rows,
+                          unsigned n_tok) {
+  const auto s = miso::kernels::qgemm_shape(
+      batch(count, format, nullptr, nullptr, nullptr, nullptr, 256, n_rows, n_tok, 0));
+  return s.index + (s.deep ? 10 : 0);
 }
 
 }  // extern "C"

@@ -11,8 +11,8 @@ Cases: the reference's fixture tensors (Q4_K K = 8192 N = 2, Q6_K K = 4096 N = 4
 tests/test_qgemm.hip:199-208), the attention's projections on random blocks (attn_q 2048 -> 8192,
 attn_k 2048 -> 512, attn_output 4096 -> 2048, attn_v Q6_K 2048 -> 512) with token counts that
 leave partial tiles, one token, a row stride ldy > n_rows with canaries past each row, and the
-Python layer's reference error messages. Q4_K's 128-token tiles equal its 64 x 64 tiles bit for
-bit.
+Python layer's reference error messages. Every tile shape that qgemm_launch takes, and the mixed
+q / k / v launch, equal the 64 x 64 kernel of the engine's own gemm() bit for bit.
 """
 from __future__ import annotations
 
@@ -150,11 +150,10 @@ def test_q6k_shapes(O, attn, torch_mod, k, n, n_tok):
 
 @pytest.mark.parametrize("k,n,n_tok", [(2048, 8192, 600), (2048, 2000, 2100), (4096, 2048, 2048)])
 def test_q4k_token_tiles_bit_identical(O, attn, torch_mod, k, n, n_tok):
-    """Q4_K runs 128 x 128 tiles (qgemm_q4k_big_kernel) when they give every CU one, as in every
-    case here (the last token tile partial in the first two, the last row tile in the second; the
-    third is attn_output's shape, k = 4096); at most 64 tokens always run 64 x 64 tiles
-    (qgemm_kernel). Each output element is the same arithmetic in the same order either way, so
-    the product equals, bit for bit, the same product computed 64 tokens at a time."""
+    """A product equals, bit for bit, the same product computed 64 tokens at a time (64 x 64 tiles, a
+    deep ring): whatever shape the whole takes (64 x 64 with the shallow ring for the first two, the
+    last token tile partial, the last row tile in the second; 128 x 128 for the third, attn_output's
+    shape), each output element is the same arithmetic in the same order."""
     torch = torch_mod
     rng = np.random.default_rng(k + n + n_tok)
     r1 = to_dev(torch, O.q4k_repack_r1(random_blocks(rng, n, k)))
@@ -206,10 +205,9 @@ def test_python_layer_reference_errors(attn, torch_mod):
 @pytest.mark.parametrize("k,n,n_tok", [(2048, 8192, 33), (2048, 2000, 700), (2048, 8100, 515),
                                        (4096, 2048, 4000), (2048, 9216, 1025), (256, 130, 260)])
 def test_wide_tiles_bit_identical(O, attn, torch_mod, k, n, n_tok):
-    """Every tile shape qgemm_launch picks (64 x 64, 128 x 64, 128 x 128, 256 x 128 here, the last
-    token and row tiles partial, and one block of k) against the 64 x 64 kernel's arithmetic: a
-    product of at most 64 tokens takes 64 x 64 tiles, so 64 tokens at a time give the same bits;
-    the first 64 also meet the reference test's bound."""
+    """A product of either format equals the same product computed 64 tokens at a time, bit for bit
+    (partial token and row tiles, one block of k); the first tokens also meet the reference test's
+    bound. Which shapes these are, and the 64 x 64 kernel: the tests below."""
     torch = torch_mod
     rng = np.random.default_rng(k + n + n_tok)
     for fmt in ("q4_k", "q6_k"):
@@ -222,3 +220,87 @@ def test_wide_tiles_bit_identical(O, attn, torch_mod, k, n, n_tok):
                                 for t in range(0, n_tok, 64)])
         assert np.array_equal(whole, parts), fmt
         check(O, attn, torch, fmt, blocks, n, k, x[:5], "wide")
+
+
+# The tile shapes of qgemm_launch (drop_qgemm_shape).
+S64, S64_DEEP, S128_64, S128, S256 = 0, 10, 1, 2, 3
+
+
+def shape_of(O, products, n_tok):
+    fmt = np.array([f for f, _ in products], np.int32)
+    rows = np.array([n for _, n in products], np.uint32)
+    return O.drop_in().drop_qgemm_shape(len(products), fmt.ctypes.data, rows.ctypes.data, n_tok)
+
+
+# Every shape with both formats, whole tiles and partial last token and row tiles, one block of k and
+# attn_output's k; few tokens in many row tiles.
+SHAPES = [("q4_k", 256, 130, 260, S64_DEEP), ("q4_k", 2048, 512, 1, S64_DEEP),
+          ("q4_k", 2048, 8100, 129, S128_64), ("q4_k", 4096, 2048, 512, S64_DEEP),
+          ("q4_k", 2048, 4096, 500, S128_64), ("q4_k", 2048, 8100, 500, S128),
+          ("q4_k", 4096, 2048, 2047, S128), ("q4_k", 2048, 8150, 1030, S64),
+          ("q4_k", 2048, 8150, 1000, S256), ("q4_k", 4096, 2048, 4000, S256),
+          ("q6_k", 256, 130, 260, S64), ("q6_k", 2048, 512, 2049, S128_64),
+          ("q6_k", 2048, 1000, 2000, S128_64), ("q6_k", 2048, 2000, 2050, S64),
+          ("q6_k", 2048, 2000, 1700, S128), ("q6_k", 512, 2040, 3900, S256)]
+
+
+@pytest.mark.parametrize("fmt,k,n,n_tok,shape", SHAPES)
+def test_every_tile_shape_equals_the_64x64_kernel(O, attn, torch_mod, fmt, k, n, n_tok, shape):
+    """Per output element every shape of qgemm_launch does qgemm_kernel's arithmetic in its order: the
+    same bits as that kernel (what the engine's own gemm() launches), which meets the reference
+    test's bound here too."""
+    torch = torch_mod
+    f = 0 if fmt == "q4_k" else 1
+    assert shape_of(O, [(f, n)], n_tok) == shape
+    rng = np.random.default_rng(k + n + n_tok)
+    blocks = random_blocks(rng, n, k) if f == 0 else random_q6k_blocks(rng, n, k)
+    r1 = to_dev(torch, O.q4k_repack_r1(blocks) if f == 0 else O.q6k_repack_r1(blocks, n, k))
+    x = xs_normal(rng, n_tok, k)
+    inp = attn.GemmInput(n_tok, k)
+    attn.gemm_input(to_dev(torch, x.reshape(-1)), k, n_tok, inp)
+    wide, small = (torch.full((n_tok * (n + 3),), CANARY, device="cuda") for _ in range(2))
+    attn.gemm(r1, fmt, n, k, inp, wide, n + 3)
+    torch.cuda.synchronize()
+    assert O.drop_in().drop_qgemm_kernel(f, r1.data_ptr(), inp.xh.data_ptr(), inp.xs.data_ptr(),
+                                         small.data_ptr(), k, n, n_tok, n + 3) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(wide, small)
+    got = small.view(n_tok, n + 3)
+    assert bool((got[:, n:] == CANARY).all()) and bool(torch.isfinite(got).all())
+    w, mag = magnitudes(O, fmt, blocks, n, k)
+    rows = np.unique(np.concatenate([[0, n_tok - 1], rng.choice(n_tok, min(n_tok, 5))]))
+    h = x[rows].astype(np.float16).astype(np.float64)
+    bound = (k / 16.0 + 80.0) * 2.0 ** -24 * (np.abs(h) @ mag.T) + 1e-30
+    err = np.abs(to_host(got)[rows, :n].astype(np.float64) - h @ w.T)
+    print(f"[qgemm shape {shape} {fmt}] max err/bound {(err / bound).max():.3f}", flush=True)
+    assert (err <= bound).all()
+
+
+@pytest.mark.parametrize("n_tok,shape", [(13, S64_DEEP), (100, S128_64), (400, S64), (700, S256),
+                                         (2049, S128)])
+def test_mixed_batch_equals_its_products(O, attn, torch_mod, n_tok, shape):
+    """The q / k / v launch (8192 Q4_K, 512 Q4_K, 512 Q6_K rows of 2048 into one buffer): the row tiles
+    of the second and third product are spread among the first's, and each comes out as by itself."""
+    torch = torch_mod
+    k, ldy = 2048, 9216
+    products = [(0, 8192), (0, 512), (1, 512)]
+    assert shape_of(O, products, n_tok) == shape
+    rng = np.random.default_rng(n_tok)
+    w = [to_dev(torch, O.q4k_repack_r1(random_blocks(rng, n, k)) if f == 0
+                else O.q6k_repack_r1(random_q6k_blocks(rng, n, k), n, k)) for f, n in products]
+    inp = attn.GemmInput(n_tok, k)
+    attn.gemm_input(to_dev(torch, xs_normal(rng, n_tok, k).reshape(-1)), k, n_tok, inp)
+    both, single = (torch.full((n_tok * ldy,), CANARY, device="cuda") for _ in range(2))
+    at = np.cumsum([0, 8192, 512])
+    fmt = np.array([f for f, _ in products], np.int32)
+    rows = np.array([n for _, n in products], np.uint32)
+    wp = np.array([t.data_ptr() for t in w], np.uint64)
+    yp = np.array([both.data_ptr() + 4 * int(a) for a in at], np.uint64)
+    torch.cuda.synchronize()
+    assert O.drop_in().drop_qgemm_batch(3, fmt.ctypes.data, wp.ctypes.data, inp.xh.data_ptr(),
+                                        inp.xs.data_ptr(), yp.ctypes.data, k, rows.ctypes.data,
+                                        n_tok, ldy) == 0
+    for (f, n), t, a in zip(products, w, at):
+        attn.gemm(t, ("q4_k", "q6_k")[f], n, k, inp, single[int(a):], ldy)
+    torch.cuda.synchronize()
+    assert torch.equal(both, single) and not bool((both == CANARY).any())
