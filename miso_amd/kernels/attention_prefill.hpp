@@ -1501,15 +1501,9 @@ __global__ void __launch_bounds__(256) attn_prefill_merge_kernel(AttnPrefillPart
   }
 }
 
-// Launches the prefill in parts where it pays and the workspace (attn_prefill_parts_workspace_bytes)
-// holds its partials; false if neither kernel was launched.
-inline bool attn_prefill_in_parts(const AttnPrefillParams& a, void* workspace, std::size_t bytes,
+// Launches the prefill in parts of `row_blocks` row blocks per wave.
+inline void attn_prefill_in_parts(const AttnPrefillParams& a, unsigned row_blocks, void* workspace,
                                   hipStream_t stream) {
-  const unsigned row_blocks = attn_prefill_parts_row_blocks(a.pos0, a.n);
-  if (row_blocks == 0)
-    return false;
-  if (bytes < kAttnSplitCounterBytes + attn_prefill_parts_bytes(a.n, row_blocks))
-    return false;
   AttnPrefillPartsParams p{a, nullptr, nullptr,
                            attn_prefill_cuts(a.pos0, a.n, row_blocks, kAttnPartsMaxWorkers)};
   p.part_ml =
@@ -1531,7 +1525,6 @@ inline bool attn_prefill_in_parts(const AttnPrefillParams& a, void* workspace, s
     else
       attn_prefill_merge_kernel<1, false><<<rows, 256, 0, stream>>>(p);
   }
-  return true;
 }
 
 // Largest launch that one workgroup per block runs faster than balanced pairs: with few blocks the
@@ -1541,14 +1534,26 @@ inline bool attn_prefill_in_parts(const AttnPrefillParams& a, void* workspace, s
 // 0 30.8 / 29.8, 720 after 64 32.5 / 31.3, 1024 after 0 39.3 / 34.9.
 constexpr unsigned kAttnPairsMinTokens = 640;
 
-// The causal prefill with a workspace: in parts, in balanced pairs, or one workgroup per block,
-// whichever the launch's size asks for. The workspace holds the balanced form's where
-// attn_prefill_balanced(n) (the caller checks); a larger one also lets the launch run in parts.
+// The form of a causal prefill with a workspace of `bytes`: in parts where they pay and the workspace
+// holds their partials, in balanced pairs, or one workgroup per block. The workspace holds the
+// balanced form's where attn_prefill_balanced(n) (the caller checks).
+enum class AttnPrefillForm : unsigned { Plain, Pairs, Parts, WideParts };
+inline AttnPrefillForm attn_prefill_form(unsigned pos0, unsigned n, std::size_t bytes) {
+  const unsigned row_blocks = attn_prefill_parts_row_blocks(pos0, n);
+  if (row_blocks != 0 && bytes >= kAttnSplitCounterBytes + attn_prefill_parts_bytes(n, row_blocks))
+    return row_blocks == 2 ? AttnPrefillForm::WideParts : AttnPrefillForm::Parts;
+  return attn_prefill_balanced(n) && n > kAttnPairsMinTokens ? AttnPrefillForm::Pairs
+                                                             : AttnPrefillForm::Plain;
+}
+
 inline void attn_prefill_launch(const AttnPrefillParams& a, void* workspace, std::size_t bytes,
                                 hipStream_t stream) {
-  if (attn_prefill_in_parts(a, workspace, bytes, stream))
+  const AttnPrefillForm form = attn_prefill_form(a.pos0, a.n, bytes);
+  if (form == AttnPrefillForm::Parts || form == AttnPrefillForm::WideParts) {
+    attn_prefill_in_parts(a, form == AttnPrefillForm::WideParts ? 2 : 1, workspace, stream);
     return;
-  if (!attn_prefill_balanced(a.n) || a.n <= kAttnPairsMinTokens) {
+  }
+  if (form == AttnPrefillForm::Plain) {
     attn_prefill_kernel<256><<<attn_prefill_items(a.n), 256, 0, stream>>>(a);
     return;
   }

@@ -1,6 +1,6 @@
 // Test infrastructure: extern "C" launchers for what the product's own library does not launch: the
 // engine drop-in (miso_amd/engine/attention.{hpp,hip} against engine_stub/), the 64 x 64 GEMM kernel
-// that the engine's own gemm() launches, and GEMM batches of any mix. Used only by GPU tests; never
+// that the engine's own gemm() launches, GEMM batches of any mix, and the host's choices of a form. Used only by GPU tests; never
 // linked into the product.
 
 #include "engine/attention.hip"
@@ -132,6 +132,12 @@ unsigned drop_qgemm_shape(unsigned count, const int* format, const unsigned* n_r
   const auto s = miso::kernels::qgemm_shape(
       batch(count, format, nullptr, nullptr, nullptr, nullptr, 256, n_rows, n_tok, 0));
   return s.index + (s.deep ? 10 : 0);
+}
+
+// The form a causal prefill takes: 0 one workgroup per block, 1 balanced pairs, 2 parts, 3 parts with
+// two row blocks (host only).
+unsigned drop_prefill_form(unsigned pos0, unsigned n, std::uint64_t workspace_bytes) {
+  return static_cast<unsigned>(miso::kernels::attn_prefill_form(pos0, n, workspace_bytes));
 }
 
 }  // extern "C"

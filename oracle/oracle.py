@@ -519,6 +519,7 @@ def drop_in():
             "drop_engine_delete": (None, [V]),
             "drop_engine_step": (c_int, [V, c_int, V, V, V, U, c_float]),
             "drop_engine_read": (c_uint64, [V, ctypes.c_char_p, V, c_uint64]),
+            "drop_prefill_form": (U, [U, U, c_uint64]),
             "drop_qgemm_kernel": (c_int, [c_int, V, V, V, V, U, U, U, U]),
             "drop_qgemm_batch": (c_int, [U, V, V, V, V, V, U, V, U, U]),
             "drop_qgemm_shape": (U, [U, V, V, U]),

@@ -144,8 +144,8 @@ def test_layer_rejections(attn, torch_mod, layer_case):
 
 
 def test_layer_prefill_balanced_chunk(O, attn, torch_mod, layer_case):
-    """One 512-token chunk on an empty cache: the layer's prefill takes the balanced form with
-    split token blocks (chunks of up to 2048 tokens), against the layer oracle."""
+    """One 512-token chunk on an empty cache against the layer oracle (one workgroup per token block;
+    balanced pairs and parts below), and the same chunk again over the same workspace."""
     torch = torch_mod
     layer, deq, norms = layer_case
     n = ctx = 512
@@ -168,9 +168,53 @@ def test_layer_prefill_balanced_chunk(O, attn, torch_mod, layer_case):
                                  norms["inv_freq"], 0, ctx, EPS)
     got = first.reshape(n, 2048).astype(np.float64)
     err = np.sqrt(((got - ref_y) ** 2).sum(axis=1) / (ref_y ** 2).sum(axis=1))
-    print(f"[layer] 512-token balanced chunk: max rel-L2 {err.max():.2e}", flush=True)
+    print(f"[layer] 512-token chunk: max rel-L2 {err.max():.2e}", flush=True)
     assert np.isfinite(got).all()
     assert err.max() <= 5e-3, int(err.argmax())
+
+
+@pytest.mark.parametrize("pos0,n,form", [(0, 700, 1), (1536, 512, 2)])
+def test_layer_prefill_forms(O, attn, torch_mod, layer_case, monkeypatch, pos0, n, form):
+    """The layer's causal prefill in balanced pairs and in parts (drop_prefill_form), whose gates lie
+    9216 floats apart, against the layer oracle: over a workspace whose memory held NaNs before it was
+    made (only the pair counters are cleared), twice, the second time bit for bit the first."""
+    torch = torch_mod
+    layer, deq, norms = layer_case
+    ctx = pos0 + n
+    empty = torch.empty
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", lambda *a, **kw: empty(*a, **kw).fill_(float("nan")))
+        ws = attn.LayerWorkspace(max_tok=n)
+    lib = attn._lib.load()
+    workspace = 4 * (lib.miso_attn_layer_prefill_ws(n) - lib.miso_attn_layer_prefill_counters(n))
+    assert O.drop_in().drop_prefill_form(pos0, n, workspace) == form
+    rng = np.random.default_rng(n)
+    h0 = rng.standard_normal((n, 2048)).astype(np.float32)
+    delta = (0.5 * rng.standard_normal((n, 2048))).astype(np.float32)
+    k16, v16 = (rng.standard_normal((2, ctx, 256)).astype(np.float16) for _ in range(2))
+    out = []
+    for _ in range(2):
+        kc, vc = (torch.from_numpy(t).cuda().reshape(-1) for t in (k16, v16))
+        h, y = to_dev(torch, h0.reshape(-1)), torch.zeros(n * 2048, device="cuda")
+        attn.layer_prefill(layer, kc, vc, ctx, pos0, n, h, to_dev(torch, delta.reshape(-1)), y, EPS,
+                           ws)
+        out.append((to_host(y), to_host(kc), to_host(vc), to_host(ws.prefill_core)))
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+    _, ref_y, k_ref, v_ref, ref_core = O.layer_f64(
+        h0, delta, deq["q"], deq["k"], deq["v"], deq["o"], norms["attn_norm"], norms["q_norm"],
+        norms["k_norm"], norms["inv_freq"], pos0, ctx, EPS, k16=k16.view(np.uint16).copy(),
+        v16=v16.view(np.uint16).copy(), with_core=True)
+    y, kc, vc, core = out[0]
+    for got, ref, what in ((y.reshape(n, 2048), ref_y, "y"), (core, ref_core, "core")):
+        err = np.sqrt(((got - ref) ** 2).sum(axis=1) / (ref ** 2).sum(axis=1))
+        print(f"[layer] pos0 {pos0} n {n} {what} max rel-L2 {err.max():.2e}", flush=True)
+        assert np.isfinite(got).all() and err.max() <= 5e-3, what
+    for got, ref in ((kc, k_ref), (vc, v_ref)):
+        got = got.reshape(2, ctx, 256)
+        assert np.array_equal(got[:, :pos0], ref[:, :pos0])
+        g, r = (O.f16_to_f32(t[:, pos0:]).astype(np.float64) for t in (got, ref))
+        ulp = np.spacing(np.abs(r).astype(np.float16)).astype(np.float64)
+        assert (np.abs(g - r) <= ulp + 1e-4 * np.abs(r).max(axis=2, keepdims=True)).all()
 
 
 def test_layer_core_after_each_call(O, attn, torch_mod, layer_case):

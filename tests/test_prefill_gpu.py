@@ -7,9 +7,8 @@ configs C3 (2048 tokens, empty cache; every row) and C4 (8192 tokens after an 81
 a deterministic row sample covering first/last tiles and diagonal tiles), plus two size-free
 properties: chunked prefill equals one-shot prefill, and prefill row t equals decode at pos0+t+1.
 The balanced form (miso_attn_prefill_ws: heavy token blocks split between two workgroups, the
-parts merged through a workspace; 16-token blocks up to 2048 tokens, 32-token blocks from 3841
-to 4096)
-is checked the same way, on shapes with and without split blocks, plus run-to-run bit equality
+parts merged through a workspace; 16-token blocks from 641 to 2048 tokens, 32-token blocks from 3841
+to 4096) and the parts (few tokens after a prefix) are checked the same way, on shapes with and without split blocks, plus run-to-run bit equality
 and reuse of one workspace across sizes.
 Gate: |got - ref| <= 2e-3 + 1e-2 |ref| for every element (f32 output).
 """
@@ -114,6 +113,19 @@ def test_prefill_engine_stride(O, attn, torch_mod):
     assert st["ok"], st
 
 
+@pytest.mark.parametrize("pos0,n,want", [(1536, 512, 2), (33000, 471, 3), (0, 700, 1)])
+def test_prefill_engine_stride_with_workspace(O, attn, torch_mod, prefill_scratch, pos0, n, want):
+    """The same stride in parts, whose merge reads the gates, and in balanced pairs."""
+    assert form(O, prefill_scratch, pos0, n) == want
+    p = O.prefill_inputs(n, pos0, n, pos0 + n, q_scale=2.0, qg_stride=9216)
+    got = run_prefill(attn, torch_mod, p, scratch=prefill_scratch)
+    rows = np.unique(np.concatenate([np.arange(0, n, 37), np.arange(n - 17, n)]))
+    st = O.compare(got[rows], O.prefill_f64(p["q"], p["qg"], 9216, p["k"], p["v"], pos0, pos0 + n,
+                                            rows))
+    report(f"engine stride pos0={pos0} n={n}", st)
+    assert st["ok"], st
+
+
 def test_reference_prefill_kernel_agrees_with_oracle(O, attn, torch_mod, ref_kernels):
     """Second checker: the reference's own prefill kernel (built from its sources) reproduces
     the oracle within the reference's rel-L2 gate of 1e-5 (test_attn_splitk.hip:267)."""
@@ -142,6 +154,14 @@ def prefill_scratch(attn, torch_mod):
     return attn.PrefillScratch()
 
 
+PLAIN, PAIRS, IN_PARTS, WIDE_PARTS = range(4)
+
+
+def form(O, scratch, pos0, n):
+    """The form a launch takes with this workspace (attn_prefill_form)."""
+    return O.drop_in().drop_prefill_form(pos0, n, scratch.nbytes)
+
+
 def balanced_rows(pos0, n):
     """Every row up to 1200 tokens; else the first and last rows of every 64th block, the last
     128 rows (the heaviest blocks, split) and a seeded sample."""
@@ -157,7 +177,19 @@ def balanced_rows(pos0, n):
                                     (7, 999), (100, 1500), (3000, 600), (1, 2047), (0, 2049),
                                     (0, 3841), (500, 4000), (0, 4096), (4096, 4096)])
 def test_prefill_balanced_matches_oracle(O, attn, torch_mod, prefill_scratch, pos0, n):
+    """The call with a workspace, whatever form it takes: one workgroup per block up to 640 tokens and
+    at 2049, parts (3000, 600), balanced pairs the others."""
+    want = IN_PARTS if (pos0, n) == (3000, 600) else PAIRS if n > 640 and n != 2049 else PLAIN
+    assert form(O, prefill_scratch, pos0, n) == want
     check(O, attn, torch_mod, pos0, n, rows=balanced_rows(pos0, n), name="balanced",
+          scratch=prefill_scratch)
+
+
+@pytest.mark.parametrize("pos0,n", [(0, 641), (0, 657), (33, 720), (0, 1009), (64, 1025)])
+def test_prefill_pairs_match_oracle(O, attn, torch_mod, prefill_scratch, pos0, n):
+    """The smallest balanced launches: odd and even block counts, a ragged last block."""
+    assert form(O, prefill_scratch, pos0, n) == PAIRS
+    check(O, attn, torch_mod, pos0, n, rows=balanced_rows(pos0, n), name="pairs",
           scratch=prefill_scratch)
 
 
@@ -174,7 +206,8 @@ def test_prefill_balanced_repeatable(O, attn, torch_mod, prefill_scratch):
     torch = torch_mod
     p = O.prefill_inputs(777, 0, 2048, 2048, q_scale=1.0)
     first = run_prefill(attn, torch, p, scratch=prefill_scratch)
-    small = O.prefill_inputs(778, 40, 333, 400, q_scale=2.0)
+    small = O.prefill_inputs(778, 40, 777, 900, q_scale=2.0)
+    assert [form(O, prefill_scratch, *x) for x in ((0, 2048), (40, 777), (0, 4096))] == [PAIRS] * 3
     a = run_prefill(attn, torch, small, scratch=prefill_scratch)
     wide = O.prefill_inputs(779, 0, 4096, 4096, q_scale=1.0)
     w = run_prefill(attn, torch, wide, scratch=prefill_scratch)
@@ -214,6 +247,7 @@ def test_prefill_parts_match_oracle(O, attn, torch_mod, prefill_scratch, pos0, n
     rng = np.random.default_rng(n + pos0)
     rows = np.unique(np.concatenate([np.arange(min(n, 17)), np.arange(max(0, n - 33), n),
                                      rng.choice(n, min(n, 24), replace=False)]))
+    assert form(O, prefill_scratch, pos0, n) == (WIDE_PARTS if pos0 == 33000 else IN_PARTS)
     check(O, attn, torch_mod, pos0, n, rows=rows, name="parts", scratch=prefill_scratch)
     p = O.prefill_inputs(n, pos0, n, pos0 + n + 3, q_scale=2.0)
     first = run_prefill(attn, torch_mod, p, scratch=prefill_scratch)
@@ -226,20 +260,24 @@ def test_prefill_parts_match_oracle(O, attn, torch_mod, prefill_scratch, pos0, n
 
 
 def test_prefill_parts_small_workspace(O, attn, torch_mod):
-    """A workspace of the balanced form's size keeps the balanced form (bitwise the result of a
-    launch that never knew parts), and a launch outside both takes no workspace at all."""
+    """A workspace of the balanced form's size keeps the form that launch has without parts (one
+    workgroup per block for 203 tokens, bit for bit; balanced pairs for 700), and a launch outside
+    both takes no workspace at all."""
     torch = torch_mod
-    p = O.prefill_inputs(203, 2000, 203, 2203, q_scale=2.0)
-    small = attn.PrefillScratch(203)
-    need = attn.prefill_workspace_bytes(203)
-    assert small.nbytes > need
-    parts = run_prefill(attn, torch, p, scratch=small)
-    small.nbytes = need
-    pairs = run_prefill(attn, torch, p, scratch=small)
-    assert np.array_equal(run_prefill(attn, torch, p, scratch=small), pairs)
-    assert not np.array_equal(parts, pairs)
-    st = O.compare(parts, pairs.astype(np.float64))
-    assert st["ok"], st
+    for n, pos0, other in ((203, 2000, PLAIN), (700, 4099, PAIRS)):
+        p = O.prefill_inputs(n, pos0, n, pos0 + n, q_scale=2.0)
+        small = attn.PrefillScratch(n)
+        need = attn.prefill_workspace_bytes(n)
+        assert small.nbytes > need and form(O, small, pos0, n) == IN_PARTS
+        parts = run_prefill(attn, torch, p, scratch=small)
+        small.nbytes = need
+        assert form(O, small, pos0, n) == other
+        rest = run_prefill(attn, torch, p, scratch=small)
+        assert np.array_equal(run_prefill(attn, torch, p, scratch=small), rest)
+        assert np.array_equal(rest, run_prefill(attn, torch, p)) == (other == PLAIN)
+        assert not np.array_equal(parts, rest)
+        st = O.compare(parts, rest.astype(np.float64))
+        assert st["ok"], st
     wide = O.prefill_inputs(2100, 3000, 2100, 5100, q_scale=2.0)
     small.nbytes = 0
     assert np.array_equal(run_prefill(attn, torch, wide, scratch=small),
