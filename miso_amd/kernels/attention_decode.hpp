@@ -1003,8 +1003,6 @@ __device__ __attribute__((always_inline)) inline void prepare_queries(const Prep
   for (unsigned i = 0; i < 2; ++i) {
     float4* at = reinterpret_cast<float4*>(&q[2 * wave + i][4 * lane]);
     *at = prep_row(*at, w, qs.eps, rope, lane);
-    if (qs.q_out != nullptr)  // uniform
-      *reinterpret_cast<float4*>(qs.q_out + (2 * wave + i) * attn::kDim + 4 * lane) = *at;
   }
   if (owner) {  // uniform
     const float4 k = prep_row(*reinterpret_cast<const float4*>(&qs.sh->token[0][4 * lane]),
@@ -1032,6 +1030,20 @@ __device__ __attribute__((always_inline)) inline void store_token(const PrepQuer
                                                                  unsigned lane) {
   *reinterpret_cast<cdna4::half4_t*>(qs.k_row + 4 * lane) = row.k;
   *reinterpret_cast<cdna4::half4_t*>(qs.v_row + 4 * lane) = row.v;
+}
+
+// This wave's prepared query rows to q_out, once the split is done (a store among the tile copies
+// would be waited for with them).
+__device__ __attribute__((always_inline)) inline void store_queries(const float*, float (*)[256],
+                                                                   unsigned, unsigned) {}
+__device__ __attribute__((always_inline)) inline void store_queries(const PrepQuery& qs,
+                                                                   float (*q)[256], unsigned wave,
+                                                                   unsigned lane) {
+  if (qs.q_out != nullptr)  // uniform
+#pragma unroll
+    for (unsigned i = 0; i < 2; ++i)
+      *reinterpret_cast<float4*>(qs.q_out + (2 * wave + i) * attn::kDim + 4 * lane) =
+          *reinterpret_cast<const float4*>(&q[2 * wave + i][4 * lane]);
 }
 
 // Where the rows of a split lie, for the tile copies: k_at(row) / v_at(row) is the address of K /
@@ -1504,6 +1516,7 @@ __device__ __attribute__((always_inline)) inline void split_partial_tiles(
 
   if (kPrep && owner)
     store_token(q, token, lane);
+  store_queries(q, sh.q, wave, lane);
   // Relative to the true max; l summed over the lanes g of the column; the (hi, lo) columns of
   // O joined in the lanes c < 8, which store this wave's 64 dimensions of head c.
   const bool empty = n_tiles == 0;
@@ -1970,6 +1983,7 @@ __device__ __attribute__((always_inline)) inline void split_partial_waves(
 
   if (kPrep && owner)
     store_token(q, token, lane);
+  store_queries(q, sh.q, wave, lane);
   // The merge through the K slots: wave w's result in its own slot (O in the first 8 KiB, mt and
   // l after it), which only it has used.
   {

@@ -62,7 +62,7 @@ __global__ void __launch_bounds__(kBlock) qkv_gemv_kernel(Q4kGemvParams q, Q4kGe
 // The decode step's input in one launch: qkv_gemv_kernel on the residual row itself. Every workgroup
 // forms RMSNorm(h + delta) weight while its weights are in flight (24 KiB of rows from L2 and one
 // barrier more) instead of waiting for a launch that wrote it: 7.0 us against 2.1 + 5.8 us in two
-// launches. h itself is not updated here (every workgroup reads it); the first workgroup stores the
+// launches. h itself is not updated here (every workgroup reads it); the first one of k stores the
 // normed row in xn. The last workgroup tabulates the token's rotation: rope[i], rope[32 + i] = cos,
 // sin of pos inv_freq[i].
 struct QkvNormParams {
@@ -97,7 +97,7 @@ __global__ void __launch_bounds__(256) qkv_norm_gemv_kernel(Q4kGemvParams q, Q4k
     }
     return;
   }
-  const q4k_gemv_detail::NormX src{n.h, n.delta, n.weight, rest, b == 0 ? n.xn : nullptr, n.eps};
+  const q4k_gemv_detail::NormX src{n.h, n.delta, n.weight, rest, b == kVGrid ? n.xn : nullptr, n.eps};
   if (b < kVGrid) {
     q6k_gemv_detail::q6k_gemv_rows<K, 256, 1>(v, src, 0, v.n_rows, b, kVGrid, slabs, x_lds);
   } else {
