@@ -2657,12 +2657,14 @@ static_assert(sizeof(StreamLists) <= sizeof(StreamShared::merge), "the lists in 
 // longest span's tiles and about 3 more (query rows, merge). The m <= 4 with the least m (R + 3), and
 // from that estimate the first R whose spans fit m G. batch <= 2 G, so enough spans fit. The 512-key
 // spans stay where others would only add partials to merge:
-//   - they run in one round of at least 10 tiles per CU, when the memory sets the pace whatever the
-//     span (6 of 3532 .. 9803 keys);
+//   - they run in one round of more than 8 tiles per CU, when the memory sets the pace whatever the
+//     span (caches that come from memory, as the next layer's do: 2 of 18718 .. 21618 keys 23.3 us
+//     against 24.6 in 160 spans of 10 tiles, 5 of 5946 .. 7916 22.0 / 22.2; below 8 9 of 3244 .. 3654
+//     21.7 / 20.5);
 //   - others give a wave no fewer tiles in no fewer rounds (57 sequences of 782 .. 3217 keys);
-//   - others cost no less at 5 tiles a span beside its own (its partials are merged too), counted
-//     with the tiles the 512-key spans have: the longest's in one round, in more the middle of the
-//     longest's and the mean. 100 sequences of 300 keys, one round of 10 tiles: 25.4 us against 32.9
+//   - others cost no less at 7 tiles a span beside its own (its partials are merged too), counted
+//     with the tiles the spans have: the longest's in one round, in more the middle of the longest's
+//     and the mean. 100 sequences of 300 keys, one round of 10 tiles: 25.4 us against 32.9
 //     in two of 5; 238 of 23 .. 447: 51.7 against 54.5.
 // The choice stands before a workgroup's first load and one wave makes it, so its time is its
 // instruction count: quotients of counts by v_rcp_f32 (exact below 2^20: (a + 0.5) / b is at least
@@ -2699,7 +2701,7 @@ __device__ __attribute__((always_inline)) inline unsigned ragged_balanced_tiles(
   const float plain = spans(kP), rounds = ceil_quotient(plain, g);
   // More items than a workgroup's list holds: lengths beyond the caller's max_len.
   const bool may_stay = rounds <= static_cast<float>(kRaggedStreamMaxItems);
-  if (plain <= g && all >= 10.0f * g)  // uniform, as every branch below
+  if (plain <= g && all >= 8.25f * g)  // uniform, as every branch below
     return kPlain;
   float m = 0.0f, least = 0.0f, R = 0.0f;
 #pragma unroll
@@ -2717,20 +2719,24 @@ __device__ __attribute__((always_inline)) inline unsigned ragged_balanced_tiles(
   for (; R < 0x1p24f; R += __builtin_floorf(R * 0.03125f) + 1.0f) {
     if (may_stay && rounds <= m && R > kP - kW && R <= kP)
       return kPlain;
-    if (may_stay && rounds * (mean + 5.0f) <= m * (R + 8.0f)) {
-      float top = 0.0f, longest = 0.0f;
+    // Neither rule below can hold for spans of R tiles where it does not for the mean of the others.
+    if (may_stay && (rounds * (mean + 7.0f) <= m * (R + 7.0f) ||
+                     (rounds <= m && ceil_quotient(R, kW) >= ceil_quotient(mean, kW)))) {
+      float top = 0.0f, other = 0.0f;
+      auto longest = [&](float t, float span) __attribute__((always_inline)) {  // of t tiles' spans
+        return ceil_quotient(t, fmaxf(fminf(ceil_quotient(t, span), s_max), 1.0f));
+      };
 #pragma unroll
       for (unsigned i = 0; i < kStreamSeqsPerLane; ++i) {
         if (cdna4::kLanes * i >= p.batch)  // uniform
           break;
-        const float k = fminf(ceil_quotient(tiles[i], kP), s_max);
-        top = fmaxf(top, ceil_quotient(tiles[i], fmaxf(k, 1.0f)));
-        longest = fmaxf(longest, tiles[i]);
+        top = fmaxf(top, longest(tiles[i], kP));
+        other = fmaxf(other, longest(tiles[i], R));
       }
       top = cdna4::wave_allmax(top);
-      const float other = fminf(R, cdna4::wave_allmax(longest));
+      other = cdna4::wave_allmax(other);
       const float span = plain <= g ? top : 0.5f * (top + mean);
-      if (rounds * (span + 5.0f) <= m * (other + 5.0f) ||
+      if (rounds * (span + 7.0f) <= m * (other + 7.0f) ||
           (rounds <= m && ceil_quotient(other, kW) >= ceil_quotient(top, kW)))
         return kPlain;
     }

@@ -163,14 +163,15 @@ def test_ragged_balanced_spans(O, attn, torch_mod, lens, max_len):
     ([512] * 243, True),  # 486 spans in two rounds; halves would take four
     ([3217, 782] * 28, True),  # 15 tiles a span, four per wave as of 16
     ([4096] * 24, False),  # two rounds of 512 keys, one of 26 tiles
-    ([8192] * 5, True), ([8192] * 4 + [8160], False),  # one round of 10 tiles per CU, and less
+    ([8192] * 5, True), ([8192] * 4 + [2080], True),  # one round of 10 and of 8.5 tiles per CU
+    ([8192] * 4, False),  # one round of 8
     ([300] * 100, True),  # one round of 10 tiles; two of 5 cost more
     ([23, 447] * 119, True), ([1240] * 102, False),  # two rounds of 14 at most; two of 20 for three
 ])
 def test_ragged_balanced_keeps_512_key_spans(O, attn, torch_mod, lens, kept):
     """On 256 CUs: spans of 512 keys stay where they are estimated no slower (counted with the tiles
-    they really have), where others would give a wave as many tiles, and in one round of 10 tiles
-    per CU (bitwise the call with scratch for those only); any others are balanced."""
+    they really have), where others would give a wave as many tiles, and in one round of more than
+    8 tiles per CU (bitwise the call with scratch for those only); any others are balanced."""
     torch = torch_mod
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the sizes are those of 256 CUs")
