@@ -418,7 +418,7 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const QGemmParam
 // (or two waves per SIMD in the 256 x 128 tile) let one's expansion and barrier run beside the
 // other's MFMAs. Measured, Q4_K, before and after on one box: 8192 rows x 2048, 4096 tokens 354 ->
 // 196 us (389 -> 702 TFLOP/s), 2048 x 4096, 4096 tokens 158 -> 85 us (435 -> 804); matrix units
-// 40% busy, VALU 36%, LDS 32% (256 x 128): what is left is the lock step of one barrier per stage.
+// 40% busy, VALU 38%, LDS 32% (256 x 128): what is left is the lock step of one barrier per stage.
 //
 // Stage s: the MFMAs read activations and expanded weights of stage s while the same threads
 // expand stage s + 1 into the other weight buffer. kRing 3 keeps two stages of activations in
