@@ -186,6 +186,9 @@ int miso_attn_prefill(const float* q, const float* qg, const uint16_t* k_cache,
  * the faster one there (the workspace is checked all the same). */
 uint64_t miso_attn_prefill_workspace_bytes(uint32_t n);
 uint64_t miso_attn_prefill_parts_workspace_bytes(uint32_t max_n);
+/* The workspace with which n tokens after pos0 take the fastest form; 0 where that is
+ * miso_attn_prefill's (which those may call instead: the same result, no workspace). */
+uint64_t miso_attn_prefill_launch_bytes(uint32_t pos0, uint32_t n);
 int miso_attn_prefill_ws(const float* q, const float* qg, const uint16_t* k_cache,
                          const uint16_t* v_cache, float* core, uint32_t pos0, uint32_t n,
                          uint32_t max_ctx, uint32_t qg_stride, void* workspace,

@@ -33,6 +33,7 @@ SIGNATURES = {
     "miso_attn_prefill": (c_int, [P, P, P, P, P, c_uint32, c_uint32, c_uint32, c_uint32, P]),
     "miso_attn_prefill_workspace_bytes": (c_uint64, [c_uint32]),
     "miso_attn_prefill_parts_workspace_bytes": (c_uint64, [c_uint32]),
+    "miso_attn_prefill_launch_bytes": (c_uint64, [c_uint32, c_uint32]),
     "miso_attn_prefill_ws": (c_int, [P, P, P, P, P, c_uint32, c_uint32, c_uint32, c_uint32, P,
                                      c_uint64, P]),
     "miso_attn_ragged_splits": (c_uint32, [c_uint32]),

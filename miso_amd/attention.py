@@ -373,13 +373,14 @@ def attn_prep_batch_fp8(qg, k, v, q_norm, k_norm, inv_freq, cache: Fp8Cache, q, 
 
 class Fp8PrefillScratch:
     """f16 workspaces for attn_prefill_fp8 over up to max_rows cache rows (pos0 + n), and the
-    prefill's own workspace for as many tokens (PrefillScratch)."""
+    prefill's own workspace for as many tokens (PrefillScratch; with `lazy`, made by the first call
+    that uses it)."""
 
-    def __init__(self, max_rows: int, device="cuda"):
+    def __init__(self, max_rows: int, device="cuda", lazy: bool = False):
         self.max_rows = max_rows
         self.k = torch.empty(KV_HEADS * max_rows * DIM, dtype=torch.float16, device=device)
         self.v = torch.empty(KV_HEADS * max_rows * DIM, dtype=torch.float16, device=device)
-        self.prefill = PrefillScratch(max_rows, device)
+        self.prefill = None if lazy else PrefillScratch(max_rows, device)
 
 
 def attn_prefill_fp8(q, qg, cache: Fp8Cache, core, pos0: int, n: int,
@@ -388,7 +389,7 @@ def attn_prefill_fp8(q, qg, cache: Fp8Cache, core, pos0: int, n: int,
     """attn_prefill over an e4m3 cache: rows [0, pos0 + n) widened to f16 into `scratch` (made
     here when None), then the f16 causal prefill over them. Returns the scratch used."""
     if scratch is None:
-        scratch = Fp8PrefillScratch(pos0 + n, device=q.device)
+        scratch = Fp8PrefillScratch(pos0 + n, device=q.device, lazy=True)
     if pos0 + n > scratch.max_rows:
         raise ValueError("pos0 + n exceeds the scratch capacity")
     f32 = torch.float32
@@ -396,10 +397,16 @@ def attn_prefill_fp8(q, qg, cache: Fp8Cache, core, pos0: int, n: int,
     _need(qg, "qg", f32, (n - 1) * qg_stride + Q_HEADS * 2 * DIM if n else 0)
     _need(core, "core", f32, n * Q_HEADS * DIM)
     _need_fp8(cache)
-    _lib.check(_lib.load().miso_attn_prefill_fp8_ws(
-        _ptr(q), _ptr(qg), *(_ptr(b) for b in cache.buffers()), _ptr(scratch.k), _ptr(scratch.v),
-        _ptr(core), pos0, n, cache.max_ctx, qg_stride, _ptr(scratch.prefill.buf),
-        scratch.prefill.nbytes, _stream(stream)))
+    lib = _lib.load()
+    args = (_ptr(q), _ptr(qg), *(_ptr(b) for b in cache.buffers()), _ptr(scratch.k),
+            _ptr(scratch.v), _ptr(core), pos0, n, cache.max_ctx, qg_stride)
+    if scratch.prefill is None:
+        if lib.miso_attn_prefill_launch_bytes(pos0, n) == 0:
+            _lib.check(lib.miso_attn_prefill_fp8(*args, _stream(stream)))
+            return scratch
+        scratch.prefill = PrefillScratch(scratch.max_rows, q.device)
+    _lib.check(lib.miso_attn_prefill_fp8_ws(*args, _ptr(scratch.prefill.buf),
+                                            scratch.prefill.nbytes, _stream(stream)))
     return scratch
 
 

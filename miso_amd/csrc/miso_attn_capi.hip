@@ -379,6 +379,17 @@ uint64_t miso_attn_prefill_parts_workspace_bytes(uint32_t max_n) {
   return k::attn_prefill_parts_workspace_bytes(max_n);
 }
 
+uint64_t miso_attn_prefill_launch_bytes(uint32_t pos0, uint32_t n) {
+  switch (k::attn_prefill_form(pos0, n, ~std::size_t{0})) {
+    case k::AttnPrefillForm::Plain: return 0;
+    case k::AttnPrefillForm::Pairs: return k::attn_prefill_split_workspace_bytes(n);
+    case k::AttnPrefillForm::Parts:
+      return k::kAttnSplitCounterBytes + k::attn_prefill_parts_bytes(n, 1);
+    case k::AttnPrefillForm::WideParts: break;
+  }
+  return k::kAttnSplitCounterBytes + k::attn_prefill_parts_bytes(n, 2);
+}
+
 // Why a prefill of n tokens cannot use this workspace, or nullptr. A launch that would run one
 // workgroup per block takes any workspace, also none.
 static const char* bad_workspace(uint32_t n, const void* workspace, uint64_t bytes) {

@@ -275,6 +275,19 @@ def test_prefill_parts_workspace_bytes(lib):
     assert size(1) < 2.2e6 and size(16) < 34.1e6
 
 
+def test_prefill_launch_bytes(lib):
+    """What one launch makes use of: nothing, the pairs' workspace, or its own parts; never more than
+    the workspace for that many tokens."""
+    use = lib.miso_attn_prefill_launch_bytes
+    for pos0, n in ((0, 1), (0, 640), (64, 100), (0, 2049), (8192, 8192), (0, 0)):
+        assert use(pos0, n) == 0
+    for pos0, n in ((0, 641), (0, 2048), (0, 4096), (8192, 3841)):
+        assert use(pos0, n) == lib.miso_attn_prefill_workspace_bytes(n)
+    for pos0, n in ((1000, 37), (12001, 203), (200000, 16), (33000, 471), (5003, 3001)):
+        assert 1024 < use(pos0, n) <= lib.miso_attn_prefill_parts_workspace_bytes(n)
+    assert use(12001, 203) == 1024 + 2 * (128 + 13) * 128 * 258 * 4
+
+
 def test_layer_core_offsets(lib):
     """The engine's scratch.core / ps.core inside the layer workspaces: 16-byte aligned, inside
     the workspace, and before the GEMM input (f16 values and sums of [max_tok][4096]) and the causal

@@ -344,3 +344,25 @@ def test_prep_batch_fp8_then_prefill_fp8(O, attn, torch_mod):
     st = O.compare(got, ref)
     report(f"fp8 prep_batch + prefill n={n}", st)
     assert st["ok"], st
+
+
+def test_prefill_fp8_scratch_made_when_none(O, attn, torch_mod):
+    """A scratch made by the call holds the prefill's own workspace only where the launch uses it (50
+    tokens do after 700, not on an empty cache), a lazy one from the first such launch on; the results
+    are those over a scratch made beforehand, bit for bit."""
+    torch = torch_mod
+    cache = attn.Fp8Cache(750)
+    g = torch.Generator(device="cuda").manual_seed(750)
+    for codes, scale in ((cache.k8, cache.k_scale), (cache.v8, cache.v_scale)):
+        codes.copy_(torch.randint(0, 64, codes.shape, generator=g, dtype=torch.uint8, device="cuda"))
+        scale.fill_(0.5)
+    full, lazy = attn.Fp8PrefillScratch(750), attn.Fp8PrefillScratch(750, lazy=True)
+    for pos0, n, given, has in ((0, 50, None, False), (700, 50, None, True), (0, 50, lazy, False),
+                                (0, 700, lazy, True)):
+        q = torch.randn(n * 4096, generator=g, device="cuda")
+        qg = torch.randn(n * 8192, generator=g, device="cuda")
+        a, b = torch.empty_like(q), torch.empty_like(q)
+        used = attn.attn_prefill_fp8(q, qg, cache, a, pos0, n, given)
+        assert (given is None or used is given) and (used.prefill is not None) == has
+        attn.attn_prefill_fp8(q, qg, cache, b, pos0, n, full)
+        assert torch.equal(a, b)
