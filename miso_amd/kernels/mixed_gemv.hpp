@@ -62,9 +62,9 @@ __global__ void __launch_bounds__(kBlock) qkv_gemv_kernel(Q4kGemvParams q, Q4kGe
 // The decode step's input in one launch: qkv_gemv_kernel on the residual row itself. Every workgroup
 // forms RMSNorm(h + delta) weight while its weights are in flight (24 KiB of rows from L2 and one
 // barrier more) instead of waiting for a launch that wrote it: 7.0 us against 2.1 + 5.8 us in two
-// launches. h itself is not updated here (every workgroup reads it); the first one of k stores the
-// normed row in xn. The last workgroup tabulates the token's rotation: rope[i], rope[32 + i] = cos,
-// sin of pos inv_freq[i].
+// launches. h itself is not updated here (every workgroup reads it). The last workgroup has no
+// rows: it stores the normed row in xn (the same arithmetic) and tabulates the token's rotation,
+// rope[i], rope[32 + i] = cos, sin of pos inv_freq[i].
 struct QkvNormParams {
   const float* h;
   const float* delta;   // or nullptr
@@ -95,9 +95,30 @@ __global__ void __launch_bounds__(256) qkv_norm_gemv_kernel(Q4kGemvParams q, Q4k
       n.rope[threadIdx.x] = c;
       n.rope[32 + threadIdx.x] = s;
     }
+    const unsigned e = 8 * threadIdx.x;
+    float f[8], ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      f[i] = n.h[e + i];
+    if (n.delta != nullptr)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        f[i] += n.delta[e + i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      ss = __builtin_fmaf(f[i], f[i], ss);
+    ss = cdna4::wave_allsum(ss);
+    if (threadIdx.x % 64 == 0)
+      rest[threadIdx.x / 64] = ss;
+    __syncthreads();
+    const float total = (rest[0] + rest[1]) + (rest[2] + rest[3]);
+    const float r = 1.0f / __builtin_sqrtf(total * (1.0f / K) + n.eps);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      n.xn[e + i] = f[i] * r * n.weight[e + i];
     return;
   }
-  const q4k_gemv_detail::NormX src{n.h, n.delta, n.weight, rest, b == kVGrid ? n.xn : nullptr, n.eps};
+  const q4k_gemv_detail::NormX src{n.h, n.delta, n.weight, rest, n.eps};
   if (b < kVGrid) {
     q6k_gemv_detail::q6k_gemv_rows<K, 256, 1>(v, src, 0, v.n_rows, b, kVGrid, slabs, x_lds);
   } else {

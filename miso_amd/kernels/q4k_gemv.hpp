@@ -143,7 +143,7 @@ union XArea {
 // Where the K activations come from. PlainX: the K floats of x. NormX: RMSNorm(h + delta) weight
 // of a residual row (delta may be null), eps added to the mean square; the rows of delta and weight
 // wait in `rest` (2 K + 4 floats of LDS), and the sum of squares is the one of a 256-thread
-// workgroup with 8 consecutive elements per thread. With `out` the workgroup stores the row there.
+// workgroup with 8 consecutive elements per thread.
 struct PlainX {
   const float* x;
 };
@@ -152,7 +152,6 @@ struct NormX {
   const float* delta;
   const float* weight;
   float* rest;
-  float* out;  // or nullptr
   float eps;
 };
 
@@ -213,10 +212,6 @@ __device__ inline void convert_x(const Src& src, XArea<A, K>& xa) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       f[i] = f[i] * r * src.rest[K + e + i];
-    if (src.out != nullptr) {  // uniform
-      *reinterpret_cast<float4*>(src.out + e) = v[0][0];
-      *reinterpret_cast<float4*>(src.out + e + 4) = v[0][1];
-    }
   } else {
     __syncthreads();  // every float is read before the converted form overwrites the area
   }
