@@ -376,11 +376,14 @@ class Fp8PrefillScratch:
     prefill's own workspace for as many tokens (PrefillScratch; with `lazy`, made by the first call
     that uses it)."""
 
+    prefill: Optional[PrefillScratch] = None
+
     def __init__(self, max_rows: int, device="cuda", lazy: bool = False):
         self.max_rows = max_rows
         self.k = torch.empty(KV_HEADS * max_rows * DIM, dtype=torch.float16, device=device)
         self.v = torch.empty(KV_HEADS * max_rows * DIM, dtype=torch.float16, device=device)
-        self.prefill = None if lazy else PrefillScratch(max_rows, device)
+        if not lazy:
+            self.prefill = PrefillScratch(max_rows, device)
 
 
 def attn_prefill_fp8(q, qg, cache: Fp8Cache, core, pos0: int, n: int,

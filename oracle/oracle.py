@@ -512,7 +512,10 @@ def drop_in():
     """ctypes handle of oracle/_build/libdrop_in.so (drop_in_capi.hip)."""
     global _drop_in
     if _drop_in is None:
-        L = ctypes.CDLL(str(HERE / "_build" / "libdrop_in.so"))
+        path = HERE / "_build" / "libdrop_in.so"
+        if not path.exists():
+            raise RuntimeError(f"{path} missing: run `make -C oracle drop_in`")
+        L = ctypes.CDLL(str(path))
         V, U = c_void_p, c_uint32
         sig = {
             "drop_engine_new": (V, [V, V, V, V, V, V, U, U]),
