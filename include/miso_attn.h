@@ -219,9 +219,10 @@ int miso_attn_decode_ragged(const float* q, const float* gate, const uint16_t* k
 
 /* The same with balanced spans for small batches: part_m and part_l hold `partials` floats and
  * part_o 256 times as many. With partials >= miso_attn_ragged_balanced_partials(batch, max_len)
- * (scratch of that size also serves fewer and shorter sequences), batches whose spans miso_attn_ragged_chunk keeps at 512 keys take the span that fills the CUs
- * evenly for their lengths (128 keys or more; the last 4 floats of part_m carry it to the merge);
- * otherwise the call is miso_attn_decode_ragged. */
+ * (scratch of that size also serves fewer and shorter sequences), batches whose spans
+ * miso_attn_ragged_chunk keeps at 512 keys take the span that fills the CUs evenly for their
+ * lengths (128 keys or more; the last 4 floats of part_m carry it to the merge); otherwise the
+ * call is miso_attn_decode_ragged. */
 uint64_t miso_attn_ragged_balanced_partials(uint32_t batch, uint32_t max_len);
 int miso_attn_decode_ragged_ws(const float* q, const float* gate, const uint16_t* k_cache,
                                const uint16_t* v_cache, const uint64_t* kv_offsets,

@@ -443,8 +443,9 @@ inline const char* decode_step(const Weights& w, attn::half_t* k_cache, attn::ha
                               ws.part_o, keys,      max_ctx, n_splits};
   const AttnCombineParams comb{ws.part_m, ws.part_l, ws.part_o, ws.proj, ws.core, n_splits};
   // Four launches where the formats are the model's and the cache holds a key, the rotation table
-  // in ws.core until the combine writes that: 21.7 us at 4096 keys against 25.3 us in the six launches below (the small kernels are
-  // launch- and latency-bound, and the prep hides under the split's first tile).
+  // in ws.core until the combine writes that: 21.7 us at 4096 keys against 25.3 us in the six
+  // launches below (the small kernels are launch- and latency-bound, and the prep hides under the
+  // split's first tile).
   if (qkv_mix(w) && len >= 1) {
     qkv_norm_launch(w, h, delta, eps, len, ws.xn, ws.core, ws.proj, stream);
     attn_prep_split_kernel<256><<<dim3(n_splits, 2), 256, 0, stream>>>(AttnPrepSplitParams{

@@ -229,9 +229,9 @@ constexpr unsigned kAttnPartsJobTiles = 12;
 //     prefix makes costly: 2100 after 8000 336 against 506, 3001 after 5003 363 against 388; 3001
 //     after 0 112 against 104 and 3300 after 4000 352 against 343 (one workgroup per block kept).
 //   - Two row blocks per wave (half the LDS reads per MFMA, twice the prologue and partial) pay
-//     from about 150 one-block tiles per worker (and with tokens for both): 512 after 32000 280 against 330 with one, 700
-//     after 14000 207 against 223; 512 after 4096 (34 tiles) 78 against 65, 2500 after 2500 (145)
-//     206 against 190.
+//     from about 150 one-block tiles per worker (and with tokens for both): 512 after 32000 280
+//     against 330 with one, 700 after 14000 207 against 223; 512 after 4096 (34 tiles) 78 against
+//     65, 2500 after 2500 (145) 206 against 190.
 constexpr unsigned kAttnPartsMaxTokens = 3072;
 static_assert(kAttnPartsMaxTokens / kAttnQBlock < 1u << 9, "a block in the top 9 bits of a place");
 inline unsigned attn_prefill_parts_row_blocks(unsigned pos0, unsigned n) {
@@ -491,11 +491,11 @@ __device__ __attribute__((always_inline)) inline void scale_acc(float16_t (&o)[8
 // Softmax decision for one block of one tile. `acc`: the block's S^T accumulator (raw scores in
 // log2 units; element r = key k0 + 8 (r / 4) + 4 hi + r % 4, the lane's row). Keys past `lim` are
 // masked when kMasked. The reference max m moves only when the tile's row max exceeds it by more
-// than the slack (2^8), decided wave-wide so the rescale branch is uniform; on the first tile with a
-// finite score (m = kNoMax before it) it always moves. Writes the f16 numerators 2^(s - m) as the block's two P^T operands,
-// updates l = l corr + their sum (the sum of the rounded values the MFMAs use), and returns
-// corr = 2^(m_old - m_new), the factor the block's O must be scaled by (1 if m stayed; `moved`
-// says whether any lane's m moved).
+// than the slack (2^8), decided wave-wide so the rescale branch is uniform; on the first tile with
+// a finite score (m = kNoMax before it) it always moves. Writes the f16 numerators 2^(s - m) as the
+// block's two P^T operands, updates l = l corr + their sum (the sum of the rounded values the MFMAs
+// use), and returns corr = 2^(m_old - m_new), the factor the block's O must be scaled by (1 if m
+// stayed; `moved` says whether any lane's m moved).
 template <bool kMasked>
 __device__ __attribute__((always_inline)) inline float decide_block(const float16_t& acc,
                                                                    float& m, float& l,

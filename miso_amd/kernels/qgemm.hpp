@@ -848,11 +848,12 @@ __global__ void __launch_bounds__(64 * WM * WN, kWavesPerSimd) qgemm_wide_kernel
 // kGroup (token tiles swept across the row tiles) keeps the ~32 to 96 tiles an XCD runs at once
 // within its 4 MiB of L2 also at k = 4096: 2048 rows x 4096, 512 tokens in 64 x 64 tiles 36 us
 // in groups of 8, 31 in groups of 4.
-// 64 x 64 tiles, one workgroup per CU: nothing hides a stage's wait, and weights come from memory (a
-// model's layers do not stay in the L2s), so Q4_K takes four stages in the ring. Weights of 80
-// matrices in turn, with two stages and four: 2048 rows x 4096, 13 tokens 30.8 / 26.4 us, 512 tokens
-// 34.8 / 27.3; 8192 rows x 2048, 64 tokens 19.6 / 15.8; a whole layer over 512 tokens 125 / 118. Q6_K
-// waits for its weights' registers at every other stage, and stays with two: 512 rows x 2048 19.5 / 20.9.
+// 64 x 64 tiles, one workgroup per CU: nothing hides a stage's wait, and weights come from memory
+// (a model's layers do not stay in the L2s), so Q4_K takes four stages in the ring. Weights of 80
+// matrices in turn, with two stages and four: 2048 rows x 4096, 13 tokens 30.8 / 26.4 us, 512
+// tokens 34.8 / 27.3; 8192 rows x 2048, 64 tokens 19.6 / 15.8; a whole layer over 512 tokens 125 /
+// 118. Q6_K waits for its weights' registers at every other stage, and stays with two: 512 rows x
+// 2048 19.5 / 20.9.
 struct QGemmShape {
   unsigned index;  // 0 .. 3: 64 x 64, 128 x 64, 128 x 128, 256 x 128
   unsigned tiles;  // the launch's workgroups

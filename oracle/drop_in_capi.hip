@@ -1,7 +1,7 @@
 // Test infrastructure: extern "C" launchers for what the product's own library does not launch: the
-// engine drop-in (miso_amd/engine/attention.{hpp,hip} against engine_stub/), the 64 x 64 GEMM kernel
-// that the engine's own gemm() launches, GEMM batches of any mix, and the host's choices of a form. Used only by GPU tests; never
-// linked into the product.
+// engine drop-in (miso_amd/engine/attention.{hpp,hip} against engine_stub/), the 64 x 64 GEMM
+// kernel that the engine's own gemm() launches, GEMM batches of any mix, and the host's choices of
+// a form. Used only by GPU tests; never linked into the product.
 
 #include "engine/attention.hip"
 

@@ -6,10 +6,10 @@ blocks, a 32-key sub-chunk crossing, a non-empty prefix) with q = 2 N(0,1), then
 configs C3 (2048 tokens, empty cache; every row) and C4 (8192 tokens after an 8192-token prefix;
 a deterministic row sample covering first/last tiles and diagonal tiles), plus two size-free
 properties: chunked prefill equals one-shot prefill, and prefill row t equals decode at pos0+t+1.
-The balanced form (miso_attn_prefill_ws: heavy token blocks split between two workgroups, the
-parts merged through a workspace; 16-token blocks from 641 to 2048 tokens, 32-token blocks from 3841
-to 4096) and the parts (few tokens after a prefix) are checked the same way, on shapes with and without split blocks, plus run-to-run bit equality
-and reuse of one workspace across sizes.
+The balanced form (miso_attn_prefill_ws: heavy token blocks split between two workgroups, the parts
+merged through a workspace; 16-token blocks from 641 to 2048 tokens, 32-token blocks from 3841 to
+4096) and the parts (few tokens after a prefix) are checked the same way, on shapes with and without
+split blocks, plus run-to-run bit equality and reuse of one workspace across sizes.
 Gate: |got - ref| <= 2e-3 + 1e-2 |ref| for every element (f32 output).
 """
 from __future__ import annotations
